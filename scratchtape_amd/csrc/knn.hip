@@ -100,6 +100,122 @@ __global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ keys
     quantize_row([&](int i) { return k[i]; }, d, codes + r * (d / 4), scales + r);
 }
 
+// Rows of up to QD_MAX columns (d % 16 == 0) from 16-byte aligned keys: one wave per QR keys.
+//
+// Bound by HBM (4 d + d/4 + 4 bytes per key).  The thread-per-key form below
+// touches 64 rows per load instruction and reads every key twice; here a wave
+// reads its QR rows once as one contiguous run of 16-byte loads (lane l of
+// load i holds float4 64 i + l of the run), all in flight together, and keeps
+// them in registers.  The sum of squares is the contract's serial f32 sum over
+// a row, so the run also goes through LDS (rows padded by 4 floats: the 16
+// rows' 16-byte reads start 4 banks apart and cover all 64 banks) and lane r
+// sums row r in index order.  The codes need no division per component:
+// x / scale + 1.5 and the two roundings are monotone in x, so each code step
+// is a threshold on x (quantize_steps), found once per row.
+// 2^20 keys x 256: 4,635 us before, 245 us now (4.7 TB/s; a 1 GiB copy on this
+// card moves 5.1 TB/s).  16 rows per wave leaves room for nine
+// waves per CU (16.6 KB of LDS each).
+constexpr int QR = 16;       // keys per wave
+constexpr int QD_MAX = 256;  // widest row held in registers (QR * QD_MAX / 256 float4 per lane)
+
+// Smallest x with code >= 1, >= 2, >= 3 for a finite scale s >= 1e-30: with
+// q = fl(x / s) and y = fl(q + 1.5), round-half-away(y) >= 1, 2, 3 iff y >=
+// 0.5, 1.5, 2.5.  y >= 0.5 iff q >= -1 iff x >= -s; y >= 1.5 iff q >= -2^-24
+// (1.5 - 2^-24 ties to the even 1.5) iff x >= -s 2^-24 (s 2^-24 is a normal
+// number); y >= 2.5 holds for x = s and at most a few floats below it, walked
+// here with the expression itself.
+__device__ __forceinline__ float quantize_step3(float s) {
+    float t = s;
+    for (int i = 0; i < 8; i++) {  // at most two steps are taken
+        const float p = __uint_as_float(__float_as_uint(t) - 1u);
+        if (!(p / s + 1.5f >= 2.5f)) break;
+        t = p;
+    }
+    return t;
+}
+
+__global__ __launch_bounds__(64) void k_quantize_rows(const float *__restrict__ keys, int64_t n, int32_t d,
+                                                      uint8_t *__restrict__ codes, float *__restrict__ scales) {
+    constexpr int NL = QR * QD_MAX / 256;  // loads per lane at the widest row
+    __shared__ __attribute__((aligned(16))) float rowbuf[QR * (QD_MAX + 4)];
+    __shared__ float s_scale[QR], s_t3[QR];
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    const int lane = threadIdx.x;
+    const int64_t r0 = (int64_t)blockIdx.x * QR;
+    const int nr = (int)min((int64_t)QR, n - r0);  // keys of this wave
+    const int q4 = d >> 2;                         // float4 per row
+    const int inv = (65535 + q4) / q4;             // e / q4 = e inv >> 16 for e < 1024, q4 <= 64
+    const int total = nr * q4;                     // float4 of the run
+    const f4 *src = reinterpret_cast<const f4 *>(keys + r0 * d);
+    f4 x[NL];
+#pragma unroll
+    for (int i = 0; i < NL; i++)
+        if (64 * i < total) {  // uniform; the last load's lanes past the run repeat its last float4
+            const int e = 64 * i + lane;
+            x[i] = __builtin_nontemporal_load(src + (e < total ? e : total - 1));
+        }
+    const int pitch = d + 4;
+#pragma unroll
+    for (int i = 0; i < NL; i++)
+        if (64 * i < total) {
+            const int e = 64 * i + lane;
+            const int r = e * inv >> 16, c = e - r * q4;
+            if (e < total) *reinterpret_cast<f4 *>(rowbuf + r * pitch + 4 * c) = x[i];
+        }
+    __syncthreads();
+    if (lane < nr) {
+        const f4 *row = reinterpret_cast<const f4 *>(rowbuf + lane * pitch);
+        float ss = 0.f;
+#pragma unroll 4
+        for (int c = 0; c < q4; c++) {
+            const f4 v = row[c];
+            ss += v.x * v.x;
+            ss += v.y * v.y;
+            ss += v.z * v.z;
+            ss += v.w * v.w;
+        }
+        float scale = 0.9957f * sqrtf(ss / (float)d);
+        if (!(scale >= 1e-30f)) scale = 1e-30f;
+        s_scale[lane] = scale;
+        s_t3[lane] = quantize_step3(scale);
+        scales[r0 + lane] = scale;
+    }
+    __syncthreads();
+    // Each float4 is one byte of codes; the quad's four bytes make a dword, and
+    // lane j of the quad keeps load 4 t + j's, so that a wave stores four
+    // loads' codes at once.
+    uint32_t *dst = reinterpret_cast<uint32_t *>(codes + r0 * (d / 4));
+    const int sub = lane & 3;
+#pragma unroll
+    for (int t = 0; t < NL; t += 4) {
+        uint32_t keep = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int i = t + j;
+            if (64 * i < total) {  // uniform
+                const int e = min(64 * i + lane, total - 1);
+                const int r = e * inv >> 16;
+                const float s = s_scale[r], t3 = s_t3[r], t1 = -s, t2 = -s * 0x1p-24f;
+                uint32_t b = 0;
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    const float v = x[i][c];
+                    uint32_t u = (uint32_t)(v >= t1) + (uint32_t)(v >= t2) + (uint32_t)(v >= t3);
+                    // An infinite scale (the sum overflowed): x / scale is 0 for a finite x, NaN otherwise.
+                    if (t3 > 3.4028235e38f) u = fabsf(v) <= 3.4028235e38f ? 2u : 0u;
+                    b |= u << (2 * c);
+                }
+                uint32_t w = b << (8 * sub);
+                w |= st::xor_lane(w, 1, lane);
+                w |= st::xor_lane(w, 2, lane);
+                if (sub == j) keep = w;
+            }
+        }
+        const int e0 = 64 * (t + sub) + (lane & ~3);  // first float4 of this lane's dword
+        if (e0 < total) dst[e0 >> 2] = keep;
+    }
+}
+
 // The reference's stored per-key norm (knn.rs:216): sum over the dims, in
 // order, of f16((u - 1.5) scale)^2 in f32; one thread per key.
 __global__ __launch_bounds__(256) void k_key_norms(const uint8_t *__restrict__ codes, const float *__restrict__ scales,
@@ -1124,8 +1240,13 @@ extern "C" st_status st_knn_quantize_2bit(const float *keys, int64_t n, int64_t 
     if ((reinterpret_cast<uintptr_t>(codes) & 3) != 0) return st::fail(ST_ERR_INVALID, "codes must be 4-byte aligned");
     if (n == 0) return ST_OK;
     if (!st::device_ok()) return ST_ERR_NO_DEVICE;
-    hipLaunchKernelGGL(k_quantize, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st::stream_of(stream), keys, n,
-                       (int32_t)d, codes, scales);
+    // Wider rows, and keys that are not 16-byte aligned, take a thread per key.
+    if (d <= QD_MAX && (reinterpret_cast<uintptr_t>(keys) & 15) == 0 && cdiv(n, QR) <= INT32_MAX)
+        hipLaunchKernelGGL(k_quantize_rows, dim3((unsigned)cdiv(n, QR)), dim3(64), 0, st::stream_of(stream), keys, n,
+                           (int32_t)d, codes, scales);
+    else
+        hipLaunchKernelGGL(k_quantize, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st::stream_of(stream), keys, n,
+                           (int32_t)d, codes, scales);
     ST_LAUNCH_CHECK();
     return ST_OK;
 }

@@ -12,6 +12,32 @@ pytestmark = pytest.mark.gpu
 D = 256
 
 
+@pytest.mark.parametrize("d", [16, 48, 64, 208, 256, 272])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 1003])
+def test_quantizer_widths_and_tails(dev, n, d):
+    """The wave-per-16-keys form (d <= 256, aligned keys) at its edges, bit for bit against the oracle and against the
+    thread-per-key form (keys that start 4 bytes off)."""
+    rng = np.random.default_rng(1000 * d + n)
+    keys = (rng.standard_normal((n, d)) * 2.0 ** rng.integers(-40, 40, (n, 1))).astype(np.float32)
+    codes, scales = knn.quantize_2bit(torch.from_numpy(keys).to(dev))
+    wc, ws = oracle.quantize_2bit(keys, d)
+    np.testing.assert_array_equal(codes.cpu().numpy(), wc)
+    np.testing.assert_array_equal(scales.cpu().numpy(), ws)
+    # Components on the code steps (multiples of the scale and their neighbours), and rows that are not ordinary numbers.
+    keys[:, 0] = ws
+    keys[:, 1] = -np.nextafter(ws, np.float32(np.inf))
+    odd = [0.0, 1e-38, 1e-45, 3e38, np.inf, -np.inf, np.nan]
+    for i in range(min(n, len(odd))):
+        keys[i, rng.integers(0, d)] = odd[i]
+    keys[n - 1, :] = 0.0
+    buf = torch.zeros(n * d + 1, device=dev)
+    buf[1:] = torch.from_numpy(keys.reshape(-1)).to(dev)
+    a = knn.quantize_2bit(buf[1:].clone().view(n, d))
+    b = knn.quantize_2bit(buf[1:].view(n, d))
+    assert torch.equal(a[0], b[0])
+    assert torch.equal(a[1].view(torch.int32), b[1].view(torch.int32))
+
+
 def test_quantizer_is_bit_exact(dev):
     rng = np.random.default_rng(1)
     keys = rng.standard_normal((5000, D)).astype(np.float32)
