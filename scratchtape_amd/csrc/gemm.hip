@@ -12,13 +12,21 @@
 //  - f16 route: v_mfma_f32_16x16x32_f16; f32 operands are read from HBM with
 //    128-bit loads and rounded to f16 (round to nearest even) on the way into
 //    LDS.  f32 route: v_mfma_f32_16x16x4_f32 on f32 LDS tiles.
-//  - LDS holds both operands k-contiguous ([row][k], rows padded by 16 bytes
-//    so the 128-bit fragment reads of 8 lanes hit distinct banks).  An operand
-//    whose k is contiguous in memory (A not transposed, B transposed) is copied
-//    as vectors; the others are loaded as 4x4 blocks and transposed in
-//    registers.  k-stages of 64 (f16) / 32 (f32); two LDS buffers and two
-//    register sets, so stage s+2 is in flight from global memory while stage s
-//    feeds the MFMAs and stage s+1 is written to LDS; one barrier per stage.
+//  - LDS holds an operand [row][k] (rows padded by 16 bytes, so the 128-bit
+//    fragment reads of 8 lanes hit distinct banks) or, for an f32 operand whose
+//    rows are contiguous in memory (A transposed, B not), [k][row] as loaded.
+//    The f16 route turns the latter's 4x4 blocks in registers.  k-stages of 64
+//    (f16) / 32 (f32); two LDS buffers and two register sets, so stage s+2 is
+//    in flight from global memory while stage s feeds the MFMAs and stage s+1
+//    is written to LDS; one barrier per stage and no branch around the loads.
+//  - Bound: f32 by the matrix cores (busy 70 % of the CUs' time at 3001 x 2000
+//    x 1003) once there are workgroups to overlap, by the LDS round and barrier
+//    of a k-stage with one workgroup per CU.  The form before loaded every
+//    element of a ragged or misaligned shape by itself, guarded, and waited for
+//    each load where it was issued.  Single calls, us before and now:
+//    3000 x 250 x 1001 forward 45 -> 26, dW 55 -> 31, dX 50 -> 22; 3001 x 2000 x
+//    1003 273 -> 116, 239 -> 138, 273 -> 121 (104 TFLOP/s); 96 products of
+//    200 x 80 x 200 52 -> 22; f16 8192 x 1056 x 1056 237 -> 71.
 //  - Workgroups are remapped so that each of the 8 XCDs works on a contiguous
 //    run of tiles, which share operand panels in that XCD's L2.
 //  - Fragment k-order: each lane reads its k-run as one 128-bit LDS read and
@@ -36,6 +44,7 @@
 #include <vector>
 
 #include "common.h"
+#include "dma_tile.h"
 #include "gemm_dma.h"
 
 namespace {
@@ -82,12 +91,28 @@ __device__ __forceinline__ void store4(void *dst, float x0, float x1, float x2, 
     }
 }
 
+// How a tile's operands are read (Stager), for any shape and alignment:
+//  - WHOLE (the matrix is at least one tile in both dimensions): a last tile
+//    that would cross the edge is moved back to end there and stores only the
+//    rows and columns that are its own, so every load is a 16-byte load (4-byte
+//    alignment is enough) with no guard;
+//  - otherwise (fewer than 32 rows or columns): element by element, the rows
+//    past the matrix repeating its last one.  They feed output rows and columns
+//    that are not stored.
+// The partial k-stage comes first and is loaded element by element.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
 // Stages one operand's ROWS x BK tile (logical rows = m for A, n for B; k
-// across) from global memory into registers, then into LDS as [row][k].
+// across) from global memory into registers, then into LDS.
 // KCONTIG: element (r, kk) at base[r*ld + kk]; else at base[kk*ld + r].
-template <int ROWS, int BK, bool KCONTIG, bool FAST, bool F16>
+template <int ROWS, int BK, bool KCONTIG, bool WHOLE, bool F16>
 struct Stager {
+    // LDS tile: [row][k] with rows LDS_K apart, or (KROWS) [k][row] with lines
+    // LDS_R apart, written as loaded.
+    static constexpr bool KROWS = !KCONTIG && !F16;
     static constexpr int LDS_K = BK + (F16 ? 8 : 4);
+    static constexpr int LDS_R = ROWS + 4;
+    static constexpr int SIZE = KROWS ? BK * LDS_R : ROWS * LDS_K;
     // KCONTIG: 4-wide vectors along k.  Else 4x4 blocks (4 k x 4 rows).
     static constexpr int UNITS = KCONTIG ? ROWS * BK / 4 : ROWS * BK / 16;
     static constexpr int PER = (UNITS + THREADS - 1) / THREADS;
@@ -103,47 +128,73 @@ struct Stager {
             for (int x = 0; x < (KCONTIG ? 1 : 4); x++) cs[i][x] = 0.f;
     }
 
-    __device__ __forceinline__ void load(const float *__restrict__ base, int64_t ld, int row0,
-                                         int row_lim, int k0, int k_lim, int tid) {
+    // Four rows from `row` of one k-line, or (KCONTIG) four k of one row.
+    static __device__ __forceinline__ f32x4 rows4(const float *line, int row, int row_lim) {
+        if constexpr (WHOLE) return *reinterpret_cast<const f32x4u *>(line + row);
+        return f32x4{line[min(row, row_lim - 1)], line[min(row + 1, row_lim - 1)], line[min(row + 2, row_lim - 1)],
+                     line[min(row + 3, row_lim - 1)]};
+    }
+
+    // Loads the tile of the first k-stage: nk <= BK of k from k0, zeros behind
+    // them.
+    __device__ __forceinline__ void load_first(const float *__restrict__ base, int64_t ld, int row0, int row_lim,
+                                               int k0, int nk, int tid) {
 #pragma unroll
         for (int i = 0; i < PER; i++) {
             const int u = tid + THREADS * i;
             if (UNITS % THREADS != 0 && u >= UNITS) break;
             if constexpr (KCONTIG) {
                 const int rr = u / (BK / 4), kq = (u % (BK / 4)) * 4;
-                const float *src = base + (int64_t)(row0 + rr) * ld + (k0 + kq);
-                if constexpr (FAST) {
-                    r[i][0] = *reinterpret_cast<const f32x4 *>(src);
-                } else {
-                    const bool rok = row0 + rr < row_lim;
+                const float *row = base + (int64_t)(WHOLE ? row0 + rr : min(row0 + rr, row_lim - 1)) * ld + k0;
 #pragma unroll
-                    for (int e = 0; e < 4; e++) r[i][0][e] = (rok && k0 + kq + e < k_lim) ? src[e] : 0.f;
+                for (int e = 0; e < 4; e++) {
+                    const float v = row[min(kq + e, nk - 1)];
+                    r[i][0][e] = kq + e < nk ? v : 0.f;
                 }
             } else {
                 const int rq = (u % (ROWS / 4)) * 4, kq = (u / (ROWS / 4)) * 4;
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    const float *src = base + (int64_t)(k0 + kq + e) * ld + (row0 + rq);
-                    if constexpr (FAST) {
-                        r[i][e] = *reinterpret_cast<const f32x4 *>(src);
-                    } else {
-                        const bool kok = k0 + kq + e < k_lim;
-#pragma unroll
-                        for (int x = 0; x < 4; x++) r[i][e][x] = (kok && row0 + rq + x < row_lim) ? src[x] : 0.f;
-                    }
+                    const f32x4 v = rows4(base + (int64_t)(k0 + min(kq + e, nk - 1)) * ld, row0 + rq, row_lim);
+                    r[i][e] = kq + e < nk ? v : f32x4{0.f, 0.f, 0.f, 0.f};
                 }
             }
         }
     }
 
-    __device__ __forceinline__ void add_cs() {
+    // Loads the tile of a whole k-stage, without a branch.
+    __device__ __forceinline__ void load(const float *__restrict__ base, int64_t ld, int row0, int row_lim, int k0,
+                                         int tid) {
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const int u = tid + THREADS * i;
+            if (UNITS % THREADS != 0 && u >= UNITS) break;
+            if constexpr (KCONTIG) {
+                const int rr = u / (BK / 4), kq = (u % (BK / 4)) * 4;
+                const float *row = base + (int64_t)(WHOLE ? row0 + rr : min(row0 + rr, row_lim - 1)) * ld + kq;
+                r[i][0] = *reinterpret_cast<const f32x4u *>(row + k0);
+            } else {
+                const int rq = (u % (ROWS / 4)) * 4, kq = (u / (ROWS / 4)) * 4;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    r[i][e] = rows4(base + (int64_t)(kq + e) * ld + (int64_t)k0 * ld, row0 + rq, row_lim);
+            }
+        }
+    }
+
+    // Adds the tile's values to the column sums (`on`: uniform, without a branch).
+    __device__ __forceinline__ void add_cs(bool on) {
 #pragma unroll
         for (int i = 0; i < PER; i++) {
             if constexpr (KCONTIG) {
-                cs[i][0] += ((r[i][0][0] + r[i][0][1]) + r[i][0][2]) + r[i][0][3];
+                const float t = cs[i][0] + (((r[i][0][0] + r[i][0][1]) + r[i][0][2]) + r[i][0][3]);
+                cs[i][0] = on ? t : cs[i][0];
             } else {
 #pragma unroll
-                for (int x = 0; x < 4; x++) cs[i][x] += ((r[i][0][x] + r[i][1][x]) + r[i][2][x]) + r[i][3][x];
+                for (int x = 0; x < 4; x++) {
+                    const float t = cs[i][x] + (((r[i][0][x] + r[i][1][x]) + r[i][2][x]) + r[i][3][x]);
+                    cs[i][x] = on ? t : cs[i][x];
+                }
             }
         }
     }
@@ -160,8 +211,12 @@ struct Stager {
             } else {
                 const int rq = (u % (ROWS / 4)) * 4, kq = (u / (ROWS / 4)) * 4;
 #pragma unroll
-                for (int x = 0; x < 4; x++)
-                    store4<F16>(lds + (rq + x) * LDS_K + kq, r[i][0][x], r[i][1][x], r[i][2][x], r[i][3][x]);
+                for (int x = 0; x < 4; x++) {
+                    if constexpr (KROWS)
+                        *reinterpret_cast<f32x4 *>(lds + (kq + x) * LDS_R + rq) = r[i][x];
+                    else
+                        store4<F16>(lds + (rq + x) * LDS_K + kq, r[i][0][x], r[i][1][x], r[i][2][x], r[i][3][x]);
+                }
             }
         }
     }
@@ -190,33 +245,37 @@ struct Stager {
     }
 };
 
-template <int BM, int BN, int BK, bool TA, bool TB, bool F16, bool FAST>
+template <int BM, int BN, int BK, bool TA, bool TB, bool F16, bool WHOLE>
 __global__ __launch_bounds__(THREADS) void k_gemm(GemmArgs g) {
     using T = typename std::conditional<F16, _Float16, float>::type;
-    using SA = Stager<BM, BK, !TA, FAST, F16>;
-    using SB = Stager<BN, BK, TB, FAST, F16>;
+    using SA = Stager<BM, BK, !TA, WHOLE, F16>;
+    using SB = Stager<BN, BK, TB, WHOLE, F16>;
     constexpr int LDS_K = SA::LDS_K;
     constexpr int WM = BM / 2, WN = BN / 2;
     constexpr int FM = WM / 16, FN = WN / 16;
     static_assert(BK % (F16 ? 32 : 16) == 0, "k stage");
-    __shared__ __attribute__((aligned(16))) T As[2][BM * LDS_K];
-    __shared__ __attribute__((aligned(16))) T Bs[2][BN * LDS_K];
+    __shared__ __attribute__((aligned(16))) T As[2][SA::SIZE];
+    __shared__ __attribute__((aligned(16))) T Bs[2][SB::SIZE];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     // Workgroups are dealt to the 8 XCDs round-robin by linear id; remap so
-    // each XCD gets a contiguous run of tiles (x fastest), which share A rows
-    // (and k-slices) in that XCD's L2.
-    int64_t lin = blockIdx.x + (int64_t)gridDim.x * (blockIdx.y + (int64_t)gridDim.y * blockIdx.z);
-    const int64_t total = (int64_t)gridDim.x * gridDim.y * gridDim.z;
+    // each XCD gets a contiguous run of tiles (columns fastest), which share A
+    // rows (and k-slices) in that XCD's L2.
+    int64_t lin = blockIdx.x + (int64_t)gridDim.x * blockIdx.z;
+    const int64_t total = (int64_t)gridDim.x * gridDim.z;
     if (total % 8 == 0) lin = (lin % 8) * (total / 8) + lin / 8;
-    const int bx = (int)(lin % gridDim.x);
-    const int by = (int)((lin / gridDim.x) % gridDim.y);
-    const int64_t z = lin / ((int64_t)gridDim.x * gridDim.y);
+    const int nbx = (g.n + BN - 1) / BN;
+    const int64_t z = lin / gridDim.x;
+    const int tile = (int)(lin % gridDim.x);
+    const int bx = tile % nbx, by = tile / nbx;
     const int64_t zb = z / g.splits;
     const int slice = (int)(z % g.splits);
-    const int row0 = by * BM, col0 = bx * BN;
+    // The tile's own rows and columns begin at row_own, col_own; the last tile
+    // of a row or column of tiles may be moved back to row0, col0.
+    const int row_own = by * BM, col_own = bx * BN;
+    const int row0 = WHOLE ? min(row_own, g.m - BM) : row_own, col0 = WHOLE ? min(col_own, g.n - BN) : col_own;
     const int kbeg = slice * g.slice_k;
     const int kend = min(g.k, kbeg + g.slice_k);
     const int nst = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
@@ -238,30 +297,31 @@ __global__ __launch_bounds__(THREADS) void k_gemm(GemmArgs g) {
 #pragma unroll
         for (int j = 0; j < FN; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+    // The partial k-stage comes first (k1 of k), so that every later one is
+    // whole.
+    const int k1 = nst > 0 ? kend - kbeg - (nst - 1) * BK : 0;
+    const int kfull = kbeg + k1 - BK;  // stage st >= 1 begins at kfull + st BK
+    auto load = [&](int p, int st) {
+        const int k0 = kfull + st * BK;
+        sa[p].load(abase, g.a.ld, row0, g.m, k0, tid);
+        sb[p].load(bbase, g.b.ld, col0, g.n, k0, tid);
+    };
+    auto stage = [&](int p, bool live) {
+        sb[p].add_cs(live);
+        sa[p].store(As[p], tid);
+        sb[p].store(Bs[p], tid);
+    };
     if (nst > 0) {
-        sa[0].load(abase, g.a.ld, row0, g.m, kbeg, kend, tid);
-        sb[0].load(bbase, g.b.ld, col0, g.n, kbeg, kend, tid);
-    }
-    if (nst > 1) {
-        sa[1].load(abase, g.a.ld, row0, g.m, kbeg + BK, kend, tid);
-        sb[1].load(bbase, g.b.ld, col0, g.n, kbeg + BK, kend, tid);
-    }
-    if (nst > 0) {
-        if (do_cs) sb[0].add_cs();
-        sa[0].store(As[0], tid);
-        sb[0].store(Bs[0], tid);
+        sa[0].load_first(abase, g.a.ld, row0, g.m, kbeg, k1, tid);
+        sb[0].load_first(bbase, g.b.ld, col0, g.n, kbeg, k1, tid);
+        if (nst > 1) load(1, 1);
+        stage(0, true);
     }
     __syncthreads();
 
-    auto body = [&](auto pc, int st) {
-        constexpr int P = decltype(pc)::value;
-        if (st + 2 < nst) {
-            const int k0 = kbeg + (st + 2) * BK;
-            sa[P].load(abase, g.a.ld, row0, g.m, k0, kend, tid);
-            sb[P].load(bbase, g.b.ld, col0, g.n, k0, kend, tid);
-        }
-        const T *as = As[P] + (wm * WM + (lane & 15)) * LDS_K;
-        const T *bs = Bs[P] + (wn * WN + (lane & 15)) * LDS_K;
+    auto multiply = [&](int p) {
+        const T *as = As[p] + (wm * WM + (lane & 15)) * (SA::KROWS ? 1 : LDS_K);
+        const T *bs = Bs[p] + (wn * WN + (lane & 15)) * (SB::KROWS ? 1 : LDS_K);
         if constexpr (F16) {
 #pragma unroll
             for (int ks = 0; ks < BK / 32; ks++) {
@@ -282,10 +342,22 @@ __global__ __launch_bounds__(THREADS) void k_gemm(GemmArgs g) {
             for (int kc = 0; kc < BK / 16; kc++) {
                 f32x4 af[FM], bf[FN];
                 const int ko = kc * 16 + 4 * (lane >> 4);
+                // Four k of a row at once, or ([k][row] tiles) one k of each line: the lane groups' lines are
+                // 4 LDS_R = 16 banks apart, so the 64 lanes of a read hit 64 banks.
 #pragma unroll
-                for (int i = 0; i < FM; i++) af[i] = *reinterpret_cast<const f32x4 *>(as + i * 16 * LDS_K + ko);
+                for (int i = 0; i < FM; i++) {
+                    if constexpr (SA::KROWS)
+                        for (int e = 0; e < 4; e++) af[i][e] = as[(ko + e) * SA::LDS_R + i * 16];
+                    else
+                        af[i] = *reinterpret_cast<const f32x4 *>(as + i * 16 * LDS_K + ko);
+                }
 #pragma unroll
-                for (int j = 0; j < FN; j++) bf[j] = *reinterpret_cast<const f32x4 *>(bs + j * 16 * LDS_K + ko);
+                for (int j = 0; j < FN; j++) {
+                    if constexpr (SB::KROWS)
+                        for (int e = 0; e < 4; e++) bf[j][e] = bs[(ko + e) * SB::LDS_R + j * 16];
+                    else
+                        bf[j] = *reinterpret_cast<const f32x4 *>(bs + j * 16 * LDS_K + ko);
+                }
 #pragma unroll
                 for (int s = 0; s < 4; s++)
 #pragma unroll
@@ -295,26 +367,35 @@ __global__ __launch_bounds__(THREADS) void k_gemm(GemmArgs g) {
                             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i][s], bf[j][s], acc[i][j], 0, 0, 0);
             }
         }
-        if (st + 1 < nst) {
-            if (do_cs) sb[P ^ 1].add_cs();
-            sa[P ^ 1].store(As[P ^ 1], tid);
-            sb[P ^ 1].store(Bs[P ^ 1], tid);
-        }
-        __syncthreads();
     };
-    for (int st = 0; st < nst; st += 2) {
-        body(std::integral_constant<int, 0>(), st);
-        if (st + 1 < nst) body(std::integral_constant<int, 1>(), st + 1);
+    // Stages st and st + 1 per trip, stage st in LDS and st + 1 in flight at
+    // its head.  No branch inside: the loads past the last stage repeat it, so
+    // that the compiler can count the loads in flight (behind a condition it
+    // waits for all of them, a memory round trip per stage), and the asm keeps
+    // them above the multiplication.
+    for (int st = 0; st + 1 < nst; st += 2) {
+        load(0, min(st + 2, nst - 1));
+        asm volatile("" ::: "memory");
+        multiply(0);
+        stage(1, true);
+        __syncthreads();
+        load(1, min(st + 3, nst - 1));
+        asm volatile("" ::: "memory");
+        multiply(1);
+        stage(0, st + 2 < nst);
+        __syncthreads();
     }
+    if (nst & 1) multiply(0);
+    __syncthreads();
 
     // Column sums of this slice of B (tile row 0 only), reduced in slot order.
     if (do_cs) {
         float *red = reinterpret_cast<float *>(As[0]);  // BN * SLOTS floats fit in As
-        static_assert(BN * SB::SLOTS * 4 <= BM * LDS_K * (int)sizeof(T), "column-sum buffer");
+        static_assert(BN * SB::SLOTS * 4 <= SA::SIZE * (int)sizeof(T), "column-sum buffer");
         sb[0].merge_cs(sb[1]);
         sb[0].put_cs(red, tid);
         __syncthreads();
-        if (tid < BN && col0 + tid < g.n) {
+        if (tid < BN && col0 + tid >= col_own && col0 + tid < g.n) {
             float tot = 0.f;
 #pragma unroll
             for (int s = 0; s < SB::SLOTS; s++) tot += red[tid * SB::SLOTS + s];
@@ -327,26 +408,44 @@ __global__ __launch_bounds__(THREADS) void k_gemm(GemmArgs g) {
     }
 
     // Epilogue: lane holds rows 4*(lane/16)+r, column lane%16 of each block.
+    // A row of blocks' mask, residual and output values are loaded together
+    // (one memory round trip, not one per element); elements past the matrix
+    // read its last row or column.
     const int64_t o0 = (z / g.o_group) * g.o_stride + (z % g.o_group) * g.o_inner;
+    float bv[FN];
+#pragma unroll
+    for (int j = 0; j < FN; j++)
+        bv[j] = g.bias ? g.bias[zb * g.bias_stride + min(col0 + wn * WN + j * 16 + (lane & 15), g.n - 1)] : 0.f;
 #pragma unroll
     for (int i = 0; i < FM; i++) {
+        float mk[FN][4], rs[FN][4], pv[FN][4];
+        int64_t idx[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            idx[r] = o0 + (int64_t)min(row0 + wm * WM + i * 16 + 4 * (lane >> 4) + r, g.m - 1) * g.ldo;
+        auto gather = [&](const float *src, float (&v)[FN][4]) {
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    v[j][r] = src[idx[r] + min(col0 + wn * WN + j * 16 + (lane & 15), g.n - 1)];
+        };
+        if (g.mask) gather(g.mask, mk);
+        if (g.res) gather(g.res, rs);
+        if (g.accumulate) gather(g.out, pv);
 #pragma unroll
         for (int j = 0; j < FN; j++) {
             const int col = col0 + wn * WN + j * 16 + (lane & 15);
-            if (!FAST && col >= g.n) continue;
-            const float bv = g.bias ? g.bias[zb * g.bias_stride + col] : 0.f;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int row = row0 + wm * WM + i * 16 + 4 * (lane >> 4) + r;
-                if (!FAST && row >= g.m) continue;
                 float v = acc[i][j][r];
-                const int64_t idx = o0 + (int64_t)row * g.ldo + col;
-                if (g.bias) v += bv;
+                if (g.bias) v += bv[j];
                 if (g.relu && v < 0.f) v = 0.f;
-                if (g.mask && g.mask[idx] <= 0.f) v = 0.f;
-                if (g.res) v += g.res[idx];
-                if (g.accumulate) v += g.out[idx];
-                g.out[idx] = v;
+                if (g.mask && mk[j][r] <= 0.f) v = 0.f;
+                if (g.res) v += rs[j][r];
+                if (g.accumulate) v += pv[j][r];
+                const int row = row0 + wm * WM + i * 16 + 4 * (lane >> 4) + r;
+                if (WHOLE ? col >= col_own && row >= row_own : col < g.n && row < g.m) g.out[idx[r] + col] = v;
             }
         }
     }
@@ -361,8 +460,7 @@ __global__ __launch_bounds__(256) void k_split_sum(const float *__restrict__ par
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e < batch * len) {
         const int64_t b = e / len, i = e % len;
-        float v = 0.f;
-        for (int s = 0; s < splits; s++) v += partial[(b * splits + s) * len + i];
+        float v = dma::sum_slices(partial + b * splits * len + i, len, splits, 0.f);
         float *o = out + b * o_stride + i;
         if (accumulate) v += *o;
         *o = v;
@@ -370,8 +468,7 @@ __global__ __launch_bounds__(256) void k_split_sum(const float *__restrict__ par
         const int64_t c = e - batch * len;
         if (c < batch * n) {
             const int64_t b = c / n, j = c % n;
-            float v = 0.f;
-            for (int s = 0; s < splits; s++) v += cs_part[(b * splits + s) * n + j];
+            const float v = dma::sum_slices(cs_part + b * splits * n + j, n, splits, 0.f);
             cs_dst[b * cs_stride + j] += v;
         }
     }
@@ -379,40 +476,29 @@ __global__ __launch_bounds__(256) void k_split_sum(const float *__restrict__ par
 
 using KernelFn = void (*)(GemmArgs);
 
-template <int BM, int BN, int BK, bool F16>
-KernelFn pick_kernel(bool ta, bool tb, bool fast) {
-#define ST_K(TA, TB, FA) &k_gemm<BM, BN, BK, TA, TB, F16, FA>
-    if (fast) {
-        if (!ta && !tb) return ST_K(false, false, true);
-        if (!ta && tb) return ST_K(false, true, true);
-        if (ta && !tb) return ST_K(true, false, true);
-        return ST_K(true, true, true);
-    }
-    if (!ta && !tb) return ST_K(false, false, false);
-    if (!ta && tb) return ST_K(false, true, false);
-    if (ta && !tb) return ST_K(true, false, false);
-    return ST_K(true, true, false);
-#undef ST_K
+template <int BM, int BN, int BK, bool F16, bool WHOLE>
+KernelFn pick_trans(bool ta, bool tb) {
+    if (!ta && !tb) return &k_gemm<BM, BN, BK, false, false, F16, WHOLE>;
+    if (!ta && tb) return &k_gemm<BM, BN, BK, false, true, F16, WHOLE>;
+    if (ta && !tb) return &k_gemm<BM, BN, BK, true, false, F16, WHOLE>;
+    return &k_gemm<BM, BN, BK, true, true, F16, WHOLE>;
 }
 
 struct TileCfg {
     int bm, bn;
+    int64_t splits, slice_k;
 };
 
+template <int BK, bool F16>
+KernelFn pick_kernel(const TileCfg &tc, bool ta, bool tb, bool whole) {
+    if (!whole) return pick_trans<32, 32, BK, F16, false>(ta, tb);
+    if (tc.bm == 128 && tc.bn == 128) return pick_trans<128, 128, BK, F16, true>(ta, tb);
+    if (tc.bm == 128) return pick_trans<128, 64, BK, F16, true>(ta, tb);
+    if (tc.bm == 64) return pick_trans<64, 64, BK, F16, true>(ta, tb);
+    return pick_trans<32, 32, BK, F16, true>(ta, tb);
+}
+
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
-// Output tile for a problem: the largest of 128x128, 128x64, 64x64 that gives
-// at least one wave of workgroups (256 CUs), else 64x64.
-TileCfg choose_tile(int64_t batch, int64_t m, int64_t n) {
-    const int64_t cus = 256;
-    if (batch * cdiv(m, 128) * cdiv(n, 128) >= cus) return {128, 128};
-    if (batch * cdiv(m, 128) * cdiv(n, 64) >= cus) return {128, 64};
-    return {64, 64};
-}
-
-bool aligned4(const float *p, int64_t off, int64_t stride, int64_t inner, int64_t ld) {
-    return ((reinterpret_cast<uintptr_t>(p + off) & 15) == 0) && stride % 4 == 0 && inner % 4 == 0 && ld % 4 == 0;
-}
 
 st_status check_ref(const st_matref *r, const char *what) {
     if (!r) return st::fail(ST_ERR_INVALID, "%s is NULL", what);
@@ -481,23 +567,63 @@ st::DmaGemm make_dma(const st_matref *a, const st_matref *b, const st_matref *ou
     return d;
 }
 
-// Split-k of the any-shape kernel, as the reference allows it
-// (matmul.rs:117-123): no epilogue but +=, packed out, and only when the
-// output tiles alone leave CUs idle.  Enough slices to give every CU a
-// workgroup, each keeping at least 4 k-stages.
-void kgemm_splits(const TileCfg &tc, int BK, const st_epilogue &epi, const st_matref *out, int64_t batch, int64_t m,
-                  int64_t k, int64_t n, int64_t &splits, int64_t &slice_k) {
-    const int64_t tiles = batch * cdiv(m, tc.bm) * cdiv(n, tc.bn);
-    const int64_t og = out->group > 0 ? out->group : 1;
+// Output tile and split-k of the any-shape kernel, by an estimate of the time.
+// A workgroup alone on its CU takes `alone` us per k-stage (its matrix-core time
+// plus the LDS round and barrier that nothing hides); W workgroups per CU
+// overlap and take W `shared` per stage; `lead` stages stand for each
+// workgroup's first loads and its stores.  The constants are fitted to f32
+// products from 64 x 80 x 64 (20 workgroups of 32 x 32: 5.0 us, 64 x 64: 8.2) to
+// 3001 x 1003 x 2000 (32 x 32: 150 us, 64 x 64: 120, 128 x 64: 129, 128 x 128:
+// 152) and agree with them to about 15 %; the f16 ones, where a stage is
+// bound by its loads and conversions, to f16 shapes.
+// Split-k as the reference allows it (matmul.rs:117-123): no epilogue but +=,
+// packed out; each slice at least 4 k-stages, the partials summed by a launch of
+// its own.
+TileCfg plan_tiles(bool f16, bool ta, bool tb, const st_epilogue &epi, const st_matref *out, int64_t batch, int64_t m, int64_t k,
+                   int64_t n) {
+    struct Cand {
+        int bm, bn;
+        double alone, shared, lead;        // us per 32-deep f32 stage
+        double alone16, shared16, lead16;  // us per 64-deep f16 stage
+    };
+    // 32 x 32 tiles of operands whose rows are contiguous load with a quarter of the threads.
+    const double narrow = ta && !tb ? 1.45 : ta || !tb ? 1.1 : 1.0;
+    const Cand cands[] = {{128, 128, 2.46, 2.05, 3.0, 1.4, 1.3, 8.0},
+                          {128, 64, 1.38, 1.28, 3.0, 0.76, 0.53, 8.0},
+                          {64, 64, 0.80, 0.59, 3.0, 0.56, 0.33, 8.0},
+                          {32, 32, 0.36, 0.19 * narrow, 1.5, 0.29, 0.145, 8.0}};
+    const int BK = f16 ? 64 : 32;
     const bool epi_free = !epi.bias && !epi.relu && !epi.mask && !epi.residual;
-    const bool packed_out = (out->ld == 0 || out->ld == n) && og == 1;
-    splits = 1;
+    const bool packed_out = (out->ld == 0 || out->ld == n) && out->group <= 1;
     const int64_t cus = 256;
-    if (epi_free && packed_out && tiles < cus)
-        splits = std::max<int64_t>(1, std::min<int64_t>(cdiv(cus, tiles), k / (4 * BK)));
-    slice_k = cdiv(cdiv(k, splits), BK) * BK;
-    if (slice_k == 0) slice_k = BK;
-    splits = std::max<int64_t>(1, cdiv(k, slice_k));
+    // Only products whose 64 x 64 tiles leave CUs idle are split, into slices
+    // that give every CU one or, for small outputs, more (8 MB of partials).
+    const int64_t tiles64 = batch * cdiv(m, 64) * cdiv(n, 64);
+    int64_t most = 1;
+    if (epi_free && packed_out && tiles64 < cus) {
+        const int64_t part = (int64_t)sizeof(float) * batch * (m * n + (epi.has_col_sum ? n : 0));
+        most = std::max<int64_t>(1, std::min<int64_t>(std::max(cdiv(cus, tiles64), (8 << 20) / part), k / (4 * BK)));
+    }
+    TileCfg best = {32, 32, 1, std::max<int64_t>(1, cdiv(k, BK)) * BK};
+    double best_t = -1;
+    for (const Cand &c : cands) {
+        if (c.bm > 32 && (m < c.bm || n < c.bn)) continue;  // (see WHOLE)
+        const int64_t tiles = batch * cdiv(m, c.bm) * cdiv(n, c.bn);
+        for (int64_t sp = 1; sp <= most; sp++) {
+            const int64_t slice = std::max<int64_t>(1, cdiv(cdiv(k, sp), BK)) * BK;
+            const int64_t splits = std::max<int64_t>(1, cdiv(k, slice));
+            if (splits != sp) continue;
+            const double stages = (double)(slice / BK), w = (double)cdiv(tiles * splits, cus);
+            const double per_wg = stages + (f16 ? c.lead16 : c.lead);
+            double t = per_wg * std::max(f16 ? c.alone16 : c.alone, w * (f16 ? c.shared16 : c.shared));
+            if (splits > 1) t += 3.0 + 8.0 * (double)(splits * batch * m * n) / 4e6;
+            if (best_t < 0 || t < best_t) {
+                best_t = t;
+                best = {c.bm, c.bn, splits, slice};
+            }
+        }
+    }
+    return best;
 }
 
 // Bytes of split-k scratch gemm_impl would request for these arguments (0
@@ -510,9 +636,7 @@ size_t gemm_impl_scratch(const st_matref *a, const st_matref *b, const st_matref
     const st::DmaGemm d = make_dma(a, b, out, batch, m, k, n, epi, f16);
     size_t dma = 0;
     if ((dma = st::gemm_dma_scratch(d)) || st::gemm_dma_takes(d)) return dma;
-    const TileCfg tc = choose_tile(batch, m, n);
-    int64_t splits = 1, slice_k = 0;
-    kgemm_splits(tc, f16 ? 64 : 32, epi, out, batch, m, k, n, splits, slice_k);
+    const int64_t splits = plan_tiles(f16, a->trans, b->trans, epi, out, batch, m, k, n).splits;
     if (splits <= 1) return 0;
     return sizeof(float) * (size_t)(batch * splits * m * n + (epi.has_col_sum ? batch * splits * n : 0));
 }
@@ -541,12 +665,10 @@ st_status gemm_impl(const st_matref *a, const st_matref *b, const st_matref *out
         if (st::gemm_dma(make_dma(a, b, out, batch, m, k, n, epi, f16), stream, &ds)) return ds;
     }
 
-    TileCfg tc = choose_tile(batch, m, n);
-    const int BK = f16 ? 64 : 32;
-    int64_t splits = 1, slice_k = 0;
-    kgemm_splits(tc, BK, epi, out, batch, m, k, n, splits, slice_k);
+    const TileCfg tc = plan_tiles(f16, a->trans, b->trans, epi, out, batch, m, k, n);
+    const int64_t splits = tc.splits, slice_k = tc.slice_k;
     if (batch * splits > 65535) return st::fail(ST_ERR_INVALID, "batch %lld too large for one launch", (long long)batch);
-    if (cdiv(m, tc.bm) > 65535) return st::fail(ST_ERR_INVALID, "m = %lld too large for one launch", (long long)m);
+    if (cdiv(m, 128) > 65535) return st::fail(ST_ERR_INVALID, "m = %lld too large for one launch", (long long)m);
 
     GemmArgs g;
     std::memset(&g, 0, sizeof g);
@@ -591,19 +713,12 @@ st_status gemm_impl(const st_matref *a, const st_matref *b, const st_matref *out
         g.cs_direct = 1;
     }
 
-    const bool fast = m % tc.bm == 0 && n % tc.bn == 0 && k % BK == 0 && slice_k % BK == 0 &&
-                      aligned4(a->p, a->off, a->stride, a->inner, lda) && aligned4(b->p, b->off, b->stride, b->inner, ldb);
-    KernelFn fn;
-    if (f16) {
-        if (tc.bm == 128 && tc.bn == 128) fn = pick_kernel<128, 128, 64, true>(a->trans, b->trans, fast);
-        else if (tc.bm == 128) fn = pick_kernel<128, 64, 64, true>(a->trans, b->trans, fast);
-        else fn = pick_kernel<64, 64, 64, true>(a->trans, b->trans, fast);
-    } else {
-        if (tc.bm == 128 && tc.bn == 128) fn = pick_kernel<128, 128, 32, false>(a->trans, b->trans, fast);
-        else if (tc.bm == 128) fn = pick_kernel<128, 64, 32, false>(a->trans, b->trans, fast);
-        else fn = pick_kernel<64, 64, 32, false>(a->trans, b->trans, fast);
-    }
-    dim3 grid((unsigned)cdiv(n, tc.bn), (unsigned)cdiv(m, tc.bm), (unsigned)(batch * splits));
+    const bool whole = m >= tc.bm && n >= tc.bn;
+    const KernelFn fn = f16 ? pick_kernel<64, true>(tc, a->trans, b->trans, whole)
+                            : pick_kernel<32, false>(tc, a->trans, b->trans, whole);
+    const int64_t tiles = cdiv(n, tc.bn) * cdiv(m, tc.bm);
+    if (tiles > INT32_MAX / THREADS) return st::fail(ST_ERR_INVALID, "m = %lld too large for one launch", (long long)m);
+    dim3 grid((unsigned)tiles, 1, (unsigned)(batch * splits));
     hipLaunchKernelGGL(fn, grid, dim3(THREADS), 0, stream, g);
     ST_LAUNCH_CHECK();
 

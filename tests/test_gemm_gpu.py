@@ -265,6 +265,23 @@ def tape_forms(dev, m, k, n, use_f16, seed):
             assert rel_err(g, want32) <= 2e-3, (name, m, k, n)
 
 
+# The any-shape kernel around its tile edges (32, 64 and 128 rows and columns, k-stages of 32 and 64): last tiles
+# moved back to the edge, fewer rows or columns than a tile, a partial first k-stage; odd offsets and strides.  The
+# last f32 shapes are large enough for 128-row tiles, the last f16 ones for each tile.
+EDGE_F32 = [(1, 1, 1), (3, 5, 2), (31, 2, 33), (32, 31, 32), (33, 32, 31), (64, 33, 63), (65, 64, 64), (127, 65, 32),
+            (33, 1, 129), (200, 80, 200), (97, 300, 4), (1, 257, 130), (2500, 33, 2300), (1300, 3, 700)]
+EDGE_F16 = [(64, 32, 32), (64, 96, 160), (192, 64, 96), (320, 160, 1056), (4096, 32, 1056), (6400, 64, 1120)]
+
+
+@pytest.mark.parametrize("route,shape", [(False, s) for s in EDGE_F32] + [(True, s) for s in EDGE_F16])
+def test_any_shape_kernel_at_tile_edges(dev, route, shape):
+    m, k, n = shape
+    batch = 2 if m * n < 10000 else 1
+    for i, (ta, tb) in enumerate([(False, False), (False, True), (True, False), (True, True)]):
+        epi = (True, i % 2 == 0, True, True, True) if i < 3 else (False, False, False, False, True)
+        run_case(dev, 300 + 2 * i, (batch, m, k, n, ta, tb) + epi, route)
+
+
 @pytest.mark.parametrize("use_f16", [False, True])
 def test_tape_forms_256_cube(dev, use_f16):
     tape_forms(dev, 256, 256, 256, use_f16, 42)
