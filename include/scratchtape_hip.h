@@ -292,6 +292,27 @@ st_status st_knn_search_masked_2bit(const uint8_t *codes, const float *scales, i
                                     int64_t nq, int64_t d, int64_t k, int64_t *out_idx,
                                     float *out_dist, st_stream stream);
 
+/* No reference counterpart: the two searches with memory of the caller's for
+ * the candidate lists of a small batch.  st_knn_split_bytes(nq) is what a
+ * batch of nq queries can use (0: nothing).  With `work` (device memory, 8-byte
+ * aligned, at least so large; the call's own until its work on `stream` is done)
+ * a batch too small to give every CU a query is scanned by several workgroups
+ * per query, whose lists a second launch merges.  Without it (NULL, or too
+ * small) these are st_knn_search_ivf_2bit and st_knn_search_masked_2bit.  The
+ * results are the same. */
+int64_t st_knn_split_bytes(int64_t nq);
+st_status st_knn_search_ivf_2bit_split(const uint8_t *codes, const float *scales,
+                                       const int64_t *cell_start, int64_t ncells, int64_t max_cell,
+                                       const float *queries, const int32_t *probes, int64_t nq,
+                                       int64_t nprobe, int64_t d, int64_t k, int64_t *out_idx,
+                                       float *out_dist, void *work, int64_t work_bytes,
+                                       st_stream stream);
+st_status st_knn_search_masked_2bit_split(const uint8_t *codes, const float *scales, int64_t nkeys,
+                                          const float *queries, const int64_t *lohi, int64_t always,
+                                          int64_t nq, int64_t d, int64_t k, int64_t *out_idx,
+                                          float *out_dist, void *work, int64_t work_bytes,
+                                          st_stream stream);
+
 /* Benchmark support, no reference counterpart: fills rows [row0, row0 + n)
  * of a synthetic 2-bit store with keys drawn N(0,1) from a counter-based
  * generator (seed, global row, component) and quantised as

@@ -311,6 +311,43 @@ extern "C" {
         out_dist: *mut f32,
         stream: st_stream,
     ) -> st_status;
+    /// The two searches with the caller's memory for the candidate lists of a small batch
+    /// (`st_knn_split_bytes(nq)` bytes), whose queries are then scanned by several workgroups each.
+    pub fn st_knn_split_bytes(nq: i64) -> i64;
+    pub fn st_knn_search_ivf_2bit_split(
+        codes: *const u8,
+        scales: *const f32,
+        cell_start: *const i64,
+        ncells: i64,
+        max_cell: i64,
+        queries: *const f32,
+        probes: *const i32,
+        nq: i64,
+        nprobe: i64,
+        d: i64,
+        k: i64,
+        out_idx: *mut i64,
+        out_dist: *mut f32,
+        work: *mut c_void,
+        work_bytes: i64,
+        stream: st_stream,
+    ) -> st_status;
+    pub fn st_knn_search_masked_2bit_split(
+        codes: *const u8,
+        scales: *const f32,
+        nkeys: i64,
+        queries: *const f32,
+        lohi: *const i64,
+        always: i64,
+        nq: i64,
+        d: i64,
+        k: i64,
+        out_idx: *mut i64,
+        out_dist: *mut f32,
+        work: *mut c_void,
+        work_bytes: i64,
+        stream: st_stream,
+    ) -> st_status;
     /// Synthetic stores of the reference's seeded generator (benchmark and test support).
     pub fn st_knn_synth_store_2bit(
         seed: u64,

@@ -69,6 +69,10 @@ SIGNATURES = {
     "st_attention_fused_bwd": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _f32, _vp],
     "st_knn_quantize_2bit": [_vp, _i64, _i64, _vp, _vp, _vp],
     "st_knn_search_ivf_2bit": [_vp, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp],
+    "st_knn_split_bytes": [_i64],
+    "st_knn_search_ivf_2bit_split": [_vp, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _i64,
+                                     _vp],
+    "st_knn_search_masked_2bit_split": [_vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp],
     "st_knn_key_norms_2bit": [_vp, _vp, _i64, _i64, _vp, _vp],
     "st_knn_set_scan_order": [_i32],
     "st_knn_search_masked_2bit": [_vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp],
@@ -88,7 +92,7 @@ SIGNATURES = {
     "st_version": [],
 }
 _RESTYPES = {"st_last_error": ctypes.c_char_p, "st_version": ctypes.c_char_p, "st_f16_enabled": _i32,
-             "st_knn_centroid_digit_bytes": _i64}
+             "st_knn_centroid_digit_bytes": _i64, "st_knn_split_bytes": _i64}
 
 _lib = None
 

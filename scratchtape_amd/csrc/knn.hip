@@ -554,17 +554,33 @@ __device__ __attribute__((noinline)) Kept merge_new_keys(lds_u64 *wl, int na, in
     return k;
 }
 
-// grid: one workgroup of 1024 threads per query.  IVF mode (MASKED false):
+// grid: nsplit workgroups of 512 threads per query.  IVF mode (MASKED false):
 // the query scans its probed cells (probes, cell_start).  MASKED: it scans
 // the keys g < always and lo <= g < hi of the store's nkeys (lohi [nq, 2]),
 // as two row segments; cell_start, probes, ncells and nprobe are unused.
+//
+// nsplit == 1: the workgroup writes the query's results.  nsplit > 1 (few
+// queries: one workgroup each would leave most CUs idle): workgroup s scans
+// the s-th run of the query's chunks, at least SPLIT_MIN of them, and writes
+// its k smallest keys, sorted and NONE-padded, to parts[(q nsplit + s) KMAX];
+// workgroup 0 writes the number of runs to runs[q], and k_merge_splits combines
+// their lists.  A query of one run is finished by workgroup 0.  The k smallest
+// keys of the whole lie among the runs' k smallest, so the results are the
+// same.  Bound by latency: about 25 us from launch to output for any run (first
+// loads 4, the two merges of each wave's list 3 each, barriers, the final ranks
+// 1 to 5), then 0.7 us per chunk and wave.  4 queries of 1,270 chunks: 203 us
+// unsplit, 36 in 32 runs with the merge; 32 queries of 330: 60 and 39.
+constexpr int SPLIT_MIN = 4 * SW;  // chunks per run (four per wave)
+constexpr int SPLIT_MAX = 32;      // runs per query
+
 template <bool MASKED>
 __global__ __launch_bounds__(STH) void k_search(const uint8_t *codes, const float *scales,
                                                 const int64_t *__restrict__ cell_start, int64_t ncells,
                                                 const float *__restrict__ queries, const int32_t *__restrict__ probes,
                                                 int32_t nq, int32_t nprobe, int32_t k, int64_t *__restrict__ out_idx,
                                                 float *__restrict__ out_dist, const int64_t *__restrict__ lohi,
-                                                int64_t always, int64_t nkeys) {
+                                                int64_t always, int64_t nkeys, int32_t nsplit,
+                                                uint64_t *__restrict__ parts, int32_t *__restrict__ runs) {
     __shared__ uint64_t cand[SW * CAPW];  // per-wave candidate lists
     __shared__ uint64_t fin[SW * KMAX];   // the final gather
     __shared__ uint64_t s_tau;            // shared threshold (only decreases)
@@ -576,7 +592,8 @@ __global__ __launch_bounds__(STH) void k_search(const uint8_t *codes, const floa
     __shared__ int32_t s_len[PROBE_MAX], s_cpre[PROBE_MAX + 1];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int64_t q = blockIdx.x;
+    const int64_t q = blockIdx.x / (uint32_t)nsplit;
+    const int32_t split = (int32_t)(blockIdx.x % (uint32_t)nsplit);
 
     if (wave == 0) {
         const QInfo qi = quantize_query(queries + q * D, lane, s_Q);
@@ -650,14 +667,22 @@ __global__ __launch_bounds__(STH) void k_search(const uint8_t *codes, const floa
     }
     __syncthreads();
 
+    // This workgroup's run of chunks, [begin, nchunks) (uniform).
+    const int np = s_np;
+    const int64_t nrows = s_nrows;
+    const int32_t all = s_cpre[np];
+    const int32_t run = nsplit == 1 ? all : max(SPLIT_MIN, (all + nsplit - 1) / nsplit);
+    const bool last = all <= run;  // one run: this query's results are written here
+    const int32_t begin = split * run;  // split * run < 2^31: run <= nchunks / nsplit + SPLIT_MIN
+    const int32_t nchunks = min(all, begin + run);
+    if (split > 0 && begin >= all) return;
+    if (nsplit > 1 && split == 0 && tid == 0) runs[q] = last ? 1 : (all + run - 1) / run;
+
     const int row = lane >> 4, col = lane & 15;
     v8i aq[2];
     build_aq(s_Q, 1, row, col, aq);
     const float qs = s_qs;
     const int32_t sq = s_sq;
-    const int np = s_np;
-    const int32_t nchunks = s_cpre[np];
-    const int64_t nrows = s_nrows;
     const int32_t c2_base = 9 * D;
 
     // The waves take chunks of the query's cells (taken in order) from a
@@ -670,12 +695,12 @@ __global__ __launch_bounds__(STH) void k_search(const uint8_t *codes, const floa
     int ccell = 0;
     int32_t c0 = 0;
     while (c0 < np - 1 && s_cpre[c0 + 1] == 0) c0++;
-    const int64_t safe_row0 = nchunks > 0 ? s_r0[c0] : 0;
+    const int64_t safe_row0 = all > 0 ? s_r0[c0] : 0;
     auto fetch = [&](auto small, Chunk &ch) {
         constexpr bool SMALL = decltype(small)::value;
         int32_t gl = 0;
         if (lane == 0) gl = atomicAdd(&s_next, 1);
-        const int32_t g = __builtin_amdgcn_readfirstlane(gl);
+        const int32_t g = begin + __builtin_amdgcn_readfirstlane(gl);
         ch.g = g;
         while (ccell < np - 1 && g >= s_cpre[ccell + 1]) ccell++;
         const bool live = g < nchunks;
@@ -785,7 +810,7 @@ __global__ __launch_bounds__(STH) void k_search(const uint8_t *codes, const floa
             }
         }
     };
-    if (nchunks > 0) {  // uniform over the workgroup
+    if (nchunks > begin) {  // uniform over the workgroup
         if (nrows < 64)
             scan(std::integral_constant<bool, true>());
         else
@@ -813,15 +838,93 @@ __global__ __launch_bounds__(STH) void k_search(const uint8_t *codes, const floa
         const uint64_t e = fin[t];
         int r = 0;
         for (int j = 0; j < cnt; j++) r += fin[j] < e;
-        if (r < k) {
+        if (r < k && !last) {
+            parts[(int64_t)blockIdx.x * KMAX + r] = e;
+        } else if (r < k) {
             const float v = qn + unfkey((uint32_t)(e >> 32));
             out_idx[q * k + r] = (int64_t)(uint32_t)e;
             out_dist[q * k + r] = v > 0.f ? v : 0.f;
         }
     }
     for (int j = cnt + tid; j < k; j += STH) {
-        out_idx[q * k + j] = -1;
-        out_dist[q * k + j] = __builtin_inff();
+        if (!last) {
+            parts[(int64_t)blockIdx.x * KMAX + j] = NONE;
+        } else {
+            out_idx[q * k + j] = -1;
+            out_dist[q * k + j] = __builtin_inff();
+        }
+    }
+}
+
+// grid: one workgroup of MTH threads per query.  Combines the query's nsplit
+// sorted lists of k keys (parts, as k_search writes them): each wave merges
+// every MW-th list into its own (the minimum of each of its keys and the
+// list's mirrored key is a bitonic sequence holding the KMAX smallest of both;
+// a bitonic merge sorts it), all lists' loads in flight together, then the
+// waves' lists are merged pairwise in LDS.  The time does not depend on how
+// the keys lie over the lists (gathering the keys below a bound taken from the
+// lists and ranking them took 6 us, or 305 us with one short list).
+constexpr int MW = 8;
+constexpr int MTH = MW * 64;
+__global__ __launch_bounds__(MTH) void k_merge_splits(const uint64_t *__restrict__ parts,
+                                                      const int32_t *__restrict__ runs, const float *__restrict__ queries, int32_t nsplit, int32_t k,
+                                                      int64_t *__restrict__ out_idx, float *__restrict__ out_dist) {
+    __shared__ uint64_t lists[MW][KMAX];
+    __shared__ int16_t sQ[D];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t q = blockIdx.x;
+    const uint64_t *P = parts + q * nsplit * KMAX;
+    const int n = runs[q];  // lists in use
+    if (n <= 1) return;     // k_search wrote the results
+    constexpr int PER = SPLIT_MAX / MW;
+    // Element 64 r + lane of the wave's first list, and of the others mirrored.
+    uint64_t x[PER][2];
+#pragma unroll
+    for (int i = 0; i < PER; i++)
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const int l = wave + MW * i, e = i == 0 ? 64 * r + lane : KMAX - 1 - (64 * r + lane);
+            x[i][r] = l < n && e < k ? P[l * KMAX + e] : NONE;
+        }
+    float qn = 0.f;
+    if (wave == 0) qn = quantize_query(queries + q * D, lane, sQ).qn;
+    uint64_t c[2] = {x[0][0], x[0][1]};
+#pragma unroll
+    for (int i = 1; i < PER; i++) {
+        if (wave + MW * i >= n) break;  // uniform over the wave
+#pragma unroll
+        for (int r = 0; r < 2; r++) c[r] = c[r] < x[i][r] ? c[r] : x[i][r];
+        bitonic_stage<2, 128, 64>(c, lane);
+    }
+#pragma unroll
+    for (int step = 1; step < MW; step <<= 1) {
+        if ((wave & (2 * step - 1)) == step) {
+            lists[wave][lane] = c[0];
+            lists[wave][64 + lane] = c[1];
+        }
+        __syncthreads();
+        if ((wave & (2 * step - 1)) == 0 && wave + step < n) {
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                const uint64_t b = lists[wave + step][KMAX - 1 - (64 * r + lane)];
+                c[r] = c[r] < b ? c[r] : b;
+            }
+            bitonic_stage<2, 128, 64>(c, lane);
+        }
+    }
+    if (wave != 0) return;
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const int rank = 64 * r + lane;
+        if (rank >= k) continue;
+        if (c[r] != NONE) {
+            const float v = qn + unfkey((uint32_t)(c[r] >> 32));
+            out_idx[q * k + rank] = (int64_t)(uint32_t)c[r];
+            out_dist[q * k + rank] = v > 0.f ? v : 0.f;
+        } else {
+            out_idx[q * k + rank] = -1;
+            out_dist[q * k + rank] = __builtin_inff();
+        }
     }
 }
 
@@ -1295,10 +1398,59 @@ extern "C" st_status st_knn_synth_keys_f32(uint64_t seed, int64_t row0, int64_t 
     return ST_OK;
 }
 
+// Workgroups per query of a query-major scan of nq queries that has memory for
+// their lists: one per CU in all.  20 queries' worth of runs of 40 chunks each
+// take 36 us, merge included, where one workgroup per query takes 118 to 200;
+// two per CU (512 in all) measured 51 against 36 us at 16 queries of 632
+// chunks, 61 against 56 at 64, and 74 against 79 at 100.
+static int64_t query_splits(int64_t nq) {
+    const int64_t n = nq > 0 ? 256 / nq : 1;
+    return n < 2 ? 1 : std::min<int64_t>(n, SPLIT_MAX);
+}
+
+// The lists, then each query's number of runs.
+extern "C" int64_t st_knn_split_bytes(int64_t nq) {
+    const int64_t s = query_splits(nq);
+    return s > 1 ? nq * (s * KMAX + 1) * (int64_t)sizeof(uint64_t) : 0;
+}
+
+struct SplitWork {
+    int64_t nsplit;
+    uint64_t *parts;
+    int32_t *runs;
+};
+
+// The split of nq queries in the caller's memory, when it is large enough.
+static SplitWork split_work(void *work, int64_t work_bytes, int64_t nq) {
+    if (!work || work_bytes < st_knn_split_bytes(nq) || (reinterpret_cast<uintptr_t>(work) & 7) != 0)
+        return {1, nullptr, nullptr};
+    const int64_t s = query_splits(nq);
+    uint64_t *parts = static_cast<uint64_t *>(work);
+    return {s, parts, reinterpret_cast<int32_t *>(parts + nq * s * KMAX)};
+}
+
+// Combines the lists of a split scan (k_search with nsplit > 1).
+static st_status merge_splits(const SplitWork &w, const float *queries, int64_t nq, int64_t k, int64_t *out_idx,
+                              float *out_dist, hipStream_t s) {
+    hipLaunchKernelGGL(k_merge_splits, dim3((unsigned)nq), dim3(MTH), 0, s, w.parts, w.runs, queries,
+                       (int32_t)w.nsplit, (int32_t)k, out_idx, out_dist);
+    ST_LAUNCH_CHECK();
+    return ST_OK;
+}
+
 extern "C" st_status st_knn_search_ivf_2bit(const uint8_t *codes, const float *scales, const int64_t *cell_start,
                                             int64_t ncells, int64_t max_cell, const float *queries,
                                             const int32_t *probes, int64_t nq, int64_t nprobe, int64_t d,
                                             int64_t k, int64_t *out_idx, float *out_dist, st_stream stream) {
+    return st_knn_search_ivf_2bit_split(codes, scales, cell_start, ncells, max_cell, queries, probes, nq, nprobe, d, k,
+                                        out_idx, out_dist, nullptr, 0, stream);
+}
+
+extern "C" st_status st_knn_search_ivf_2bit_split(const uint8_t *codes, const float *scales,
+                                                  const int64_t *cell_start, int64_t ncells, int64_t max_cell,
+                                                  const float *queries, const int32_t *probes, int64_t nq,
+                                                  int64_t nprobe, int64_t d, int64_t k, int64_t *out_idx,
+                                                  float *out_dist, void *work, int64_t work_bytes, st_stream stream) {
     st::clear_error();
     if (!codes || !scales || !cell_start || !queries || !probes || !out_idx || !out_dist)
         return st::fail(ST_ERR_INVALID, "search_ivf: NULL buffer");
@@ -1322,11 +1474,14 @@ extern "C" st_status st_knn_search_ivf_2bit(const uint8_t *codes, const float *s
     const int64_t npairs = nq * nprobe;
     const bool cells = g_scan_order == 2 || (g_scan_order == 0 && 3 * npairs >= 2 * ncells);
     if (!cells) {
-        hipLaunchKernelGGL(k_search<false>, dim3((unsigned)nq), dim3(STH), 0, s, codes, scales, cell_start, ncells,
-                           queries, probes, (int32_t)nq, (int32_t)nprobe, (int32_t)k, out_idx, out_dist, nullptr,
-                           (int64_t)0, (int64_t)0);
+        // Cells too small for that many runs (max_cell bounds them) give fewer.
+        SplitWork w = split_work(work, work_bytes, nq);
+        w.nsplit = std::max<int64_t>(1, std::min(w.nsplit, nprobe * cdiv(max_cell, 64) / SPLIT_MIN));
+        hipLaunchKernelGGL(k_search<false>, dim3((unsigned)(nq * w.nsplit)), dim3(STH), 0, s, codes, scales,
+                           cell_start, ncells, queries, probes, (int32_t)nq, (int32_t)nprobe, (int32_t)k, out_idx,
+                           out_dist, nullptr, (int64_t)0, (int64_t)0, (int32_t)w.nsplit, w.parts, w.runs);
         ST_LAUNCH_CHECK();
-        return ST_OK;
+        return w.nsplit > 1 ? merge_splits(w, queries, nq, k, out_idx, out_dist, s) : ST_OK;
     }
     if (ncells > INT32_MAX) return st::fail(ST_ERR_INVALID, "search_ivf: too many cells for the cell-major scan");
     // Scratch: per-cell counts, fill counters and unit offsets, the unit
@@ -1374,6 +1529,15 @@ extern "C" st_status st_knn_search_masked_2bit(const uint8_t *codes, const float
                                                const float *queries, const int64_t *lohi, int64_t always,
                                                int64_t nq, int64_t d, int64_t k, int64_t *out_idx, float *out_dist,
                                                st_stream stream) {
+    return st_knn_search_masked_2bit_split(codes, scales, nkeys, queries, lohi, always, nq, d, k, out_idx, out_dist,
+                                           nullptr, 0, stream);
+}
+
+extern "C" st_status st_knn_search_masked_2bit_split(const uint8_t *codes, const float *scales, int64_t nkeys,
+                                                     const float *queries, const int64_t *lohi, int64_t always,
+                                                     int64_t nq, int64_t d, int64_t k, int64_t *out_idx,
+                                                     float *out_dist, void *work, int64_t work_bytes,
+                                                     st_stream stream) {
     st::clear_error();
     if (!codes || !scales || !queries || !lohi || !out_idx || !out_dist)
         return st::fail(ST_ERR_INVALID, "search_masked: NULL buffer");
@@ -1389,9 +1553,14 @@ extern "C" st_status st_knn_search_masked_2bit(const uint8_t *codes, const float
     if (nq == 0) return ST_OK;
     if (nq > INT32_MAX) return st::fail(ST_ERR_INVALID, "search_masked: too many queries for one call");
     if (!st::device_ok()) return ST_ERR_NO_DEVICE;
-    hipLaunchKernelGGL(k_search<true>, dim3((unsigned)nq), dim3(STH), 0, st::stream_of(stream), codes, scales,
-                       nullptr, (int64_t)0, queries, nullptr, (int32_t)nq, 0, (int32_t)k, out_idx, out_dist, lohi,
-                       always, nkeys);
+    // The ranges are on the device: every query is split as if it saw the whole
+    // store, and the workgroups past its last run end at once.
+    const hipStream_t s = st::stream_of(stream);
+    SplitWork w = split_work(work, work_bytes, nq);
+    w.nsplit = std::max<int64_t>(1, std::min(w.nsplit, cdiv(nkeys, 64) / SPLIT_MIN));
+    hipLaunchKernelGGL(k_search<true>, dim3((unsigned)(nq * w.nsplit)), dim3(STH), 0, s, codes, scales, nullptr,
+                       (int64_t)0, queries, nullptr, (int32_t)nq, 0, (int32_t)k, out_idx, out_dist, lohi, always,
+                       nkeys, (int32_t)w.nsplit, w.parts, w.runs);
     ST_LAUNCH_CHECK();
-    return ST_OK;
+    return w.nsplit > 1 ? merge_splits(w, queries, nq, k, out_idx, out_dist, s) : ST_OK;
 }

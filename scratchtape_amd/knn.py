@@ -116,6 +116,17 @@ def _check_out(out, nq: int, k: int, device) -> Tuple[torch.Tensor, torch.Tensor
     return idx, dist
 
 
+def _split_work(nq: int, device, stream) -> Tuple[Optional[torch.Tensor], int, int]:
+    """Memory for a small batch's candidate lists (st_knn_split_bytes): the tensor (held by the caller until its launch
+    is enqueued), its address and its size.  It is an allocation of the current stream, which keeps it until the work
+    enqueued there is done, so a call on another stream gets none."""
+    nbytes = int(_lib.lib().st_knn_split_bytes(nq))
+    if nbytes <= 0 or (stream is not None and _stream(stream) != _stream(None)):
+        return None, 0, 0
+    work = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    return work, work.data_ptr(), nbytes
+
+
 class KnnStore2bit:
     """A cell-contiguous 2-bit key store on the device.
 
@@ -178,11 +189,12 @@ class KnnStore2bit:
             dist = torch.empty((nq, k), dtype=torch.float32, device=queries.device)
         else:
             idx, dist = _check_out(out, nq, k, queries.device)
-        _lib.call("st_knn_search_ivf_2bit", _dptr(self.codes, torch.uint8, "codes"),
+        work, wptr, wbytes = _split_work(nq, queries.device, stream)
+        _lib.call("st_knn_search_ivf_2bit_split", _dptr(self.codes, torch.uint8, "codes"),
                   _dptr(self.scales, torch.float32, "scales"), self.cell_start_dev.data_ptr(), self.ncells,
                   self.max_cell, _dptr(queries, torch.float32, "queries"), _dptr(probes, torch.int32, "probes"),
                   nq, nprobe, d, k, _dptr(idx, torch.int64, "idx"), _dptr(dist, torch.float32, "dist"),
-                  _stream(stream))
+                  wptr, wbytes, _stream(stream))
         return idx, dist
 
     def search_masked(self, queries: torch.Tensor, lohi: torch.Tensor, always: int = 0, k: int = KMAX,
@@ -199,8 +211,9 @@ class KnnStore2bit:
             dist = torch.empty((nq, k), dtype=torch.float32, device=queries.device)
         else:
             idx, dist = _check_out(out, nq, k, queries.device)
-        _lib.call("st_knn_search_masked_2bit", _dptr(self.codes, torch.uint8, "codes"),
+        work, wptr, wbytes = _split_work(nq, queries.device, stream)
+        _lib.call("st_knn_search_masked_2bit_split", _dptr(self.codes, torch.uint8, "codes"),
                   _dptr(self.scales, torch.float32, "scales"), len(self), _dptr(queries, torch.float32, "queries"),
                   _dptr(lohi, torch.int64, "lohi"), always, nq, d, k, _dptr(idx, torch.int64, "idx"),
-                  _dptr(dist, torch.float32, "dist"), _stream(stream))
+                  _dptr(dist, torch.float32, "dist"), wptr, wbytes, _stream(stream))
         return idx, dist

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import oracle
-from scratchtape_amd import knn
+from scratchtape_amd import _lib, knn
 
 pytestmark = pytest.mark.gpu
 D = 256
@@ -325,6 +325,51 @@ def test_masked_search_matches_oracle(dev, always, k):
     lohi = torch.from_numpy(np.stack([lo, hi], 1).astype(np.int64)).to(dev)
     idx, dist = store.search_masked(torch.from_numpy(queries).to(dev), lohi, always, k)
     widx, wdist = oracle.knn_search_masked(codes, scales, queries, lo, hi, always, k)
+    np.testing.assert_array_equal(idx.cpu().numpy(), widx)
+    np.testing.assert_array_equal(dist.cpu().numpy(), wdist)
+
+
+def unsplit_masked(store, queries, lohi, always, k):
+    """search_masked through st_knn_search_masked_2bit: one workgroup per query."""
+    nq = queries.shape[0]
+    idx = torch.empty((nq, k), dtype=torch.int64, device=queries.device)
+    dist = torch.empty((nq, k), device=queries.device)
+    _lib.call("st_knn_search_masked_2bit", store.codes.data_ptr(), store.scales.data_ptr(), len(store),
+              queries.data_ptr(), lohi.data_ptr(), always, nq, D, k, idx.data_ptr(), dist.data_ptr(),
+              torch.cuda.current_stream().cuda_stream)
+    return idx, dist
+
+
+# Small batches split a query over several workgroups, in runs of at least 32 chunks of 64 keys: no key, one run, its
+# edge, a second run of one key, many runs, and as many as there can be; 1 query (32 runs at most), 100 (2), 128 (2)
+# and 129 (not split).
+@pytest.mark.parametrize("nq", [1, 9, 100, 128, 129])
+@pytest.mark.parametrize("k", [128, 5])
+def test_split_search_equals_one_workgroup_per_query(dev, nq, k):
+    rng = np.random.default_rng(60 + nq)
+    n, always = 90000, 130
+    codes = torch.empty((n, D // 4), dtype=torch.uint8, device=dev)
+    scales = torch.empty(n, dtype=torch.float32, device=dev)
+    knn.synth_store_2bit(9, 0, codes, scales)
+    order = torch.argsort(scales)  # norms rise with the row: the nearest keys of a query lie in a few runs
+    cuts = np.array([0, 2000, 2048, 2049, 2112, 10000, 10001, 60000, n])
+    store = knn.KnnStore2bit(codes[order].contiguous(), scales[order].contiguous(), cuts)
+    q = torch.from_numpy(rng.standard_normal((nq, D)).astype(np.float32)).to(dev)
+    length = np.array([0, 3, 1900, 2048, 2049, 4096, 30000, 80000])[np.arange(nq) % 8]
+    lo = rng.integers(always, n - length)
+    lohi = torch.from_numpy(np.stack([lo, lo + length], 1)).to(dev)
+    for first in (0, always):
+        got, want = store.search_masked(q, lohi, first, k), unsplit_masked(store, q, lohi, first, k)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    # The same store by cells, each query probing four of them (an empty one, a cell again, whole cells).
+    probes = np.stack([rng.permutation(8)[:4] for _ in range(nq)]).astype(np.int32)
+    probes[0] = [7, 7, 3, -1]
+    knn.set_scan_order(1)
+    try:
+        idx, dist = store.search_ivf(q, torch.from_numpy(probes).to(dev), k)
+    finally:
+        knn.set_scan_order(0)
+    widx, wdist = oracle.knn_search(store.codes.cpu().numpy(), store.scales.cpu().numpy(), cuts, q.cpu().numpy(), probes, k)
     np.testing.assert_array_equal(idx.cpu().numpy(), widx)
     np.testing.assert_array_equal(dist.cpu().numpy(), wdist)
 
