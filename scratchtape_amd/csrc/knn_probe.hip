@@ -57,8 +57,7 @@ constexpr int TILE = 16;                   // vectors per digit tile
 constexpr int TILE_BYTES = TILE * 2 * D;   // 8192
 constexpr int PROBE_MAX = 16;              // ivf.rs:126
 constexpr int QG = 64;                     // queries per k_probe_part workgroup (4 query tiles x 16)
-constexpr int TPS = 12;                    // centroid tiles per slice, at most
-constexpr int HT = TPS / 2;                // tiles per wave (two waves per query tile)
+constexpr int HT_MAX = 6;                  // centroid tiles per wave (two waves per query tile), at most
 constexpr int PART_T = 512;                // k_probe_part threads
 constexpr int CAPQ = 64;                   // candidate slot per (query, slice)
 constexpr int64_t CAND_BUDGET = 256ll << 20;  // bytes of candidate slots per query chunk
@@ -196,15 +195,22 @@ constexpr int32_t INONE = 0x7fffffff;
 // group) = (idx / gy, idx % gy) with idx dealt so that the gy workgroups of a
 // slice are consecutive on one XCD (workgroup ids go round robin over the 8
 // XCDs), which then reads the slice's digits from HBM once.
+//
+// A slice is 2 HT tiles: 12 when there are enough (slice, query group) pairs
+// to fill the chip, fewer for small indexes and batches, where each workgroup
+// is a chain of latencies (staging, scoring, threshold, candidates) and more
+// workgroups shorten it.
+template <int HT>
 __global__ __launch_bounds__(PART_T) void k_probe_part(const float *__restrict__ queries, int32_t nq,
                                                     const int8_t *__restrict__ cdig, const int32_t *__restrict__ cexp,
                                                     const double *__restrict__ cnorm, int32_t nlist, int32_t S,
                                                     int32_t gy, int32_t nprobe, uint64_t *__restrict__ ck,
                                                     int32_t *__restrict__ ci, int32_t *__restrict__ pcnt) {
+    constexpr int TPS = 2 * HT;
     __shared__ v4i s_b[TPS * TILE_BYTES / 16];
     __shared__ double s_cn[TPS * TILE];
     __shared__ int32_t s_ce[TPS * TILE];
-    __shared__ uint32_t s_x[2][4][64][4];  // per (half, query tile, lane, u): minima, then counts
+    __shared__ uint32_t s_x[2][4][64][4];  // per (half, query tile, lane, u): sorted minima, then counts
     __shared__ v4i s_q[4 * TILE_BYTES / 16];  // the workgroup's 64 queries as 4 digit tiles
     __shared__ int32_t s_qe[QG];              // and their exponents
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -220,7 +226,7 @@ __global__ __launch_bounds__(PART_T) void k_probe_part(const float *__restrict__
         const v4i *src = reinterpret_cast<const v4i *>(cdig + (int64_t)t0 * TILE_BYTES);
         const int n16 = nts * (TILE_BYTES / 16);
 #pragma unroll
-        for (int i = 0; i < TPS * TILE_BYTES / 16 / PART_T; i++)
+        for (int i = 0; i < TPS * TILE_BYTES / 16 / PART_T; i++)  // (TILE_BYTES / 16 == PART_T)
             if (i * PART_T + tid < n16) s_b[i * PART_T + tid] = src[i * PART_T + tid];
         if (tid < nts * TILE) {
             const int32_t c = t0 * TILE + tid;
@@ -296,7 +302,7 @@ __global__ __launch_bounds__(PART_T) void k_probe_part(const float *__restrict__
     // The MFMAs of TG tiles at a time, k-step by k-step: TG independent
     // accumulator chains interleaved keep the matrix core busy (each MFMA's
     // input is TG instructions old); the group's keys are formed afterwards.
-    constexpr int TG = 3;
+    constexpr int TG = HT % 3 == 0 ? 3 : HT;
     static_assert(HT % TG == 0, "tile groups");
 #pragma unroll
     for (int g0 = 0; g0 < HT; g0 += TG) {
@@ -343,35 +349,39 @@ __global__ __launch_bounds__(PART_T) void k_probe_part(const float *__restrict__
         }
     }
 
-    // Per query, the nprobe-th smallest of its 16 lanes' minima: for a given u
-    // the 16 lanes of an (h, parity) group hold one query, one per centroid
-    // position c16 (lane bits 1..4), so a bitonic sort over c16 by shuffles
-    // puts the r-th smallest in the group's lane c16 = r.
+    // Per query, the nprobe-th smallest of the 32 minima of its lanes in both
+    // halves: for a given u the 16 lanes of an (h, parity) group hold one
+    // query, one per centroid position c16 (lane bits 1..4).  Each half sorts
+    // its 16 minima over c16 (bitonic, by shuffles); the minimum of each and
+    // the other half's mirrored one is a bitonic sequence of the 16 smallest of
+    // the 32, which a bitonic merge sorts: the r-th smallest is in c16 = r.
+    auto order = [&](uint32_t x, int kk) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < 4; u++) s_x[half][qt][lane][u] = mn[u];
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 4; u++) mn[u] = min(mn[u], s_x[half ^ 1][qt][lane][u]);
-    __syncthreads();
-    uint32_t tau[4];
+        for (int j = kk >> 1; j > 0; j >>= 1) {
+            const uint32_t y = st::xor_lane(x, 2 * j, lane);
+            const bool take_min = ((c16 & j) == 0) == ((c16 & kk) == 0);
+            x = take_min ? min(x, y) : max(x, y);
+        }
+        return x;
+    };
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-        uint32_t x = mn[u];
+        mn[u] = order(order(order(order(mn[u], 2), 4), 8), 16);
+        s_x[half][qt][lane][u] = mn[u];
+    }
+    __syncthreads();
+    uint32_t tau[4];
+    const int mirror = lane ^ 30;  // the same group's lane of 15 - c16
 #pragma unroll
-        for (int kk = 2; kk <= 16; kk <<= 1) {
-#pragma unroll
-            for (int j = kk >> 1; j > 0; j >>= 1) {
-                const uint32_t y = st::xor_lane(x, 2 * j, lane);
-                const bool take_min = ((c16 & j) == 0) == ((c16 & kk) == 0);
-                x = take_min ? min(x, y) : max(x, y);
-            }
-        }
+    for (int u = 0; u < 4; u++) {
+        const uint32_t x = order(min(mn[u], s_x[half ^ 1][qt][mirror][u]), 16);
         // Lane 32 h + 2 (nprobe - 1) + odd's x: four uniform reads, one picked per lane.
         const int b = 2 * (nprobe - 1);
         const uint32_t t0 = st::lane_value(x, b), t1 = st::lane_value(x, b + 1), t2 = st::lane_value(x, b + 32),
                        t3 = st::lane_value(x, b + 33);
         tau[u] = h ? (odd ? t3 : t2) : (odd ? t1 : t0);
     }
+    __syncthreads();
 
     // Candidates: the keys at or below their query's threshold, written at the
     // count of the group's earlier candidates (a prefix sum over c16), from the
@@ -505,114 +515,94 @@ __device__ __forceinline__ int slot_entry(int32_t c, int e) {
 
 __device__ __forceinline__ int slot_size(int32_t c) { return (c & 0xffff) + ((c >> 16) & 0xffff); }
 
-// Candidates per lane held in registers by the merge: the first and last 16
-// entries of its slot.  With 12 + 12, one query in ~30 of the benchmark's
-// batch had a slot end past it and took the general path (twice as long, and
-// the whole launch waited for it); 16 + 16 keeps the arrays in registers (at
-// 20 + 20 the compiler moves them to scratch memory).
-constexpr int MREG = 32;
-
-// One wave per query (a workgroup of one wave, so the queries spread over
-// every CU): probes[q][0, nprobe) by (key, id)
-// ascending over the candidates of its S slots (lane l takes slots l, l + 64,
-// ..).  A threshold on the high 32 bits of the keys is the nprobe-th smallest
-// of the 64 lanes' minima, so at least nprobe candidates lie at or below it
-// and every member of the top nprobe does; those (about nprobe) are gathered
-// in LDS and sorted by the wave.  More than 64 of them (equal or near-equal
-// distances) switch to nprobe successive minimum searches over all the
-// candidates, which is exact for any input.
-__global__ __launch_bounds__(256) void k_probe_merge(const uint64_t *__restrict__ ck, const int32_t *__restrict__ ci,
-                                                     const int32_t *__restrict__ pcnt, int32_t nqc, int32_t S,
-                                                     int32_t nprobe, int32_t *__restrict__ probes) {
-    __shared__ uint64_t s_k[4][64];
-    __shared__ int32_t s_i[4][64];
+// grid: one workgroup of MERGE_W waves per query: probes[q][0, nprobe) by
+// (key, id) ascending over the candidates of its S slots.  With S <= 64 the
+// workgroup holds whole slots in registers: thread t takes slot t % P (P the
+// power of two from S on, at least 4) and P / 4 of its entries, outermost ones
+// first, so the entries of a few slots spread over every lane.  Wave 0 loads
+// its entries with the counts, the others only if some slot of theirs has as
+// many (one more round trip, for large nprobe or crowded slices).  The
+// nprobe-th smallest of a wave's 64 lane minima (high 32 bits) has at least
+// nprobe candidates at or below it; those up to the smallest of the waves'
+// such bounds (about nprobe) are gathered in LDS and sorted by wave 0.  More
+// than 64 of them (equal or near-equal distances), or more slots, take a
+// general path: one wave, the slots re-read, which is exact for any input.
+// (One wave per query with a lane per slot took the general path for
+// nearly every query at nprobe = 16, and whenever there were fewer slots than
+// probes: 4 queries x 16 probes over 4,096 cells took 64 us for both launches,
+// 15 now; 4,096 queries over 12,288 cells 873, 328 now.)
+constexpr int MERGE_W = 4;
+constexpr int ME_MAX = CAPQ / MERGE_W;  // entries per thread, at most
+__global__ __launch_bounds__(64 * MERGE_W) void k_probe_merge(const uint64_t *__restrict__ ck,
+                                                              const int32_t *__restrict__ ci,
+                                                              const int32_t *__restrict__ pcnt, int32_t S,
+                                                              int32_t nprobe, int32_t *__restrict__ probes) {
+    __shared__ uint64_t wk[64];
+    __shared__ int32_t wi[64];
+    __shared__ uint32_t s_tau[MERGE_W];
+    __shared__ int32_t s_count;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t q = (int64_t)blockIdx.x * (blockDim.x >> 6) + w;
-    if (q >= nqc) return;
+    const int64_t q = blockIdx.x;
     const uint64_t *qk = ck + q * S * CAPQ;
     const int32_t *qi = ci + q * S * CAPQ;
     const int32_t *qc = pcnt + q * S;
-    uint64_t *wk = s_k[w];
-    int32_t *wi = s_i[w];
 
-    // Gathers the candidates at or below tau (there are `total`, at most 64)
-    // into the wave's LDS rows, lane `pos` onwards, then sorts them.
-    auto finish = [&](uint64_t k, int32_t id, int total) {
-        __builtin_amdgcn_s_waitcnt(0xc07f);  // this wave's LDS stores are done
-        __builtin_amdgcn_wave_barrier();
-        k = lane < total ? wk[lane] : KNONE;
-        id = lane < total ? wi[lane] : INONE;
+    // Sorts the `total` (at most 64) gathered candidates and writes the probes.
+    auto finish = [&](int total) {
+        uint64_t k = lane < total ? wk[lane] : KNONE;
+        int32_t id = lane < total ? wi[lane] : INONE;
         wave_sort_pair(k, id, lane);
         if (lane < nprobe) probes[q * nprobe + lane] = lane < total ? id : -1;
     };
 
-    // One slot per lane with at most MREG / 2 candidates at either end (the
-    // usual case): the ends' entries are loaded with the count, not after it
-    // (each load one coalesced row of the slots), then selected from registers.
-    const int32_t c0 = lane < S ? qc[lane] : 0;
-    uint64_t kk[MREG];
-    int32_t ii[MREG];
     if (S <= 64) {
+        if (threadIdx.x == 0) s_count = 0;
+        const int lp = S <= 4 ? 2 : 32 - __builtin_clz((unsigned)S - 1), n = 1 << (lp - 2);
+        const int slot = threadIdx.x & ((1 << lp) - 1), o0 = (threadIdx.x >> lp) * n;
+        const bool mine = slot < S;
+        const int32_t c0 = mine ? qc[slot] : 0;
+        const int ca = c0 & 0xffff, cb = (c0 >> 16) & 0xffff;  // entries from the slot's start, from its end
+        // Entry o of the outermost-first order: from the start (o even) or the end.
+        auto at = [&](int e) { return ((o0 + e) & 1) ? CAPQ - 1 - ((o0 + e) >> 1) : (o0 + e) >> 1; };
+        uint64_t kk[ME_MAX];
+        int32_t ii[ME_MAX];
+        const bool any = w == 0 || __ballot(max(ca, cb) > (o0 >> 1)) != 0;
 #pragma unroll
-        for (int e = 0; e < MREG; e++) {
-            const int at = e < MREG / 2 ? e : CAPQ - 1 - (e - MREG / 2);
-            kk[e] = lane < S ? qk[(int64_t)at * S + lane] : KNONE;
-            ii[e] = lane < S ? qi[(int64_t)at * S + lane] : INONE;
-        }
-    }
-    const int ca = c0 & 0xffff, cb = (c0 >> 16) & 0xffff;
-    if (S <= 64 && !__ballot(ca > MREG / 2 || cb > MREG / 2)) {
-#pragma unroll
-        for (int e = 0; e < MREG; e++) {
-            const bool valid = e < MREG / 2 ? e < ca : e - MREG / 2 < cb;
-            if (!valid) {
-                kk[e] = KNONE;
-                ii[e] = INONE;
-            }
+        for (int e = 0; e < ME_MAX; e++) {
+            const bool in = any && mine && e < n;
+            kk[e] = in ? qk[(int64_t)at(e) * S + slot] : KNONE;
+            ii[e] = in ? qi[(int64_t)at(e) * S + slot] : INONE;
         }
         uint32_t m = 0xffffffffu;
 #pragma unroll
-        for (int e = 0; e < MREG; e++) m = min(m, (uint32_t)(kk[e] >> 32));
-        const uint32_t tau = st::lane_value(wave_sort_u32(m, lane), nprobe - 1);
-        uint32_t pm = 0;
+        for (int e = 0; e < ME_MAX; e++) {
+            if (at(e) >= ca && at(e) < CAPQ - cb) kk[e] = KNONE;  // no candidate there
+            m = min(m, (uint32_t)(kk[e] >> 32));
+        }
+        const uint32_t tw = any ? st::lane_value(wave_sort_u32(m, lane), nprobe - 1) : 0xffffffffu;
+        if (lane == 0) s_tau[w] = tw;
+        __syncthreads();
+        uint32_t tau = s_tau[0];
 #pragma unroll
-        for (int e = 0; e < MREG; e++) pm |= (uint32_t)(kk[e] != KNONE && (uint32_t)(kk[e] >> 32) <= tau) << e;
-        const int mine = __popc(pm);
-        const int incl = st::wave_incl_scan(mine);
-        const int total = st::lane_value(incl, 63);
-        if (total <= 64) {
-            int pos = incl - mine;
+        for (int i = 1; i < MERGE_W; i++) tau = min(tau, s_tau[i]);
 #pragma unroll
-            for (int e = 0; e < MREG; e++) {
-                if ((pm >> e) & 1) {
+        for (int e = 0; e < ME_MAX; e++) {
+            if (kk[e] != KNONE && (uint32_t)(kk[e] >> 32) <= tau) {
+                const int pos = atomicAdd(&s_count, 1);
+                if (pos < 64) {
                     wk[pos] = kk[e];
                     wi[pos] = ii[e];
-                    pos++;
                 }
             }
-            finish(0, 0, total);
+        }
+        __syncthreads();
+        const int total = s_count;
+        if (w != 0) return;
+        if (total <= 64) {
+            finish(total);
             return;
         }
-        uint64_t lk = 0;
-        int32_t li = -1;
-        int32_t res = -1;
-        for (int r = 0; r < nprobe; r++) {
-            uint64_t bk = KNONE;
-            int32_t bi = INONE;
-#pragma unroll
-            for (int e = 0; e < MREG; e++) {
-                if (kk[e] != KNONE && lt(lk, li, kk[e], ii[e]) && lt(kk[e], ii[e], bk, bi)) {
-                    bk = kk[e];
-                    bi = ii[e];
-                }
-            }
-            wave_min(bk, bi);
-            if (bk == KNONE && bi == INONE) break;
-            if (lane == r) res = bi;
-            lk = bk;
-            li = bi;
-        }
-        if (lane < nprobe) probes[q * nprobe + lane] = res;
+    } else if (w != 0) {
         return;
     }
 
@@ -645,7 +635,9 @@ __global__ __launch_bounds__(256) void k_probe_merge(const uint64_t *__restrict_
                 }
             }
         }
-        finish(0, 0, total);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        finish(total);
         return;
     }
     uint64_t lk = 0;
@@ -721,8 +713,19 @@ extern "C" st_status st_knn_probe(const int8_t *digits, const int32_t *cexp, con
     if (!st::device_ok()) return ST_ERR_NO_DEVICE;
     const hipStream_t s = st::stream_of(stream);
 
+    // Tiles per slice: the fewest (of 2, 4, 6, 12) that leave at most 64 slices
+    // (k_probe_merge's fast path) and one workgroup per CU.
+    const int64_t ntiles = cdiv(nlist, TILE), groups = cdiv(nq, QG);
+    int ht = HT_MAX;
+    for (const int c : {1, 2, 3}) {
+        const int64_t sl = cdiv(ntiles, 2 * c);
+        if (sl <= 64 && sl * groups <= 256) {
+            ht = c;
+            break;
+        }
+    }
     // Queries in chunks (multiples of 64) whose candidate slots fit CAND_BUDGET.
-    const int64_t ntiles = cdiv(nlist, TILE), S = cdiv(ntiles, TPS);
+    const int64_t S = cdiv(ntiles, 2 * ht);
     const int64_t per_q = S * CAPQ * (int64_t)(sizeof(uint64_t) + sizeof(int32_t)) + S * (int64_t)sizeof(int32_t);
     int64_t chunk = CAND_BUDGET / per_q;
     chunk = chunk < QG ? QG : chunk / QG * QG;
@@ -735,14 +738,15 @@ extern "C" st_status st_knn_probe(const int8_t *digits, const int32_t *cexp, con
     int32_t *ci = reinterpret_cast<int32_t *>(ck + chunk * S * CAPQ);
     int32_t *pcnt = ci + chunk * S * CAPQ;
 
+    auto part = ht == 1 ? k_probe_part<1> : ht == 2 ? k_probe_part<2> : ht == 3 ? k_probe_part<3> : k_probe_part<HT_MAX>;
     for (int64_t q0 = 0; q0 < nq; q0 += chunk) {
         const int64_t nqc = nq - q0 < chunk ? nq - q0 : chunk;
         const int64_t gy = cdiv(nqc, QG);
-        hipLaunchKernelGGL(k_probe_part, dim3((unsigned)(S * gy)), dim3(PART_T), 0, s, queries + q0 * D, (int32_t)nqc, digits,
+        hipLaunchKernelGGL(part, dim3((unsigned)(S * gy)), dim3(PART_T), 0, s, queries + q0 * D, (int32_t)nqc, digits,
                            cexp, cnorm, (int32_t)nlist, (int32_t)S, (int32_t)gy, (int32_t)nprobe, ck, ci, pcnt);
         ST_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_probe_merge, dim3((unsigned)nqc), dim3(64), 0, s, ck, ci, pcnt, (int32_t)nqc,
-                           (int32_t)S, (int32_t)nprobe, probes + q0 * nprobe);
+        hipLaunchKernelGGL(k_probe_merge, dim3((unsigned)nqc), dim3(64 * MERGE_W), 0, s, ck, ci, pcnt, (int32_t)S,
+                           (int32_t)nprobe, probes + q0 * nprobe);
         ST_LAUNCH_CHECK();
     }
     return ST_OK;

@@ -42,6 +42,21 @@ def test_probe_matches_the_oracle(dev, nlist, nq, nprobe):
     np.testing.assert_array_equal(got, oracle.knn_probe(cent, queries, nprobe))
 
 
+# Slices of 2, 4, 6 and 12 tiles of 16 centroids, slot counts around the merge's powers of two (1 to 64, and 65),
+# last slices of one tile, one to many query groups.
+@pytest.mark.parametrize("nlist,nq", [(16, 70), (33, 5), (130, 3), (1000, 65), (1041, 257), (2048, 3), (2049, 130),
+                                      (4090, 40), (4100, 330), (6145, 64), (12480, 64), (12481, 10)])
+def test_probe_slices_and_merge_layouts(dev, nlist, nq):
+    rng = np.random.default_rng(nlist + nq)
+    cent = rng.standard_normal((nlist, D)).astype(np.float32)
+    cent[nlist // 2:nlist // 2 + 12] = cent[0]  # ties within and across slices
+    queries = rng.standard_normal((nq, D)).astype(np.float32)
+    queries[0] = cent[0]
+    for nprobe in (1, 7, 16):
+        _, got = run_probe(dev, cent, queries, nprobe)
+        np.testing.assert_array_equal(got, oracle.knn_probe(cent, queries, nprobe))
+
+
 def test_probe_edge_cases(dev):
     rng = np.random.default_rng(32)
     nlist = 200
