@@ -233,10 +233,11 @@ st_status st_knn_key_norms_2bit(const uint8_t *codes, const float *scales, int64
  * 2^32 keys (cell_start[ncells] < 2^32: key indices are 32-bit inside the
  * top-k keys).  A batch whose nq * nprobe probes reach 2/3 of ncells or
  * more (each cell probed 2/3 of a time or more on average; the reference
- * groups such batches by cell, ivf.rs:491-499) is scanned cell-major: each probed cell is read once
- * for up to four of its queries, with the per-pair lists in the library's
- * kNN scratch arena (nq * nprobe * 1 KiB; serialise such calls per device,
- * and run one before capturing a graph).  Smaller batches use no scratch. */
+ * groups such batches by cell, ivf.rs:491-499) may be scanned cell-major, where
+ * that is estimated to be faster: each probed cell is read once for up to four
+ * of its queries, with the per-pair lists in the library's kNN scratch arena
+ * (nq * nprobe * 1 KiB; serialise such calls per device, and run one before
+ * capturing a graph).  Smaller batches use no scratch. */
 st_status st_knn_search_ivf_2bit(const uint8_t *codes, const float *scales,
                                  const int64_t *cell_start, int64_t ncells, int64_t max_cell,
                                  const float *queries, const int32_t *probes, int64_t nq,

@@ -42,6 +42,7 @@
 // the MALL, bought nothing: on this device a MALL-resident buffer reads no
 // faster than a stream from HBM.)
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 
@@ -1398,6 +1399,28 @@ extern "C" st_status st_knn_synth_keys_f32(uint64_t seed, int64_t row0, int64_t 
     return ST_OK;
 }
 
+// Estimated times (us) of the two scan orders, both on the largest cell.
+// Query-major (k_search) reads each probed cell once per query that probes it,
+// at the device's streaming rate; cell-major (k_group_*, k_search_cells,
+// k_merge_parts) has about 100 us of grouping, first units and merges, then
+// rounds of 1,536 workgroups (six per CU), each 38 us of set-up and merges and
+// 15.5 ns per key.  Fitted to both orders at 4 to 8,192 queries x 2, 8 and 16
+// probes over 64 to 12,288 cells of 300 to 10,172 keys: of 147 such batches the
+// estimate takes the slower order at 4, by at most 1.4x.  (Cell-major from 2/3
+// of a probe per cell on, whatever the sizes, was right for the 125M-key index
+// and took 67 us instead of 37 for 256 x 2 probes of 64 cells of 300 keys, 159
+// instead of 68 for 256 x 16 of 400 x 1,000.)  Below that share the batch stays
+// query-major, which needs no scratch.
+static double query_major_us(int64_t nq, int64_t nprobe, int64_t max_cell) {
+    return 25.0 + 0.04 * (double)nq + (double)(nq * nprobe) * (double)max_cell * 68.0 / 7e6;
+}
+
+static double cell_major_us(int64_t nq, int64_t nprobe, int64_t ncells, int64_t max_cell) {
+    const double pairs = (double)(nq * nprobe), probed = (double)ncells * -std::expm1(-pairs / (double)ncells);
+    const double units = std::max(probed, pairs / QG + 0.375 * probed);  // ceil(probes / QG) over the probed cells
+    return 100.0 + std::max(1.0, units / 1536.0) * (38.0 + 0.0155 * (double)max_cell);
+}
+
 // Workgroups per query of a query-major scan of nq queries that has memory for
 // their lists: one per CU in all.  20 queries' worth of runs of 40 chunks each
 // take 36 us, merge included, where one workgroup per query takes 118 to 200;
@@ -1466,13 +1489,10 @@ extern "C" st_status st_knn_search_ivf_2bit_split(const uint8_t *codes, const fl
     if (nq > INT32_MAX / PROBE_MAX) return st::fail(ST_ERR_INVALID, "search_ivf: too many queries for one call");
     if (!st::device_ok()) return ST_ERR_NO_DEVICE;
     const hipStream_t s = st::stream_of(stream);
-    // Query-major (a workgroup per query, each probed cell read once per
-    // query that probes it) unless the batch probes the cells 2/3 of a time
-    // or more on average: then cell-major, each probed cell read once for up
-    // to QG queries (12,288 cells x 8 probes: 0.42 against 0.48 ms at 512
-    // queries, 0.82 against 0.78 ms at 1,024).
     const int64_t npairs = nq * nprobe;
-    const bool cells = g_scan_order == 2 || (g_scan_order == 0 && 3 * npairs >= 2 * ncells);
+    const bool cells =
+        g_scan_order == 2 || (g_scan_order == 0 && 3 * npairs >= 2 * ncells &&
+                              cell_major_us(nq, nprobe, ncells, max_cell) < query_major_us(nq, nprobe, max_cell));
     if (!cells) {
         // Cells too small for that many runs (max_cell bounds them) give fewer.
         SplitWork w = split_work(work, work_bytes, nq);
