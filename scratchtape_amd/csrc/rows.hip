@@ -21,13 +21,15 @@
 //    chunks (4 row lanes per column, combined in a fixed order) and
 //    k_ln_bwd_sum adds the chunks in ascending order;
 //  - vector path (d % 4 == 0 up to 1024, 16-byte aligned rows and parameter
-//    sets): k_ln_bwd4 sums 16-row chunks (each of 4 waves adds its rows in
-//    row order; the 4 waves' sums are added in wave order) and
+//    sets): k_ln_bwd4 sums chunks of 16 rows or more (each of 4 waves adds its
+//    rows in row order; the 4 waves' sums are added in wave order) and
 //    k_ln_bwd_sum4 adds a column's chunks as 16 slices, each slice's chunks
 //    in ascending order, the 16 slice sums in a fixed tree order.
 // The two paths add in different orders, so their last bits can differ;
 // each is deterministic.  Contraction is off so that scale*x - m rounds the
 // product first, as the reference's CPU tape does.
+#include <algorithm>
+
 #include "common.h"
 #include "lanes.h"
 
@@ -237,7 +239,8 @@ __global__ __launch_bounds__(256) void k_ln_bwd_sum(const float *__restrict__ pa
 // ---- Vector forms for rows of d % 4 == 0 up to 1024 wide, 16-byte aligned:
 // lane l of a row's wave owns the float4 columns 4 l + 256 i, i < NV.
 
-constexpr int LNV_ROWS = 16;  // rows per backward workgroup (4 per wave)
+constexpr int LNV_ROWS = 16;       // rows a backward workgroup takes at a time (4 per wave)
+constexpr int LNV_CHUNKS = 1024;  // chunks (workgroups) per model, at most, once rows allow it
 
 __device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
 // Output rows (y, dx) through nontemporal stores: they stream out as the
@@ -301,9 +304,10 @@ __global__ __launch_bounds__(256) void k_ln_fwd4(const float *__restrict__ x, in
     }
 }
 
-// The backward's row pass.  grid (chunks of LNV_ROWS rows per model, models);
-// wave w takes rows w, w + 4, .. of its chunk: dx as k_ln_bwd_dx, and each
-// lane adds dy xhat and dy of its columns over the wave's rows (in row order).
+// The backward's row pass.  grid (chunks of `rows_pc` rows per model, models),
+// rows_pc a multiple of LNV_ROWS; wave w takes rows w, w + 4, .. of its chunk:
+// dx as k_ln_bwd_dx, and each lane adds dy xhat and dy of its columns over the
+// wave's rows (in row order).
 // The four waves' sums are added in a fixed order into the chunk's partial,
 // part[(m nch + c) 2d + j], which k_ln_bwd_sum4 adds up.  dy and x are read
 // once for both gradients.
@@ -312,12 +316,12 @@ __global__ __launch_bounds__(256) void k_ln_bwd4(const float *__restrict__ dy, c
                                                  const float *__restrict__ mean, const float *__restrict__ rstd,
                                                  int64_t d, int64_t rows_pm, const float *__restrict__ params,
                                                  int64_t off, int64_t stride, float *__restrict__ dx, int32_t accumulate,
-                                                 float *__restrict__ part, int32_t nch) {
+                                                 float *__restrict__ part, int32_t nch, int32_t rows_pc) {
     __shared__ float4 sp[4][2][NV * 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int32_t c = blockIdx.x, m = blockIdx.y;
-    const int64_t rbeg = (int64_t)m * rows_pm + (int64_t)c * LNV_ROWS;
-    const int64_t rend = min((int64_t)m * rows_pm + rows_pm, rbeg + LNV_ROWS);
+    const int64_t rbeg = (int64_t)m * rows_pm + (int64_t)c * rows_pc;
+    const int64_t rend = min((int64_t)m * rows_pm + rows_pm, rbeg + rows_pc);
     const float *gm = params + off + (int64_t)m * stride;
     const float inv_d = 1.0f / (float)d;
     float4 gmv[NV], pg[NV], pb[NV];
@@ -331,8 +335,8 @@ __global__ __launch_bounds__(256) void k_ln_bwd4(const float *__restrict__ dy, c
     // RB rows' loads in flight together; a row past the chunk's end loads the
     // chunk's last row (always in bounds) and contributes nothing.
     constexpr int RB = NV >= 4 ? 2 : 4;
-#pragma unroll
-    for (int t0 = 0; t0 < LNV_ROWS / 4; t0 += RB) {
+    const int trips = (int)(rend - rbeg + 4 * RB - 1) / (4 * RB);
+    for (int t0 = 0; t0 < trips * RB; t0 += RB) {
         float4 dyv[RB][NV], xv[RB][NV];
         float mu[RB], rs[RB];
         bool live[RB];
@@ -484,7 +488,7 @@ extern "C" st_status st_layer_norm(const float *x, int64_t rows, int64_t d, cons
     const int64_t rows_pm = rows / models;
     if (ln_vec_ok(d, off, model_stride, {x, params, y})) {
         const int nv = (int)((d + 255) / 256);
-        auto k = nv == 1 ? k_ln_fwd4<1> : nv == 2 ? k_ln_fwd4<2> : k_ln_fwd4<4>;
+        auto k = nv == 1 ? k_ln_fwd4<1> : nv == 2 ? k_ln_fwd4<2> : nv == 3 ? k_ln_fwd4<3> : k_ln_fwd4<4>;
         hipLaunchKernelGGL(k, grid, dim3(256), 0, s, x, rows, d, params, off, eps, rows_pm, model_stride, y, mean,
                            rstd);
     } else {
@@ -507,15 +511,21 @@ extern "C" st_status st_layer_norm_backward(const float *dy, const float *x, con
     if (!st::device_ok()) return ST_ERR_NO_DEVICE;
     const hipStream_t s = st::stream_of(stream);
     const int64_t rows_pm = rows / models;
-    const int64_t vch = (rows_pm + LNV_ROWS - 1) / LNV_ROWS;
+    // Rows per chunk: 16, or as many more as leave LNV_CHUNKS chunks, so that the
+    // partials (2 d floats each) stay small beside the rows: at 65,536 x 768
+    // k_ln_bwd_sum4 took 22.7 us over 4,096 chunks of 16 and takes 6.6 over 1,024
+    // of 64 (forward and backward together 199 -> 187 us).
+    const int64_t rows_pc =
+        LNV_ROWS * std::max<int64_t>(1, (rows_pm + LNV_ROWS * LNV_CHUNKS - 1) / (LNV_ROWS * LNV_CHUNKS));
+    const int64_t vch = (rows_pm + rows_pc - 1) / rows_pc;
     if (ln_vec_ok(d, off, model_stride, {dy, x, params, dx}) && vch <= INT32_MAX && models <= 65535) {
         float *part = static_cast<float *>(
             st::scratch(st::SCRATCH_ROWS, (size_t)(models * vch * 2 * d) * sizeof(float), s));
         if (!part) return st::scratch_status();
         const int nv = (int)((d + 255) / 256);
-        auto k = nv == 1 ? k_ln_bwd4<1> : nv == 2 ? k_ln_bwd4<2> : k_ln_bwd4<4>;
+        auto k = nv == 1 ? k_ln_bwd4<1> : nv == 2 ? k_ln_bwd4<2> : nv == 3 ? k_ln_bwd4<3> : k_ln_bwd4<4>;
         hipLaunchKernelGGL(k, dim3((unsigned)vch, (unsigned)models), dim3(256), 0, s, dy, x, mean, rstd, d, rows_pm,
-                           params, off, model_stride, dx, accumulate, part, (int32_t)vch);
+                           params, off, model_stride, dx, accumulate, part, (int32_t)vch, (int32_t)rows_pc);
         ST_LAUNCH_CHECK();
         hipLaunchKernelGGL(k_ln_bwd_sum4, dim3((unsigned)((2 * d + 15) / 16), (unsigned)models), dim3(256), 0, s, part,
                            d, (int32_t)vch, grads, off, model_stride);

@@ -80,6 +80,13 @@ def test_layer_norm_vector_forms(dev, nrows, d, off):
     run_case(dev, nrows, d, off, seed=nrows + d)
 
 
+# Above 16 x 1,024 rows per model a chunk takes 32 rows or more: the first such size, a last chunk of one row, three
+# register columns per lane, and two models of which each does.
+@pytest.mark.parametrize("nrows,d,models", [(16385, 8, 1), (33 * 1024 + 1, 36, 1), (17000, 516, 1), (2 * 16400, 12, 2)])
+def test_layer_norm_vector_forms_with_longer_chunks(dev, nrows, d, models):
+    run_case(dev, nrows, d, 4, models, seed=nrows)
+
+
 def test_layer_norm_vector_forms_three_models(dev):
     # 272 rows per model: 17 chunks per model, over sixteen slices of two chunks (the last slice empty).
     run_case(dev, 3 * 272, 64, 8, models=3, stride=2 * 64 + 12, seed=17)
