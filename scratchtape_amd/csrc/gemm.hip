@@ -634,6 +634,7 @@ size_t gemm_impl_scratch(const st_matref *a, const st_matref *b, const st_matref
         return 0;
     const bool f16 = f16_route(use_f16, epi, b, m, k, n);
     const st::DmaGemm d = make_dma(a, b, out, batch, m, k, n, epi, f16);
+    if (st::group_of_one(d)) return st::gemm_group_scratch(&d, 1, f16, true);
     size_t dma = 0;
     if ((dma = st::gemm_dma_scratch(d)) || st::gemm_dma_takes(d)) return dma;
     const int64_t splits = plan_tiles(f16, a->trans, b->trans, epi, out, batch, m, k, n).splits;
@@ -659,10 +660,13 @@ st_status gemm_impl(const st_matref *a, const st_matref *b, const st_matref *out
     const int64_t ldb = b->ld ? b->ld : (b->trans ? k : n);
     const int64_t ldo = out->ld ? out->ld : n;
 
-    // Tile-divisible, 16-byte aligned problems run on the LDS-DMA kernel.
+    // Tile-divisible, 16-byte aligned problems run on the LDS-DMA kernel, the
+    // larger ones on the grouped kernel.
     {
+        const st::DmaGemm d = make_dma(a, b, out, batch, m, k, n, epi, f16);
+        if (st::group_of_one(d)) return st::gemm_group(&d, 1, f16, true, stream);
         st_status ds = ST_OK;
-        if (st::gemm_dma(make_dma(a, b, out, batch, m, k, n, epi, f16), stream, &ds)) return ds;
+        if (st::gemm_dma(d, stream, &ds)) return ds;
     }
 
     const TileCfg tc = plan_tiles(f16, a->trans, b->trans, epi, out, batch, m, k, n);

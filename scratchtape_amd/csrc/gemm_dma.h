@@ -50,6 +50,10 @@ bool group_tall(const DmaGemm &g);
 st_status gemm_group(const DmaGemm *items, int count, bool f16, bool tall, hipStream_t stream);
 // Bytes of split-k scratch gemm_group requests for the same arguments.
 size_t gemm_group_scratch(const DmaGemm *items, int count, bool f16, bool tall);
+// Whether a single call is better a grouped launch of one (256-row tiles, see
+// the rule at its definition) than gemm_dma.  Never true where that would use
+// scratch memory and gemm_dma would not.
+bool group_of_one(const DmaGemm &d);
 // Reads and clears the current device's count of grouped-kernel slot waits
 // that gave up; ST_ERR_HIP with a message if there were any.  The caller has
 // synchronised the work it wants covered.

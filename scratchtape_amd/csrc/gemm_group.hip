@@ -1321,7 +1321,8 @@ st_status launch_group(const st::DmaGemm *items, int count, void (*kern)(GroupAr
         }
     }
     const int64_t wgs = std::min<int64_t>(cus / XCDS * XCDS, cdiv(units, XCDS) * XCDS);
-    schedule(ga, (int)std::max<int64_t>(1, wgs / XCDS));
+    // The units of one GEMM are alike: round robin (and the kept schedule stays the last group's).
+    if (count > 1) schedule(ga, (int)std::max<int64_t>(1, wgs / XCDS));
     hipLaunchKernelGGL(kern, dim3((unsigned)std::max<int64_t>(XCDS, wgs)), dim3(C::THREADS), 0, stream, ga);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && sa.count) {
@@ -1372,6 +1373,23 @@ size_t gemm_group_scratch(const DmaGemm *items, int count, bool f16, bool tall) 
     std::vector<int64_t> splits, slice_k;
     group_splits(items, count, TM, NS, fair_part, group_cus(), splits, slice_k);
     return sizeof(float) * group_part_floats(items, count, splits);
+}
+
+// The grouped kernels' 256 x 128 tiles read the operands 1.5 times less than
+// gemm_dma's 128 x 128 and (f16) round each element once, but a CU gets few
+// units.  As single calls, gemm_dma against a group of one, us: f16 with 128
+// tiles 4096 x 256 x 1024 16.6 / 13.8, 16384 x 256 x 256 16.2 / 12.8; 512 tiles
+// 8192 x 512 x 2048 73.7 / 43.0; 2,048 tiles 16384 x 1024 x 4096 486 / 246; 64
+// tiles 4096 x 2048 x 512 33.8 / 43.2; 32 tiles 4096 x 256 x 256 8.5 / 12.7.  f32
+// with 256 tiles 8192 x 256 x 1024 53.0 / 44.7; 128 tiles 30.5 / 31.4.  Split
+// products by tiles x k-stages: 8 x 128 19.4 / 22.0 (f16) and 31.9 / 35.8 (f32),
+// 8 x 256 29.8 / 23.5 and 52.3 / 49.0, 128 x 512 710 / 330.
+bool group_of_one(const DmaGemm &d) {
+    if (!group_eligible(d) || !group_tall(d)) return false;
+    const int64_t tiles = d.batch * (d.m / Tall::TM) * (d.n / TN);
+    const bool split = can_split(d) && tiles * (d.k / BK) >= 2048;
+    if (tiles < (d.f16 ? 128 : 256) && !split) return false;
+    return gemm_group_scratch(&d, 1, d.f16 != 0, true) == 0 || gemm_dma_scratch(d) != 0;
 }
 
 st_status gemm_group(const DmaGemm *items, int count, bool f16, bool tall, hipStream_t stream) {

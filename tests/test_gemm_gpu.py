@@ -427,6 +427,21 @@ def test_grouped_random_groups_match_oracle(dev):
             check_case(p)
 
 
+# Single calls large enough for the grouped kernel's 256 x 128 tiles: 128 (f16) or 256 (f32) tiles with every
+# epilogue term, one fewer row of tiles (which are not), batches, and a product split over k with column sums.
+@pytest.mark.parametrize("case,use_f16", [
+    ((1, 2048, 128, 2048, False, False, True, True, True, True, True), True),
+    ((1, 1792, 128, 2048, False, True, True, False, False, False, False), True),
+    ((2, 1024, 160, 2048, True, True, False, False, False, True, False), True),
+    ((1, 4096, 128, 2048, False, True, True, True, True, True, True), False),
+    ((1, 3840, 128, 2048, True, False, False, False, False, False, True), False),
+    ((1, 512, 8192, 512, True, False, False, False, False, False, True), True),
+    ((1, 512, 8192, 512, True, False, False, False, False, False, True), False)])
+def test_single_calls_on_the_grouped_kernel(dev, case, use_f16):
+    with oracle.threads(8):
+        run_case(dev, 900, case, use_f16, aligned16=True, packed=True)
+
+
 @pytest.mark.parametrize("use_f16", [False, True])
 def test_grouped_step_set_matches_the_oracle(dev, use_f16):
     """The 15 GEMMs of a d_model-256 step (T = 4096) as one group -- the call the benchmark times -- against the
