@@ -113,6 +113,21 @@ def lib():
     return _lib
 
 
+_packed = {}
+
+
+def packed(name: str):
+    """Entry point `name` taking its struct arguments as bytes in the C layout (packing them is cheaper than building
+    ctypes structures)."""
+    fn = _packed.get(name)
+    if fn is None:
+        fn = lib()[name]  # a function object of its own
+        fn.argtypes = [a if a in (_i32, _i64, _f32, _u64) else _vp for a in SIGNATURES[name]]
+        fn.restype = _i32
+        _packed[name] = fn
+    return fn
+
+
 def check(status: int) -> None:
     if status != ST_OK:
         msg = lib().st_last_error().decode(errors="replace")

@@ -7,8 +7,8 @@ ScratchtapeError with the message the reference would panic with.
 """
 from __future__ import annotations
 
-import ctypes
-from dataclasses import dataclass, field, replace
+import struct
+from dataclasses import dataclass
 from typing import Optional, Tuple
 
 import torch
@@ -26,8 +26,20 @@ def _ptr(t: torch.Tensor) -> int:
     return t.data_ptr()
 
 
+# The handle of a device's current stream without a Stream object around it (a third of the call's host time).
+_current_raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+# st_matref, st_epilogue and st_gemm (scratchtape_hip.h) as the C compiler lays them out.
+_REF = struct.Struct("=Qqqiiqqq")
+_EPI = struct.Struct("=QqqQqQqiiiiqq")
+_GEMM = struct.Struct("=" + 3 * "Qqqiiqqq" + "QqqQqQqiiiiqq" + "qqqqii")
+_NO_EPI = 13 * (0,)
+
+
 def _stream(stream) -> int:
     if stream is None:
+        if _current_raw is not None:
+            return _current_raw(torch.cuda.current_device())
         return torch.cuda.current_stream().cuda_stream
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
@@ -59,11 +71,20 @@ class MatRef:
         return MatRef(h, off=col0, stride=t * cols, ld=cols, group=heads, inner=width)
 
     def with_(self, **kw) -> "MatRef":
-        return replace(self, **kw)
+        for name in kw:
+            if name not in _MATREF_FIELDS:
+                raise TypeError(f"MatRef has no field {name!r}")
+        new = object.__new__(type(self))  # dataclasses.replace, without its walk over the fields
+        new.__dict__.update(self.__dict__)
+        new.__dict__.update(kw)
+        return new
 
-    def _c(self) -> _lib.StMatRef:
-        return _lib.StMatRef(_ptr(self.h), self.off, self.stride, int(bool(self.trans)), 0, self.ld, self.group,
-                             self.inner)
+    def _fields(self) -> tuple:
+        """st_matref's fields in order."""
+        return (_ptr(self.h), self.off, self.stride, 1 if self.trans else 0, 0, self.ld, self.group, self.inner)
+
+
+_MATREF_FIELDS = frozenset(MatRef.__dataclass_fields__)
 
 
 @dataclass
@@ -78,28 +99,27 @@ class Epilogue:
     accumulate: bool = False
     col_sum: Optional[Tuple[int, int]] = None
 
-    def _c(self) -> _lib.StEpilogue:
-        e = _lib.StEpilogue()
-        if self.bias is not None:
-            e.bias, e.bias_off = _ptr(self.bias[0]), self.bias[1]
-        e.bias_stride = self.bias_stride
-        if self.mask is not None:
-            e.mask, e.mask_off = _ptr(self.mask[0]), self.mask[1]
-        if self.residual is not None:
-            e.residual, e.residual_off = _ptr(self.residual[0]), self.residual[1]
-        e.relu = int(self.relu)
-        e.accumulate = int(self.accumulate)
-        if self.col_sum is not None:
-            e.has_col_sum = 1
-            e.col_sum_off, e.col_sum_stride = self.col_sum
-        return e
+    def _fields(self) -> tuple:
+        """st_epilogue's fields in order."""
+        bias, mask, residual, col_sum = self.bias, self.mask, self.residual, self.col_sum
+        return (_ptr(bias[0]) if bias is not None else 0, bias[1] if bias is not None else 0, self.bias_stride,
+                _ptr(mask[0]) if mask is not None else 0, mask[1] if mask is not None else 0,
+                _ptr(residual[0]) if residual is not None else 0, residual[1] if residual is not None else 0,
+                int(self.relu), int(self.accumulate), 0 if col_sum is None else 1, 0,
+                *(col_sum if col_sum is not None else (0, 0)))
+
+
+def _pack(layout: struct.Struct, *fields) -> bytes:
+    try:
+        return layout.pack(*fields)
+    except struct.error as e:
+        raise TypeError(str(e)) from None
 
 
 def _call(name, a: MatRef, b: MatRef, out: MatRef, batch, m, k, n, epi, *extra, stream=None):
-    epi = epi or Epilogue()
-    ca, cb, co, ce = a._c(), b._c(), out._c(), epi._c()
-    _lib.call(name, ctypes.byref(ca), ctypes.byref(cb), ctypes.byref(co), batch, m, k, n, ctypes.byref(ce), *extra,
-              _stream(stream))
+    _lib.check(_lib.packed(name)(_pack(_REF, *a._fields()), _pack(_REF, *b._fields()), _pack(_REF, *out._fields()),
+                                 batch, m, k, n, _pack(_EPI, *(epi._fields() if epi else _NO_EPI)), *extra,
+                                 _stream(stream)))
 
 
 def matmul(a: MatRef, b: MatRef, out: MatRef, batch: int, m: int, k: int, n: int,
@@ -128,11 +148,11 @@ def matmul_grouped(calls, stream=None, noalloc: bool = False) -> None:
     No call may read or write memory that another one writes.  noalloc: the
     same through st_matmul_grouped_noalloc (split-k partials in the library's
     fixed per-device scratch; no device allocation)."""
-    calls = list(calls)
-    arr = (_lib.StGemm * max(1, len(calls)))()
-    for i, (a, b, out, batch, m, k, n, epi, use_f16) in enumerate(calls):
-        arr[i] = _lib.StGemm(a._c(), b._c(), out._c(), (epi or Epilogue())._c(), batch, m, k, n, int(bool(use_f16)), 0)
-    _lib.call("st_matmul_grouped_noalloc" if noalloc else "st_matmul_grouped", arr, len(calls), _stream(stream))
+    gemms = [_pack(_GEMM, *a._fields(), *b._fields(), *out._fields(), *(epi._fields() if epi else _NO_EPI), batch, m, k,
+                   n, 1 if use_f16 else 0, 0) for a, b, out, batch, m, k, n, epi, use_f16 in calls]
+    # (One empty struct for an empty group: the library takes no NULL array.)
+    _lib.check(_lib.packed("st_matmul_grouped_noalloc" if noalloc else "st_matmul_grouped")(
+        b"".join(gemms) or bytes(_GEMM.size), len(gemms), _stream(stream)))
 
 
 def f16_enabled() -> bool:

@@ -179,3 +179,32 @@ def test_scratch_release_without_arenas_is_a_no_op():
     if L.st_scratch_release() != _lib.ST_OK:
         # No HIP device in this process: the call reports it instead of crashing.
         assert L.st_last_error()
+
+
+def test_packed_arguments_have_the_struct_layout(monkeypatch):
+    """The bytes that matmul.py packs for st_matref, st_epilogue and st_gemm, field by field, and what is refused."""
+    import sys
+    from scratchtape_amd import Epilogue, MatRef
+    mm = sys.modules["scratchtape_amd.matmul"]
+    addr = {"a": 0x7F0000000010, "b": 0x20, "o": 0x30, "bias": 0x40, "mask": 0x50, "res": 0x60}
+    monkeypatch.setattr(mm, "_ptr", lambda t: addr[t])
+    a = MatRef("a", 1, -2, True, 3, 4, 5)
+    b, o = a.with_(h="b", trans=False), MatRef("o")
+    assert (b.off, b.group, a.trans, b.trans) == (1, 4, True, False)
+    epi = Epilogue(bias=("bias", 6), bias_stride=7, relu=True, mask=("mask", 8), residual=("res", 9), accumulate=True,
+                   col_sum=(10, 11))
+    raw = mm._pack(mm._GEMM, *a._fields(), *b._fields(), *o._fields(), *epi._fields(), 12, 13, 14, 15, 1, 0)
+    assert len(raw) == _lib.ctypes.sizeof(_lib.StGemm)
+    g = _lib.StGemm.from_buffer_copy(raw)
+    values = lambda s: [getattr(s, f) for f, _ in s._fields_]
+    assert values(g.a) == [addr["a"], 1, -2, 1, 0, 3, 4, 5] and values(g.b) == [addr["b"], 1, -2, 0, 0, 3, 4, 5]
+    assert values(g.out) == [addr["o"], 0, 0, 0, 0, 0, 1, 0]
+    assert values(g.epi) == [addr["bias"], 6, 7, addr["mask"], 8, addr["res"], 9, 1, 1, 1, 0, 10, 11]
+    assert [g.batch, g.m, g.k, g.n, g.use_f16] == [12, 13, 14, 15, 1]
+    assert mm._pack(mm._REF, *a._fields()) == raw[:56] and mm._pack(mm._EPI, *epi._fields()) == raw[168:256]
+    assert mm._pack(mm._EPI, *mm._NO_EPI) == bytes(_lib.ctypes.sizeof(_lib.StEpilogue))
+    assert mm._pack(mm._EPI, *Epilogue()._fields()) == bytes(_lib.ctypes.sizeof(_lib.StEpilogue))
+    with pytest.raises(TypeError):
+        mm._pack(mm._REF, *a.with_(off=1.5)._fields())
+    with pytest.raises(TypeError):
+        a.with_(offset=1)
