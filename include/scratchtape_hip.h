@@ -205,6 +205,22 @@ st_status st_attention_fused_bwd(const float *qkv, const float *ctx, const float
                                  const float *lse, float *dqkv, int64_t b, int64_t h, int64_t t,
                                  int64_t hd, float scale, st_stream stream);
 
+/* The f32 attention of the device tape with its scores and probabilities
+ * written out (gpu_step/tape.rs:196-212, 349-372, 475-491: the products
+ * always f32, matmul.rs:90-95): what the batched st_matmul_f32 calls and
+ * st_softmax / st_softmax_backward over the same buffers write, in one launch
+ * forward and two backward.  s, p, dp, ds [b h_count t, t]; ctx, dctx [b t, D];
+ * qkv, dqkv [b t, 3 D]; all 4-byte aligned, none of them overlapping.
+ * forward: s = Q K^T, p = softmax(scale s, causal), ctx = p V; backward: dp =
+ * dctx V^T, ds = scale p (dp - rowsum(dp p)), and dQ, dK, dV into dqkv (every
+ * element).  st_attention_fits: whether t (1..=512) and hd (1..=128) are taken. */
+int32_t st_attention_fits(int64_t t, int64_t hd);
+st_status st_attention_fwd(const float *qkv, float *s, float *p, float *ctx, int64_t b, int64_t h,
+                           int64_t t, int64_t hd, float scale, st_stream stream);
+st_status st_attention_bwd(const float *qkv, const float *dctx, const float *p, float *dp, float *ds,
+                           float *dqkv, int64_t b, int64_t h, int64_t t, int64_t hd, float scale,
+                           st_stream stream);
+
 /* ---- 2-bit kNN memory ---------------------------------------------------- */
 
 /* gpu_step/knn.rs:190-225 `tile_of` (bits = 2) on the device: keys [n, d]

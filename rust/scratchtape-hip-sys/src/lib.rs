@@ -238,6 +238,35 @@ extern "C" {
         scale: f32,
         stream: st_stream,
     ) -> st_status;
+    /// The f32 attention of the device tape (`src/gpu_step/tape.rs:196-212, 349-372`) with its
+    /// scores and probabilities written out.
+    pub fn st_attention_fits(t: i64, hd: i64) -> i32;
+    pub fn st_attention_fwd(
+        qkv: *const f32,
+        s: *mut f32,
+        p: *mut f32,
+        ctx: *mut f32,
+        b: i64,
+        h: i64,
+        t: i64,
+        hd: i64,
+        scale: f32,
+        stream: st_stream,
+    ) -> st_status;
+    pub fn st_attention_bwd(
+        qkv: *const f32,
+        dctx: *const f32,
+        p: *const f32,
+        dp: *mut f32,
+        ds: *mut f32,
+        dqkv: *mut f32,
+        b: i64,
+        h: i64,
+        t: i64,
+        hd: i64,
+        scale: f32,
+        stream: st_stream,
+    ) -> st_status;
     pub fn st_knn_quantize_2bit(
         keys: *const f32,
         n: i64,

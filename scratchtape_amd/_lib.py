@@ -67,6 +67,9 @@ SIGNATURES = {
     "st_layer_norm_backward": [_vp, _vp, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _vp, _i32, _i64, _i64, _vp],
     "st_attention_fused_fwd": [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _f32, _i32, _vp],
     "st_attention_fused_bwd": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _f32, _vp],
+    "st_attention_fits": [_i64, _i64],
+    "st_attention_fwd": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _f32, _vp],
+    "st_attention_bwd": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _f32, _vp],
     "st_knn_quantize_2bit": [_vp, _i64, _i64, _vp, _vp, _vp],
     "st_knn_search_ivf_2bit": [_vp, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp],
     "st_knn_split_bytes": [_i64],

@@ -22,7 +22,7 @@ from typing import Optional
 import torch
 
 from . import _lib, rows
-from .matmul import Epilogue, MatRef, _stream, matmul_with
+from .matmul import MatRef, _ptr, _stream, f16_route, matmul_with
 
 
 @dataclass
@@ -42,10 +42,25 @@ class AttnBuffers:
                            z(b * t * 3 * d))
 
 
+def _f32_step(qkv, dctx, buf: AttnBuffers, b: int, h: int, t: int, hd: int, use_f16: bool) -> bool:
+    """Whether st_attention_fwd / _bwd take the step: its products all run in f32 (the six have one f16 rule: t % 64 ==
+    0 and hd % 32 == 0), the sizes fit, and the buffers hold the whole problems."""
+    if (use_f16 and f16_route(t, hd, t)) or b < 1 or h < 1 or not _lib.lib().st_attention_fits(t, hd):
+        return False
+    n, tokens = b * h * t * t, b * t * h * hd
+    sizes = [(qkv, 3 * tokens), (buf.s, n), (buf.p, n), (buf.ctx, tokens)] if dctx is None else \
+        [(qkv, 3 * tokens), (dctx, tokens), (buf.p, n), (buf.dp, n), (buf.ds, n), (buf.dqkv, 3 * tokens)]
+    return all(x.numel() >= least for x, least in sizes)
+
+
 def forward(qkv: torch.Tensor, buf: AttnBuffers, b: int, h: int, t: int, hd: int, use_f16: bool,
             stream=None) -> None:
     d = h * hd
     batch, scale = b * h, hd ** -0.5
+    if _f32_step(qkv, None, buf, b, h, t, hd, use_f16):
+        _lib.call("st_attention_fwd", _ptr(qkv), _ptr(buf.s), _ptr(buf.p), _ptr(buf.ctx), b, h, t, hd, scale,
+                  _stream(stream))
+        return
     stacked = MatRef(buf.s, stride=t * t)
     matmul_with(MatRef.heads(qkv, 0, 3 * d, t, h, hd), MatRef.heads(qkv, d, 3 * d, t, h, hd).with_(trans=True),
                 stacked, batch, t, hd, t, None, use_f16, stream=stream)
@@ -59,6 +74,10 @@ def backward(qkv: torch.Tensor, dctx: torch.Tensor, buf: AttnBuffers, b: int, h:
     """dV = Pᵀ dO, dP = dO Vᵀ, dS = softmax backward, dQ = dS K, dK = dSᵀ Q, written into buf.dqkv."""
     d = h * hd
     batch, scale = b * h, hd ** -0.5
+    if _f32_step(qkv, dctx, buf, b, h, t, hd, use_f16):
+        _lib.call("st_attention_bwd", _ptr(qkv), _ptr(dctx), _ptr(buf.p), _ptr(buf.dp), _ptr(buf.ds), _ptr(buf.dqkv), b,
+                  h, t, hd, scale, _stream(stream))
+        return
     p = MatRef(buf.p, stride=t * t)
     do = MatRef.heads(dctx, 0, d, t, h, hd)
     v = MatRef.heads(qkv, 2 * d, 3 * d, t, h, hd)

@@ -147,3 +147,64 @@ def test_fused_attention_random_shapes(dev):
     rnd = random.Random(23)
     for i, t in enumerate(rnd.sample(range(32, 257, 32), 8)):
         fused_case(dev, rnd.randint(1, 3), rnd.randint(1, 4), t, rnd.random() < 0.5, 300 + i)
+
+
+# ---- st_attention_fwd / _bwd: the f32 step in three launches
+
+
+def f32_step(dev, b, h, t, hd, qkv, dctx, separate, monkeypatch):
+    """attention.step on the f32 route, fused or (separate) as its six products and two softmax passes."""
+    buf = attention.AttnBuffers.empty(b, h, t, hd, dev)
+    for x in (buf.s, buf.p, buf.ctx, buf.dp, buf.ds, buf.dqkv):
+        x.fill_(7.0)
+    with monkeypatch.context() as m:
+        if separate:
+            m.setattr(attention, "_f32_step", lambda *a: False)
+        attention.step(qkv, dctx, buf, b, h, t, hd, False)
+    return [x.cpu().double().numpy() for x in (buf.s, buf.p, buf.ctx, buf.dp, buf.ds, buf.dqkv)]
+
+
+# Sequence lengths around the 16-, 32- and 64-row blocks and tiles up to the longest, head widths of each compiled class
+# and off 4, one problem to many.
+@pytest.mark.parametrize("b,h,t,hd", [(1, 1, 1, 1), (2, 1, 3, 5), (1, 3, 16, 16), (2, 2, 17, 20), (1, 2, 31, 32),
+                                      (3, 1, 33, 33), (1, 4, 63, 64), (2, 3, 64, 80), (1, 2, 65, 100), (2, 1, 128, 128),
+                                      (1, 3, 130, 126), (5, 3, 200, 80), (1, 1, 255, 48), (1, 2, 400, 128),
+                                      (1, 1, 509, 24), (1, 1, 512, 128)])
+def test_f32_step_matches_float64_and_the_separate_launches(dev, b, h, t, hd, monkeypatch):
+    g = torch.Generator(device="cpu").manual_seed(t * 131 + hd)
+    d = h * hd
+    qkv, dctx = torch.randn(b * t, 3 * d, generator=g), torch.randn(b * t, d, generator=g)
+    assert attention._f32_step(qkv, None, attention.AttnBuffers.empty(b, h, t, hd, "cpu"), b, h, t, hd, False)
+    got = f32_step(dev, b, h, t, hd, qkv.to(dev), dctx.to(dev), False, monkeypatch)
+    old = f32_step(dev, b, h, t, hd, qkv.to(dev), dctx.to(dev), True, monkeypatch)
+    q, k, v = qkv.double().view(b, t, 3, h, hd).permute(2, 0, 3, 1, 4).contiguous()
+    do = dctx.double().view(b, t, h, hd).permute(0, 2, 1, 3)
+    s = q @ k.transpose(-1, -2)
+    scale = hd ** -0.5
+    p = torch.softmax((s * scale).masked_fill(torch.ones(t, t, dtype=torch.bool).triu(1), -np.inf), -1)
+    dp = do @ v.transpose(-1, -2)
+    ds = scale * p * (dp - (dp * p).sum(-1, keepdim=True))
+    merge = lambda x: x.permute(0, 2, 1, 3).reshape(b * t, d)
+    dqkv = torch.cat([merge(ds @ k), merge(ds.transpose(-1, -2) @ q), merge(p.transpose(-1, -2) @ do)], 1)
+    wants = [s, p, merge(p @ v), dp, ds, dqkv]
+    # Sums of up to max(t, hd) f32 terms on either side: 1e-5 of the scale for the forward, 1e-4 for what passes
+    # through the softmax's gradient (the bounds of the f32 chain's test above).
+    for name, x, y, want, tol in zip("s p ctx dp ds dqkv".split(), got, old, wants, [1e-5] * 4 + [1e-4] * 2):
+        w = want.reshape(-1).numpy()
+        top = max(np.max(np.abs(w)), 1e-30)
+        assert np.max(np.abs(x - w)) <= tol * top, name
+        assert np.max(np.abs(x - y)) <= 2 * tol * top, name
+
+
+def test_f32_step_keeps_infinities_and_nans_where_the_separate_launches_have_them(dev, monkeypatch):
+    b, h, t, hd = 2, 2, 70, 20
+    g = torch.Generator(device="cpu").manual_seed(8)
+    for part, row, value in [(0, 5, np.inf), (1, 69, np.nan), (1, 40, -np.inf), (2, 69, np.inf), (2, 10, np.nan)]:
+        qkv, dctx = torch.randn(b * t, 3 * h * hd, generator=g), torch.randn(b * t, h * hd, generator=g)
+        qkv[row, part * h * hd + 3] = value
+        got = f32_step(dev, b, h, t, hd, qkv.to(dev), dctx.to(dev), False, monkeypatch)
+        old = f32_step(dev, b, h, t, hd, qkv.to(dev), dctx.to(dev), True, monkeypatch)
+        for name, x, y in zip("s p ctx dp ds dqkv".split(), got, old):
+            fine = np.isfinite(y)
+            np.testing.assert_array_equal(np.isfinite(x), fine, err_msg=f"{name} {part} {row} {value}")
+            assert np.max(np.abs(x[fine] - y[fine]), initial=0.0) <= 2e-4 * max(np.max(np.abs(y[fine]), initial=0.0), 1.0), name
