@@ -567,12 +567,14 @@ __device__ __attribute__((noinline)) Kept merge_new_keys(lds_u64 *wl, int na, in
 // workgroup 0 writes the number of runs to runs[q], and k_merge_splits combines
 // their lists.  A query of one run is finished by workgroup 0.  The k smallest
 // keys of the whole lie among the runs' k smallest, so the results are the
-// same.  Bound by latency: about 25 us from launch to output for any run (first
-// loads 4, the two merges of each wave's list 3 each, barriers, the final ranks
-// 1 to 5), then 0.7 us per chunk and wave.  4 queries of 1,270 chunks: 203 us
-// unsplit, 36 in 32 runs with the merge; 32 queries of 330: 60 and 39.
+// same.  Bound by latency: about 16 us from launch to output for a run of 32
+// chunks (first loads 4, the two merges of each wave's list 3 each, barriers),
+// then about 0.1 us per chunk, and the merge launch.  4 queries of 1,270
+// chunks: 203 us unsplit, 34 in 32 runs with the merge; 32 queries of 234: 57
+// and 26.
 constexpr int SPLIT_MIN = 4 * SW;  // chunks per run (four per wave)
 constexpr int SPLIT_MAX = 32;      // runs per query
+constexpr int SPLIT_FROM = 48;     // a query of at most so many chunks stays whole (23 us; 2 or 3 runs take 25)
 
 template <bool MASKED>
 __global__ __launch_bounds__(STH) void k_search(const uint8_t *codes, const float *scales,
@@ -583,7 +585,6 @@ __global__ __launch_bounds__(STH) void k_search(const uint8_t *codes, const floa
                                                 int64_t always, int64_t nkeys, int32_t nsplit,
                                                 uint64_t *__restrict__ parts, int32_t *__restrict__ runs) {
     __shared__ uint64_t cand[SW * CAPW];  // per-wave candidate lists
-    __shared__ uint64_t fin[SW * KMAX];   // the final gather
     __shared__ uint64_t s_tau;            // shared threshold (only decreases)
     __shared__ uint64_t s_e8[SW];         // each wave's E8-th smallest kept key
     __shared__ int16_t s_Q[D];
@@ -672,7 +673,8 @@ __global__ __launch_bounds__(STH) void k_search(const uint8_t *codes, const floa
     const int np = s_np;
     const int64_t nrows = s_nrows;
     const int32_t all = s_cpre[np];
-    const int32_t run = nsplit == 1 ? all : max(SPLIT_MIN, (all + nsplit - 1) / nsplit);
+    const int32_t run =
+        nsplit == 1 || all <= SPLIT_FROM ? max(all, 1) : max(SPLIT_MIN, (all + nsplit - 1) / nsplit);
     const bool last = all <= run;  // one run: this query's results are written here
     const int32_t begin = split * run;  // split * run < 2^31: run <= nchunks / nsplit + SPLIT_MIN
     const int32_t nchunks = min(all, begin + run);
@@ -817,37 +819,47 @@ __global__ __launch_bounds__(STH) void k_search(const uint8_t *codes, const floa
         else
             scan(std::integral_constant<bool, false>());
     }
-    // Final: every wave sorts its list and keeps at most its best 128; the keys
-    // at or below the final threshold (a superset of the query's top 128, at
-    // most SW x 128) are gathered, and each one's rank among them (keys are
-    // distinct: the index is part of the key) is its output position.
+    // Final: every wave sorts its list and keeps at most its best 128.  A kept
+    // key at or below the final threshold (which has the query's top 128 at or
+    // below it) goes to its rank: the number of smaller keys in each wave's list,
+    // by binary search (a list's 128 slots are sorted throughout: dropped keys
+    // and NONE follow the kept ones, and keys are distinct, the index being part
+    // of them).  Ranking the gathered keys against each other took 1 us for 160
+    // of them and 5 for the 570 a short scan leaves.
     wave_compact();
     __syncthreads();
-    {
-        const uint64_t m = wave_max_u64(lane < SW ? s_e8[lane] : 0ull);
-        const uint64_t ts = s_tau;
-        const uint64_t tfin = m < ts ? m : ts;
-        for (int i = lane; i < na; i += 64) {
-            const uint64_t e = wl[i];
-            if (e <= tfin) fin[atomicAdd(&count, 1)] = e;
-        }
-    }
-    __syncthreads();
-    const int cnt = count;
     const float qn = s_qn;
-    for (int t = tid; t < cnt; t += STH) {
-        const uint64_t e = fin[t];
+    const uint64_t m8 = wave_max_u64(lane < SW ? s_e8[lane] : 0ull);
+    const uint64_t ts = s_tau, tfin = m8 < ts ? m8 : ts;
+#pragma unroll
+    for (int i = 0; i < KMAX; i += 64) {
+        const uint64_t e = wl[i + lane];
+        const bool keep = i + lane < na && e <= tfin;
+        const int kept = __popcll(__ballot(keep));
+        if (kept == 0) break;  // uniform over the wave
+        if (lane == 0) atomicAdd(&count, kept);
+        int below[SW];
+#pragma unroll
+        for (int x = 0; x < SW; x++) below[x] = 0;
+#pragma unroll
+        for (int step = KMAX / 2; step > 0; step >>= 1)
+#pragma unroll
+            for (int x = 0; x < SW; x++)
+                if (cand[x * CAPW + below[x] + step - 1] < e) below[x] += step;
         int r = 0;
-        for (int j = 0; j < cnt; j++) r += fin[j] < e;
-        if (r < k && !last) {
+#pragma unroll
+        for (int x = 0; x < SW; x++) r += below[x] + (cand[x * CAPW + below[x]] < e);
+        if (!keep || r >= k) continue;
+        if (!last) {
             parts[(int64_t)blockIdx.x * KMAX + r] = e;
-        } else if (r < k) {
+        } else {
             const float v = qn + unfkey((uint32_t)(e >> 32));
             out_idx[q * k + r] = (int64_t)(uint32_t)e;
             out_dist[q * k + r] = v > 0.f ? v : 0.f;
         }
     }
-    for (int j = cnt + tid; j < k; j += STH) {
+    __syncthreads();
+    for (int j = count + tid; j < k; j += STH) {
         if (!last) {
             parts[(int64_t)blockIdx.x * KMAX + j] = NONE;
         } else {
@@ -1496,7 +1508,8 @@ extern "C" st_status st_knn_search_ivf_2bit_split(const uint8_t *codes, const fl
     if (!cells) {
         // Cells too small for that many runs (max_cell bounds them) give fewer.
         SplitWork w = split_work(work, work_bytes, nq);
-        w.nsplit = std::max<int64_t>(1, std::min(w.nsplit, nprobe * cdiv(max_cell, 64) / SPLIT_MIN));
+        const int64_t most = nprobe * cdiv(max_cell, 64);
+        w.nsplit = most <= SPLIT_FROM ? 1 : std::max<int64_t>(1, std::min(w.nsplit, most / SPLIT_MIN));
         hipLaunchKernelGGL(k_search<false>, dim3((unsigned)(nq * w.nsplit)), dim3(STH), 0, s, codes, scales,
                            cell_start, ncells, queries, probes, (int32_t)nq, (int32_t)nprobe, (int32_t)k, out_idx,
                            out_dist, nullptr, (int64_t)0, (int64_t)0, (int32_t)w.nsplit, w.parts, w.runs);
@@ -1577,7 +1590,8 @@ extern "C" st_status st_knn_search_masked_2bit_split(const uint8_t *codes, const
     // store, and the workgroups past its last run end at once.
     const hipStream_t s = st::stream_of(stream);
     SplitWork w = split_work(work, work_bytes, nq);
-    w.nsplit = std::max<int64_t>(1, std::min(w.nsplit, cdiv(nkeys, 64) / SPLIT_MIN));
+    const int64_t most = cdiv(nkeys, 64) + 1;  // two segments
+    w.nsplit = most <= SPLIT_FROM ? 1 : std::max<int64_t>(1, std::min(w.nsplit, most / SPLIT_MIN));
     hipLaunchKernelGGL(k_search<true>, dim3((unsigned)(nq * w.nsplit)), dim3(STH), 0, s, codes, scales, nullptr,
                        (int64_t)0, queries, nullptr, (int32_t)nq, 0, (int32_t)k, out_idx, out_dist, lohi, always,
                        nkeys, (int32_t)w.nsplit, w.parts, w.runs);

@@ -340,9 +340,9 @@ def unsplit_masked(store, queries, lohi, always, k):
     return idx, dist
 
 
-# Small batches split a query over several workgroups, in runs of at least 32 chunks of 64 keys: no key, one run, its
-# edge, a second run of one key, many runs, and as many as there can be; 1 query (32 runs at most), 100 (2), 128 (2)
-# and 129 (not split).
+# Small batches split a query of more than 48 chunks of 64 keys over several workgroups, in runs of at least 32: no key,
+# one run, its edge (3,072 keys), a last run of one key, many runs, and as many as there can be; 1 query (32 runs at
+# most), 100 (2), 128 (2) and 129 (not split).
 @pytest.mark.parametrize("nq", [1, 9, 100, 128, 129])
 @pytest.mark.parametrize("k", [128, 5])
 def test_split_search_equals_one_workgroup_per_query(dev, nq, k):
@@ -352,10 +352,10 @@ def test_split_search_equals_one_workgroup_per_query(dev, nq, k):
     scales = torch.empty(n, dtype=torch.float32, device=dev)
     knn.synth_store_2bit(9, 0, codes, scales)
     order = torch.argsort(scales)  # norms rise with the row: the nearest keys of a query lie in a few runs
-    cuts = np.array([0, 2000, 2048, 2049, 2112, 10000, 10001, 60000, n])
+    cuts = np.array([0, 2000, 3072, 3073, 5248, 10000, 10001, 60000, n])
     store = knn.KnnStore2bit(codes[order].contiguous(), scales[order].contiguous(), cuts)
     q = torch.from_numpy(rng.standard_normal((nq, D)).astype(np.float32)).to(dev)
-    length = np.array([0, 3, 1900, 2048, 2049, 4096, 30000, 80000])[np.arange(nq) % 8]
+    length = np.array([80000, 3, 1900, 3072, 3073, 4097, 30000, 0])[np.arange(nq) % 8]
     lo = rng.integers(always, n - length)
     lohi = torch.from_numpy(np.stack([lo, lo + length], 1)).to(dev)
     for first in (0, always):
