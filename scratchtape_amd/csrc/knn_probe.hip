@@ -45,6 +45,8 @@
 // of the slice's tiles (two waves per SIMD hide each other's latencies).
 // dd never leaves the chip; per query only the candidates (about nprobe per
 // slice) are written and read back.
+#include <algorithm>
+
 #include "common.h"
 #include "lanes.h"
 
@@ -200,8 +202,21 @@ constexpr int32_t INONE = 0x7fffffff;
 // to fill the chip, fewer for small indexes and batches, where each workgroup
 // is a chain of latencies (staging, scoring, threshold, candidates) and more
 // workgroups shorten it.
-template <int HT>
-__global__ __launch_bounds__(PART_T) void k_probe_part(const float *__restrict__ queries, int32_t nq,
+//
+// MANY: the grid holds gw < gy workgroups per slice (about one per CU), and
+// each takes the query groups qg, qg + gw, .. against the slice that it staged
+// once; the queries' digits qdig and exponents qexp come from k_probe_prep, and
+// a wave loads the next group's straight into the registers of the last one
+// while it forms its keys.  Without it every (slice, group) pair stages the
+// slice and turns the queries into digits again, 64 times over for a large
+// index.  Bound by the VALU (about 2,000 instructions per wave and group: the
+// keys, their order, the candidates).  Both launches, us, one group each and
+// now: 4,096 queries over 12,288 cells 298 -> 180, over 6,000 (16 probes) 178 ->
+// 109, over 20,000 487 -> 370; 512 over 12,288 44 -> 39; 2,048 over 4,000 61 -> 49.
+template <int HT, bool MANY>
+__global__ __launch_bounds__(PART_T) void k_probe_part(const float *__restrict__ queries,
+                                                    const int8_t *__restrict__ qdig,
+                                                    const int32_t *__restrict__ qexp, int32_t gw, int32_t nq,
                                                     const int8_t *__restrict__ cdig, const int32_t *__restrict__ cexp,
                                                     const double *__restrict__ cnorm, int32_t nlist, int32_t S,
                                                     int32_t gy, int32_t nprobe, uint64_t *__restrict__ ck,
@@ -210,14 +225,16 @@ __global__ __launch_bounds__(PART_T) void k_probe_part(const float *__restrict__
     __shared__ v4i s_b[TPS * TILE_BYTES / 16];
     __shared__ double s_cn[TPS * TILE];
     __shared__ int32_t s_ce[TPS * TILE];
-    __shared__ uint32_t s_x[2][4][64][4];  // per (half, query tile, lane, u): sorted minima, then counts
-    __shared__ v4i s_q[4 * TILE_BYTES / 16];  // the workgroup's 64 queries as 4 digit tiles
-    __shared__ int32_t s_qe[QG];              // and their exponents
+    // Per (half, query tile, lane, u).  Each is written between the barrier after the other's and its own.
+    __shared__ uint32_t s_min[2][4][64][4];  // sorted minima
+    __shared__ int32_t s_cnt[2][4][64][4];   // candidates
+    __shared__ v4i s_q[MANY ? 1 : 4 * TILE_BYTES / 16];  // the workgroup's 64 queries as 4 digit tiles
+    __shared__ int32_t s_qe[MANY ? 1 : QG];              // and their exponents
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int qt = w & 3, half = w >> 2;  // query tile; tiles [half HT, half HT + HT) of the slice
-    const int64_t nb = (int64_t)S * gy, b = blockIdx.x;
+    const int64_t nb = (int64_t)S * gw, b = blockIdx.x;
     const int64_t idx = nb % 8 == 0 ? (b % 8) * (nb / 8) + b / 8 : b;
-    const int32_t sl = (int32_t)(idx / gy), qg = (int32_t)(idx % gy);
+    const int32_t sl = (int32_t)(idx / gw), qg0 = (int32_t)(idx % gw);
     const int32_t ntiles = (nlist + TILE - 1) / TILE;
     const int32_t t0 = sl * TPS, nts = min(TPS, ntiles - t0);
 
@@ -240,11 +257,11 @@ __global__ __launch_bounds__(PART_T) void k_probe_part(const float *__restrict__
     // rows' loads in flight together; a query past nq is a zero row).  Every
     // slice's workgroup redoes this for its query group: 64 KB of f32 reads,
     // in place of a separate launch.
-    {
+    if constexpr (!MANY) {
         float4 f[8];
 #pragma unroll
         for (int t = 0; t < 8; t++) {
-            const int32_t q = qg * QG + w * 8 + t;
+            const int32_t q = qg0 * QG + w * 8 + t;
             f[t] = q < nq ? reinterpret_cast<const float4 *>(queries + (int64_t)q * D)[lane]
                           : make_float4(0.f, 0.f, 0.f, 0.f);
         }
@@ -276,11 +293,6 @@ __global__ __launch_bounds__(PART_T) void k_probe_part(const float *__restrict__
     // query (l % 32) / 2, digit l % 2, dims 32 s + 16 (l / 32) ..
     const int h = lane >> 5, odd = lane & 1;
     const int q16 = (lane & 31) >> 1;
-    const int32_t qbase = qg * QG + qt * 16;
-    const bool wact = qbase < nq;
-    v4i a[8];
-#pragma unroll
-    for (int s = 0; s < 8; s++) a[s] = wact ? s_q[qt * (TILE_BYTES / 16) + s * 64 + lane] : v4i{0, 0, 0, 0};
 
     // Output layout of the 32 x 32 MFMA: lane l holds column l % 32 (centroid
     // c16 = (l % 32) / 2, digit l % 2) and rows 8 j + 4 h + i (i < 4, j < 4):
@@ -290,219 +302,232 @@ __global__ __launch_bounds__(PART_T) void k_probe_part(const float *__restrict__
     // 4 (2 odd + u / 2) + 2 h + u % 2.
     const int c16 = q16;
     int qu[4], qeu[4];
+    v4i a[8];
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-        qu[u] = 4 * (2 * odd + u / 2) + 2 * h + (u & 1);
-        qeu[u] = qbase + qu[u] < nq ? s_qe[qt * 16 + qu[u]] : 0;
-    }
-    // Every tile slot is scored (branch-free): a slot past the slice's tiles
-    // reads stale LDS, and its centroid ids are >= nlist, so its keys are none.
-    uint64_t key[HT][4];
-    uint32_t mn[4] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu};
-    // The MFMAs of TG tiles at a time, k-step by k-step: TG independent
-    // accumulator chains interleaved keep the matrix core busy (each MFMA's
-    // input is TG instructions old); the group's keys are formed afterwards.
-    constexpr int TG = HT % 3 == 0 ? 3 : HT;
-    static_assert(HT % TG == 0, "tile groups");
+    for (int u = 0; u < 4; u++) qu[u] = 4 * (2 * odd + u / 2) + 2 * h + (u & 1);
+    auto load_a = [&](int32_t qb) __attribute__((always_inline)) {  // qb: the wave's first query
+        const v4i *src = MANY ? reinterpret_cast<const v4i *>(qdig) + (int64_t)(qb / TILE) * (TILE_BYTES / 16)
+                              : s_q + qt * (TILE_BYTES / 16);
 #pragma unroll
-    for (int g0 = 0; g0 < HT; g0 += TG) {
-        v16i acc[TG];
+        for (int s = 0; s < 8; s++) a[s] = qb < nq ? src[s * 64 + lane] : v4i{0, 0, 0, 0};
+    };
+    auto load_e = [&](int32_t qb) __attribute__((always_inline)) {
 #pragma unroll
-        for (int t = 0; t < TG; t++)
+        for (int u = 0; u < 4; u++) qeu[u] = qb + qu[u] < nq ? (MANY ? qexp[qb + qu[u]] : s_qe[qt * 16 + qu[u]]) : 0;
+    };
+    load_a(qg0 * QG + qt * 16);
+    load_e(qg0 * QG + qt * 16);
+    for (int32_t qg = qg0; qg < gy; qg += gw) {  // one group unless MANY
+        if constexpr (MANY) asm volatile("" ::: "memory");  // the slice's norms stay in LDS between the groups
+        const int32_t qbase = qg * QG + qt * 16;
+        // Every tile slot is scored (branch-free): a slot past the slice's tiles
+        // reads stale LDS, and its centroid ids are >= nlist, so its keys are none.
+        uint64_t key[HT][4];
+        uint32_t mn[4] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu};
+        // The MFMAs of TG tiles at a time, k-step by k-step: TG independent
+        // accumulator chains interleaved keep the matrix core busy (each MFMA's
+        // input is TG instructions old); the group's keys are formed afterwards.
+        constexpr int TG = HT % 3 == 0 ? 3 : HT;
+        static_assert(HT % TG == 0, "tile groups");
 #pragma unroll
-            for (int i = 0; i < 16; i++) acc[t][i] = 0;
-#pragma unroll
-        for (int s = 0; s < 8; s++)
+        for (int g0 = 0; g0 < HT; g0 += TG) {
+            v16i acc[TG];
 #pragma unroll
             for (int t = 0; t < TG; t++)
-                acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[s], s_b[(half * HT + g0 + t) * 512 + s * 64 + lane],
-                                                              acc[t], 0, 0, 0);
 #pragma unroll
-        for (int t = 0; t < TG; t++) {
-            const int k0 = g0 + t, k = half * HT + k0;
-            // The even lane holds the products with the centroid's high digit,
-            // the odd lane those with its low digit; each sends the other the
-            // eight it needs.
-            // (Selections by a mask, not by ?: on the two elements, which the
-            // compiler would fold into a run-time index into acc.)
-            const int32_t om = -odd;
-            int32_t pch[8], pcl[8];
+                for (int i = 0; i < 16; i++) acc[t][i] = 0;
 #pragma unroll
-            for (int v = 0; v < 8; v++) {
-                const int32_t lo8 = acc[t][v], hi8 = acc[t][8 + v];
-                const int32_t own = lo8 ^ ((lo8 ^ hi8) & om);
-                const int32_t got = st::xor_lane(hi8 ^ ((lo8 ^ hi8) & om), 1, lane);
-                pch[v] = own ^ ((own ^ got) & om);
-                pcl[v] = got ^ ((own ^ got) & om);
-            }
-            const int32_t c = (t0 + k) * TILE + c16;
-            const double cn = s_cn[k * TILE + c16];
-            const int ce = s_ce[k * TILE + c16];
+            for (int s = 0; s < 8; s++)
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int o = 4 * (u / 2) + 2 * (u & 1);
-                const int64_t dot = (int64_t)pch[o] * 65536 + (int64_t)(pcl[o] + pch[o + 1]) * 256 + pcl[o + 1];
-                const double dd = cn - ldexp((double)dot, qeu[u] + ce + 1);
-                key[k0][u] = k < nts && c < nlist ? dkey(dd) : KNONE;
-                mn[u] = min(mn[u], (uint32_t)(key[k0][u] >> 32));
-            }
-        }
-    }
-
-    // Per query, the nprobe-th smallest of the 32 minima of its lanes in both
-    // halves: for a given u the 16 lanes of an (h, parity) group hold one
-    // query, one per centroid position c16 (lane bits 1..4).  Each half sorts
-    // its 16 minima over c16 (bitonic, by shuffles); the minimum of each and
-    // the other half's mirrored one is a bitonic sequence of the 16 smallest of
-    // the 32, which a bitonic merge sorts: the r-th smallest is in c16 = r.
-    auto order = [&](uint32_t x, int kk) __attribute__((always_inline)) {
+                for (int t = 0; t < TG; t++)
+                    acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+                        a[s], s_b[(half * HT + g0 + t) * 512 + s * 64 + lane], acc[t], 0, 0, 0);
+            if (MANY && g0 + TG == HT && qg + gw < gy) load_a(qbase + gw * QG);
 #pragma unroll
-        for (int j = kk >> 1; j > 0; j >>= 1) {
-            const uint32_t y = st::xor_lane(x, 2 * j, lane);
-            const bool take_min = ((c16 & j) == 0) == ((c16 & kk) == 0);
-            x = take_min ? min(x, y) : max(x, y);
-        }
-        return x;
-    };
+            for (int t = 0; t < TG; t++) {
+                const int k0 = g0 + t, k = half * HT + k0;
+                // The even lane holds the products with the centroid's high digit,
+                // the odd lane those with its low digit; each sends the other the
+                // eight it needs.
+                // (Selections by a mask, not by ?: on the two elements, which the
+                // compiler would fold into a run-time index into acc.)
+                const int32_t om = -odd;
+                int32_t pch[8], pcl[8];
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-        mn[u] = order(order(order(order(mn[u], 2), 4), 8), 16);
-        s_x[half][qt][lane][u] = mn[u];
-    }
-    __syncthreads();
-    uint32_t tau[4];
-    const int mirror = lane ^ 30;  // the same group's lane of 15 - c16
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        const uint32_t x = order(min(mn[u], s_x[half ^ 1][qt][mirror][u]), 16);
-        // Lane 32 h + 2 (nprobe - 1) + odd's x: four uniform reads, one picked per lane.
-        const int b = 2 * (nprobe - 1);
-        const uint32_t t0 = st::lane_value(x, b), t1 = st::lane_value(x, b + 1), t2 = st::lane_value(x, b + 32),
-                       t3 = st::lane_value(x, b + 33);
-        tau[u] = h ? (odd ? t3 : t2) : (odd ? t1 : t0);
-    }
-    __syncthreads();
-
-    // Candidates: the keys at or below their query's threshold, written at the
-    // count of the group's earlier candidates (a prefix sum over c16), from the
-    // slot's start by the wave of tiles 0 .. HT - 1 and from its end by the
-    // other.  The slot overflows when the two counts exceed CAPQ together.
-    int cnt[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        const int32_t q = qbase + qu[u];
-        uint32_t pm = 0;
-#pragma unroll
-        for (int k = 0; k < HT; k++) {
-            const uint64_t kk = key[k][u];
-            pm |= (uint32_t)(q < nq && kk != KNONE && (uint32_t)(kk >> 32) <= tau[u]) << k;
-        }
-        const int n = __popc(pm);
-        // Inclusive sum over the group's c16 = 0 .. 15 (lanes 32 h + 2 c16 +
-        // odd): DPP row shifts by 2, 4, 8 lanes scan the 8 positions of each
-        // 16-lane row, then the second row of each half adds the first row's
-        // total of its parity.
-        int incl = n;
-        incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xF, 0xF, true);
-        incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xF, 0xF, true);
-        incl += __builtin_amdgcn_update_dpp(0, incl, 0x118, 0xF, 0xF, true);
-        {
-            const int r0 = st::lane_value(incl, 14), r1 = st::lane_value(incl, 15), r2 = st::lane_value(incl, 46),
-                      r3 = st::lane_value(incl, 47);
-            if (lane & 16) incl += h ? (odd ? r3 : r2) : (odd ? r1 : r0);
-        }
-        {
-            const int c0 = st::lane_value(incl, 30), c1 = st::lane_value(incl, 31), c2 = st::lane_value(incl, 62),
-                      c3 = st::lane_value(incl, 63);
-            cnt[u] = h ? (odd ? c3 : c2) : (odd ? c1 : c0);
-        }
-        int pos = incl - n;
-        uint64_t *sk = ck + (int64_t)q * S * CAPQ + sl;
-        int32_t *si = ci + (int64_t)q * S * CAPQ + sl;
-#pragma unroll
-        for (int k = 0; k < HT; k++) {
-            if ((pm >> k) & 1) {
-                if (pos < CAPQ) {
-                    const int64_t at = (int64_t)(half ? CAPQ - 1 - pos : pos) * S;
-                    sk[at] = key[k][u];
-                    si[at] = (t0 + half * HT + k) * TILE + c16;
+                for (int v = 0; v < 8; v++) {
+                    const int32_t lo8 = acc[t][v], hi8 = acc[t][8 + v];
+                    const int32_t own = lo8 ^ ((lo8 ^ hi8) & om);
+                    const int32_t got = st::xor_lane(hi8 ^ ((lo8 ^ hi8) & om), 1, lane);
+                    pch[v] = own ^ ((own ^ got) & om);
+                    pcl[v] = got ^ ((own ^ got) & om);
                 }
-                pos++;
+                const int32_t c = (t0 + k) * TILE + c16;
+                const double cn = s_cn[k * TILE + c16];
+                const int ce = s_ce[k * TILE + c16];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int o = 4 * (u / 2) + 2 * (u & 1);
+                    // |hl + lh| <= 2^22 and |ll| <= 2^22, so the lower part fits 32 bits; the sum is exact.
+                    const int32_t low = (pcl[o] + pch[o + 1]) * 256 + pcl[o + 1];
+                    const double dot = (double)pch[o] * 65536.0 + (double)low;
+                    const double dd = cn - ldexp(dot, qeu[u] + ce + 1);
+                    key[k0][u] = k < nts && c < nlist ? dkey(dd) : KNONE;
+                    mn[u] = min(mn[u], (uint32_t)(key[k0][u] >> 32));
+                }
             }
         }
-        s_x[half][qt][lane][u] = (uint32_t)cnt[u];
-    }
-    __syncthreads();
-    bool over = false;
-    bool ov[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        ov[u] = cnt[u] + (int)s_x[half ^ 1][qt][lane][u] > CAPQ;
-        over |= ov[u];
-    }
 
-    // A slot that overflowed gets each half's exact top nprobe instead (at the
-    // slot's two ends): nprobe successive minima by (key, id) over the group's
-    // registers, strictly above the last one taken (the four groups of a u at
-    // once).
-    if (__ballot(over)) {
+        if (MANY && qg + gw < gy) load_e(qbase + gw * QG);
+
+        // Per query, the nprobe-th smallest of the 32 minima of its lanes in both
+        // halves: for a given u the 16 lanes of an (h, parity) group hold one
+        // query, one per centroid position c16 (lane bits 1..4).  Each half sorts
+        // its 16 minima over c16 (bitonic, by shuffles); the minimum of each and
+        // the other half's mirrored one is a bitonic sequence of the 16 smallest of
+        // the 32, which a bitonic merge sorts: the r-th smallest is in c16 = r.
+        auto order = [&](uint32_t x, int kk) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = kk >> 1; j > 0; j >>= 1) {
+                const uint32_t y = st::xor_lane(x, 2 * j, lane);
+                const bool take_min = ((c16 & j) == 0) == ((c16 & kk) == 0);
+                x = take_min ? min(x, y) : max(x, y);
+            }
+            return x;
+        };
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            const bool mine = ov[u];
-            if (!__ballot(mine)) continue;
+            mn[u] = order(order(order(order(mn[u], 2), 4), 8), 16);
+            s_min[half][qt][lane][u] = mn[u];
+        }
+        __syncthreads();
+        uint32_t tau[4];
+        const int mirror = lane ^ 30;  // the same group's lane of 15 - c16
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const uint32_t x = order(min(mn[u], s_min[half ^ 1][qt][mirror][u]), 16);
+            // Lane 32 h + 2 (nprobe - 1) + odd's x: four uniform reads, one picked per lane.
+            const int b = 2 * (nprobe - 1);
+            const uint32_t t0 = st::lane_value(x, b), t1 = st::lane_value(x, b + 1), t2 = st::lane_value(x, b + 32),
+                           t3 = st::lane_value(x, b + 33);
+            tau[u] = h ? (odd ? t3 : t2) : (odd ? t1 : t0);
+        }
+
+        // Candidates: the keys at or below their query's threshold, written at the
+        // count of the group's earlier candidates (a prefix sum over c16), from the
+        // slot's start by the wave of tiles 0 .. HT - 1 and from its end by the
+        // other.  The slot overflows when the two counts exceed CAPQ together.
+        int cnt[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
             const int32_t q = qbase + qu[u];
+            uint32_t pm = 0;
+#pragma unroll
+            for (int k = 0; k < HT; k++) {
+                const uint64_t kk = key[k][u];
+                pm |= (uint32_t)(q < nq && kk != KNONE && (uint32_t)(kk >> 32) <= tau[u]) << k;
+            }
+            const int n = __popc(pm);
+            // Inclusive sum over the group's c16 = 0 .. 15 (lanes 32 h + 2 c16 +
+            // odd): DPP row shifts by 2, 4, 8 lanes scan the 8 positions of each
+            // 16-lane row, then the second row of each half adds the first row's
+            // total of its parity.
+            int incl = n;
+            incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xF, 0xF, true);
+            incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xF, 0xF, true);
+            incl += __builtin_amdgcn_update_dpp(0, incl, 0x118, 0xF, 0xF, true);
+            {
+                const int r0 = st::lane_value(incl, 14), r1 = st::lane_value(incl, 15), r2 = st::lane_value(incl, 46),
+                          r3 = st::lane_value(incl, 47);
+                if (lane & 16) incl += h ? (odd ? r3 : r2) : (odd ? r1 : r0);
+            }
+            {
+                const int c0 = st::lane_value(incl, 30), c1 = st::lane_value(incl, 31), c2 = st::lane_value(incl, 62),
+                          c3 = st::lane_value(incl, 63);
+                cnt[u] = h ? (odd ? c3 : c2) : (odd ? c1 : c0);
+            }
+            int pos = incl - n;
             uint64_t *sk = ck + (int64_t)q * S * CAPQ + sl;
             int32_t *si = ci + (int64_t)q * S * CAPQ + sl;
-            uint64_t lk = 0;
-            int32_t li = -1;
-            int found = 0;
-            for (int r = 0; r < nprobe; r++) {
-                uint64_t bk = KNONE;
-                int32_t bi = INONE;
 #pragma unroll
-                for (int k = 0; k < HT; k++) {
-                    const uint64_t kk = key[k][u];
-                    const int32_t id = (t0 + half * HT + k) * TILE + c16;
-                    if (kk != KNONE && lt(lk, li, kk, id) && lt(kk, id, bk, bi)) {
-                        bk = kk;
-                        bi = id;
+            for (int k = 0; k < HT; k++) {
+                if ((pm >> k) & 1) {
+                    if (pos < CAPQ) {
+                        const int64_t at = (int64_t)(half ? CAPQ - 1 - pos : pos) * S;
+                        sk[at] = key[k][u];
+                        si[at] = (t0 + half * HT + k) * TILE + c16;
                     }
-                }
-#pragma unroll
-                for (int d = 2; d < 32; d <<= 1) {  // minimum over the group (lane bits 1..4)
-                    const uint64_t ko = shfl_xor_u64(bk, d);
-                    const int32_t io = st::xor_lane(bi, d, lane);
-                    if (lt(ko, io, bk, bi)) {
-                        bk = ko;
-                        bi = io;
-                    }
-                }
-                if (!(bk == KNONE && bi == INONE)) {
-                    if (mine && c16 == 0) {
-                        const int64_t at = (int64_t)(half ? CAPQ - 1 - r : r) * S;
-                        sk[at] = bk;
-                        si[at] = bi;
-                    }
-                    lk = bk;
-                    li = bi;
-                    found = r + 1;
+                    pos++;
                 }
             }
-            if (mine) cnt[u] = found;
+            s_cnt[half][qt][lane][u] = cnt[u];
         }
-    }
-    __syncthreads();
+        __syncthreads();
+        bool over = false;
+        bool ov[4];
 #pragma unroll
-    for (int u = 0; u < 4; u++) s_x[half][qt][lane][u] = (uint32_t)min(cnt[u], CAPQ);
-    __syncthreads();
-    // The slot's count: low 16 bits from its start, high 16 bits from its end.
-    if (half == 0) {
+        for (int u = 0; u < 4; u++) {
+            ov[u] = cnt[u] + s_cnt[half ^ 1][qt][lane][u] > CAPQ;
+            over |= ov[u];
+        }
+
+        // A slot that overflowed gets each half's exact top nprobe instead (at the
+        // slot's two ends): nprobe successive minima by (key, id) over the group's
+        // registers, strictly above the last one taken (the four groups of a u at
+        // once).
+        if (__ballot(over)) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const bool mine = ov[u];
+                if (!__ballot(mine)) continue;
+                const int32_t q = qbase + qu[u];
+                uint64_t *sk = ck + (int64_t)q * S * CAPQ + sl;
+                int32_t *si = ci + (int64_t)q * S * CAPQ + sl;
+                uint64_t lk = 0;
+                int32_t li = -1;
+                int found = 0;
+                for (int r = 0; r < nprobe; r++) {
+                    uint64_t bk = KNONE;
+                    int32_t bi = INONE;
+#pragma unroll
+                    for (int k = 0; k < HT; k++) {
+                        const uint64_t kk = key[k][u];
+                        const int32_t id = (t0 + half * HT + k) * TILE + c16;
+                        if (kk != KNONE && lt(lk, li, kk, id) && lt(kk, id, bk, bi)) {
+                            bk = kk;
+                            bi = id;
+                        }
+                    }
+#pragma unroll
+                    for (int d = 2; d < 32; d <<= 1) {  // minimum over the group (lane bits 1..4)
+                        const uint64_t ko = shfl_xor_u64(bk, d);
+                        const int32_t io = st::xor_lane(bi, d, lane);
+                        if (lt(ko, io, bk, bi)) {
+                            bk = ko;
+                            bi = io;
+                        }
+                    }
+                    if (!(bk == KNONE && bi == INONE)) {
+                        if (mine && c16 == 0) {
+                            const int64_t at = (int64_t)(half ? CAPQ - 1 - r : r) * S;
+                            sk[at] = bk;
+                            si[at] = bi;
+                        }
+                        lk = bk;
+                        li = bi;
+                        found = r + 1;
+                    }
+                }
+                if (mine) cnt[u] = found;
+            }
+        }
+        // The slot's count: low 16 bits from its start, high 16 bits from its end.
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const int32_t q = qbase + qu[u];
             if (c16 == 0 && q < nq)
-                pcnt[(int64_t)q * S + sl] = (int32_t)(s_x[0][qt][lane][u] | (s_x[1][qt][lane][u] << 16));
+                reinterpret_cast<uint16_t *>(pcnt)[2 * ((int64_t)q * S + sl) + half] = (uint16_t)min(cnt[u], CAPQ);
         }
+        if constexpr (!MANY) break;
     }
 }
 
@@ -530,7 +555,7 @@ __device__ __forceinline__ int slot_size(int32_t c) { return (c & 0xffff) + ((c 
 // (One wave per query with a lane per slot took the general path for
 // nearly every query at nprobe = 16, and whenever there were fewer slots than
 // probes: 4 queries x 16 probes over 4,096 cells took 64 us for both launches,
-// 15 now; 4,096 queries over 12,288 cells 873, 328 now.)
+// 15 now; 4,096 queries over 12,288 cells 873, 298 now.)
 constexpr int MERGE_W = 4;
 constexpr int ME_MAX = CAPQ / MERGE_W;  // entries per thread, at most
 __global__ __launch_bounds__(64 * MERGE_W) void k_probe_merge(const uint64_t *__restrict__ ck,
@@ -676,6 +701,21 @@ st_status launch_prep(const float *x, int64_t n, int8_t *dig, int32_t *ex, doubl
     return ST_OK;
 }
 
+// Workgroups per slice that share its gy query groups (MANY): the number whose
+// rounds of 256 workgroups take the fewest steps, a workgroup's staging counted
+// as half a query group.
+int64_t group_walkers(int64_t S, int64_t gy) {
+    int64_t best = 1, best_t = INT64_MAX;
+    for (int64_t gw = 1; gw <= std::min<int64_t>(gy, 64); gw++) {
+        const int64_t t = cdiv(S * gw, 256) * (1 + 2 * cdiv(gy, gw));
+        if (t < best_t) {
+            best_t = t;
+            best = gw;
+        }
+    }
+    return best;
+}
+
 }  // namespace
 
 extern "C" int64_t st_knn_centroid_digit_bytes(int64_t nlist, int64_t d) {
@@ -731,19 +771,43 @@ extern "C" st_status st_knn_probe(const int8_t *digits, const int32_t *cexp, con
     chunk = chunk < QG ? QG : chunk / QG * QG;
     if (chunk > nq) chunk = cdiv(nq, QG) * QG;
     if (S * cdiv(chunk, QG) > INT32_MAX) return st::fail(ST_ERR_INVALID, "probe: too many centroids");
-    char *base = static_cast<char *>(st::scratch(st::SCRATCH_KNN, (size_t)(chunk * per_q), s));
+    // With more than one workgroup per CU, about one per CU that walks the query
+    // groups (MANY), whose digits lie behind the candidates.  Without room for
+    // them (an arena that may not grow during a capture), one group each.
+    bool many = ht == HT_MAX && S * cdiv(chunk, QG) > 256;
+    const size_t part_bytes = (size_t)((chunk * per_q + 15) / 16 * 16);
+    const size_t digit_bytes = (size_t)chunk * (TILE_BYTES / TILE + sizeof(int32_t));
+    char *base = static_cast<char *>(st::scratch(st::SCRATCH_KNN, part_bytes + (many ? digit_bytes : 0), s));
+    if (!base && many) {
+        many = false;
+        st::clear_error();
+        base = static_cast<char *>(st::scratch(st::SCRATCH_KNN, part_bytes, s));
+    }
     if (!base) return st::scratch_status();
-    // [candidate keys][candidate ids][counts]
+    // [candidate keys][candidate ids][counts][query digits][query exponents]
     uint64_t *ck = reinterpret_cast<uint64_t *>(base);
     int32_t *ci = reinterpret_cast<int32_t *>(ck + chunk * S * CAPQ);
     int32_t *pcnt = ci + chunk * S * CAPQ;
+    int8_t *qdig = many ? reinterpret_cast<int8_t *>(base + part_bytes) : nullptr;
+    int32_t *qexp = many ? reinterpret_cast<int32_t *>(qdig + chunk * (TILE_BYTES / TILE)) : nullptr;
 
-    auto part = ht == 1 ? k_probe_part<1> : ht == 2 ? k_probe_part<2> : ht == 3 ? k_probe_part<3> : k_probe_part<HT_MAX>;
+    auto part = ht == 1   ? k_probe_part<1, false>
+                : ht == 2 ? k_probe_part<2, false>
+                : ht == 3 ? k_probe_part<3, false>
+                : many    ? k_probe_part<HT_MAX, true>
+                          : k_probe_part<HT_MAX, false>;
     for (int64_t q0 = 0; q0 < nq; q0 += chunk) {
         const int64_t nqc = nq - q0 < chunk ? nq - q0 : chunk;
         const int64_t gy = cdiv(nqc, QG);
-        hipLaunchKernelGGL(part, dim3((unsigned)(S * gy)), dim3(PART_T), 0, s, queries + q0 * D, (int32_t)nqc, digits,
-                           cexp, cnorm, (int32_t)nlist, (int32_t)S, (int32_t)gy, (int32_t)nprobe, ck, ci, pcnt);
+        int64_t gw = gy;
+        if (many) {
+            const st_status r = launch_prep(queries + q0 * D, nqc, qdig, qexp, nullptr, s);
+            if (r != ST_OK) return r;
+            gw = group_walkers(S, gy);
+        }
+        hipLaunchKernelGGL(part, dim3((unsigned)(S * gw)), dim3(PART_T), 0, s, queries + q0 * D, qdig, qexp,
+                           (int32_t)gw, (int32_t)nqc, digits, cexp, cnorm, (int32_t)nlist, (int32_t)S, (int32_t)gy,
+                           (int32_t)nprobe, ck, ci, pcnt);
         ST_LAUNCH_CHECK();
         hipLaunchKernelGGL(k_probe_merge, dim3((unsigned)nqc), dim3(64 * MERGE_W), 0, s, ck, ci, pcnt, (int32_t)S,
                            (int32_t)nprobe, probes + q0 * nprobe);

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import oracle
+import scratchtape_amd as st
 from scratchtape_amd import knn
 
 pytestmark = pytest.mark.gpu
@@ -55,6 +56,46 @@ def test_probe_slices_and_merge_layouts(dev, nlist, nq):
     for nprobe in (1, 7, 16):
         _, got = run_probe(dev, cent, queries, nprobe)
         np.testing.assert_array_equal(got, oracle.knn_probe(cent, queries, nprobe))
+
+
+# More (slice, query group) pairs than CUs: workgroups that walk several query groups, with last groups and tiles of
+# one query, groups that do not divide among them, and 65 slices (the merge's general path).
+@pytest.mark.parametrize("nlist,nq", [(1000, 2753), (4100, 777), (12288, 321), (12480, 330)])
+def test_probe_workgroups_walk_query_groups(dev, nlist, nq):
+    rng = np.random.default_rng(nlist + nq)
+    cent = rng.standard_normal((nlist, D)).astype(np.float32)
+    cent[nlist // 2:nlist // 2 + 80] = cent[0]  # crowded slots: more than 64 equal candidates
+    queries = rng.standard_normal((nq, D)).astype(np.float32)
+    queries[0] = queries[nq - 1] = cent[0]
+    queries[nq // 2] = 0.0
+    for nprobe in (8, 16):
+        _, got = run_probe(dev, cent, queries, nprobe)
+        np.testing.assert_array_equal(got, oracle.knn_probe(cent, queries, nprobe))
+
+
+def test_captured_probe_without_room_for_the_query_digits(dev):
+    # 2,624 queries of 6 slices leave an arena of 1.25 x 2,624 x 4,632 bytes: room for the candidates of 3,008 queries
+    # (more than 256 pairs) but not for their digits, which a capture may not grow the arena for.
+    st.lib().st_scratch_release()
+    g = torch.Generator(device=dev).manual_seed(9)
+    c = knn.Centroids(torch.randn((1000, D), generator=g, device=dev))
+    queries = torch.randn((3008, D), generator=g, device=dev)
+    c.probe(queries[:2624].contiguous(), 8)
+    out = torch.empty((3008, 8), dtype=torch.int32, device=dev)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        c.probe(queries, 8, out=out)
+    want = c.probe(queries, 8)  # grows the arena
+    for _ in range(3):
+        out.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert torch.equal(c.probe(queries, 8), want)
+    del graph
+    torch.cuda.synchronize()
+    st.lib().st_scratch_release()
 
 
 def test_probe_edge_cases(dev):
