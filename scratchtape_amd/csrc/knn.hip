@@ -101,23 +101,30 @@ __global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ keys
     quantize_row([&](int i) { return k[i]; }, d, codes + r * (d / 4), scales + r);
 }
 
-// Rows of up to QD_MAX columns (d % 16 == 0) from 16-byte aligned keys: one wave per QR keys.
+// Rows of up to QD_MAX columns (d % 16 == 0) from 16-byte aligned keys: a
+// workgroup of four waves per 64 keys.
 //
-// Bound by HBM (4 d + d/4 + 4 bytes per key).  The thread-per-key form below
-// touches 64 rows per load instruction and reads every key twice; here a wave
-// reads its QR rows once as one contiguous run of 16-byte loads (lane l of
-// load i holds float4 64 i + l of the run), all in flight together, and keeps
-// them in registers.  The sum of squares is the contract's serial f32 sum over
-// a row, so the run also goes through LDS (rows padded by 4 floats: the 16
-// rows' 16-byte reads start 4 banks apart and cover all 64 banks) and lane r
-// sums row r in index order.  The codes need no division per component:
-// x / scale + 1.5 and the two roundings are monotone in x, so each code step
-// is a threshold on x (quantize_steps), found once per row.
-// 2^20 keys x 256: 4,635 us before, 245 us now (4.7 TB/s; a 1 GiB copy on this
-// card moves 5.1 TB/s).  16 rows per wave leaves room for nine
-// waves per CU (16.6 KB of LDS each).
-constexpr int QR = 16;       // keys per wave
-constexpr int QD_MAX = 256;  // widest row held in registers (QR * QD_MAX / 256 float4 per lane)
+// Bound by HBM (4 d + d/4 + 4 bytes per key) once the instructions per key are
+// few.  Each wave reads 16 rows as one contiguous run of 16-byte loads (lane l
+// of load i holds float4 64 i + l of the run), all in flight together, and
+// keeps them in registers.  The sum of squares is the contract's serial f32 sum
+// over a row, so the rows also go through LDS, 128 columns at a time (rows
+// padded by 4 floats: 16 rows' 16-byte reads cover all 64 banks), and one wave
+// sums all 64 rows, lane r row r in index order: a wave of 16 keys on its own
+// issues as many instructions for its sums with a quarter of the lanes, and
+// that form was bound by its 3,000 instructions per 16 keys.  2^20 keys, us, a
+// thread per key, a wave per 16 keys and now: x 256 4,635, 260, 192 (6.0 TB/s);
+// x 128 147 -> 97; x 64 101 -> 46.  The codes need no division per component: x / scale + 1.5 and the
+// two roundings are monotone in x, so each code step is a threshold on x
+// (quantize_step3), found once per row.  Widths of 64, 128 and 256 know at
+// compile time which row a load belongs to; the 34 KB of LDS leave room for
+// four workgroups per CU.
+constexpr int QR = 16;             // keys per wave
+constexpr int QW = 4;              // waves per workgroup
+constexpr int QK = QR * QW;        // keys per workgroup, one lane each for the sums
+constexpr int QD_MAX = 256;        // widest row held in registers (QR * QD_MAX / 256 float4 per lane)
+constexpr int QC = 128;            // columns in LDS at a time
+static_assert(QK == 64, "one wave sums a workgroup's rows");
 
 // Smallest x with code >= 1, >= 2, >= 3 for a finite scale s >= 1e-30: with
 // q = fl(x / s) and y = fl(q + 1.5), round-half-away(y) >= 1, 2, 3 iff y >=
@@ -135,51 +142,67 @@ __device__ __forceinline__ float quantize_step3(float s) {
     return t;
 }
 
-__global__ __launch_bounds__(64) void k_quantize_rows(const float *__restrict__ keys, int64_t n, int32_t d,
-                                                      uint8_t *__restrict__ codes, float *__restrict__ scales) {
-    constexpr int NL = QR * QD_MAX / 256;  // loads per lane at the widest row
-    __shared__ __attribute__((aligned(16))) float rowbuf[QR * (QD_MAX + 4)];
-    __shared__ float s_scale[QR], s_t3[QR];
+// DW: d / 64, or 0 for any other width.
+template <int DW>
+__global__ __launch_bounds__(64 * QW, 4) void k_quantize_rows(const float *__restrict__ keys, int64_t n, int32_t d,
+                                                              uint8_t *__restrict__ codes,
+                                                              float *__restrict__ scales) {
+    constexpr int NL = DW ? QR * DW / 4 : QR * QD_MAX / 256;  // loads per lane at the widest row
+    constexpr int PITCH = (DW == 1 ? 64 : QC) + 4;
+    __shared__ __attribute__((aligned(16))) float rowbuf[QK * PITCH];
+    __shared__ float2 s_row[QK];  // scale and third step
+    __shared__ int s_inf;         // whether some scale is infinite
     typedef float f4 __attribute__((ext_vector_type(4)));
-    const int lane = threadIdx.x;
-    const int64_t r0 = (int64_t)blockIdx.x * QR;
-    const int nr = (int)min((int64_t)QR, n - r0);  // keys of this wave
-    const int q4 = d >> 2;                         // float4 per row
-    const int inv = (65535 + q4) / q4;             // e / q4 = e inv >> 16 for e < 1024, q4 <= 64
-    const int total = nr * q4;                     // float4 of the run
-    const f4 *src = reinterpret_cast<const f4 *>(keys + r0 * d);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t k0 = (int64_t)blockIdx.x * QK, r0 = k0 + QR * w;
+    const int nr = (int)max((int64_t)0, min((int64_t)QR, n - r0));  // keys of this wave
+    const int q4 = DW ? 16 * DW : d >> 2;                           // float4 per row
+    const int inv = (65535 + q4) / q4;                              // e / q4 = e inv >> 16 for e < 1024, q4 <= 64
+    const int total = nr * q4;                                      // float4 of the wave's run
+    auto row_of = [&](int i) { return DW ? i * 4 / (DW ? DW : 1) + lane / q4 : (64 * i + lane) * inv >> 16; };
+    // Lanes past the run repeat its last float4 (without a run, one of the last key).
+    const f4 *src = reinterpret_cast<const f4 *>(keys + min(r0, n - 1) * (DW ? 64 * DW : d));
+    const int last = max(total, 1) - 1;
     f4 x[NL];
 #pragma unroll
     for (int i = 0; i < NL; i++)
-        if (64 * i < total) {  // uniform; the last load's lanes past the run repeat its last float4
-            const int e = 64 * i + lane;
-            x[i] = __builtin_nontemporal_load(src + (e < total ? e : total - 1));
-        }
-    const int pitch = d + 4;
+        if (DW || 64 * i < QR * q4) x[i] = __builtin_nontemporal_load(src + min(64 * i + lane, last));
+    // The sums are taken by another wave from workgroup to workgroup, so that no SIMD has them all.
+    const bool sums = w == ((int)(blockIdx.x >> 3) & (QW - 1));
+    float ss = 0.f;
 #pragma unroll
-    for (int i = 0; i < NL; i++)
-        if (64 * i < total) {
-            const int e = 64 * i + lane;
-            const int r = e * inv >> 16, c = e - r * q4;
-            if (e < total) *reinterpret_cast<f4 *>(rowbuf + r * pitch + 4 * c) = x[i];
-        }
-    __syncthreads();
-    if (lane < nr) {
-        const f4 *row = reinterpret_cast<const f4 *>(rowbuf + lane * pitch);
-        float ss = 0.f;
+    for (int c0 = 0; c0 < (DW ? 16 * DW : QD_MAX / 4); c0 += QC / 4) {  // in float4
+        if (!DW && c0 >= q4) break;
+        if (c0 > 0) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NL; i++)
+            if (DW || 64 * i < QR * q4) {
+                const int r = row_of(i), c = 64 * i + lane - r * q4 - c0;
+                if (r < QR && c >= 0 && c < QC / 4)
+                    *reinterpret_cast<f4 *>(rowbuf + (QR * w + r) * PITCH + 4 * c) = x[i];
+            }
+        __syncthreads();
+        if (sums) {
+            const f4 *row = reinterpret_cast<const f4 *>(rowbuf + lane * PITCH);
+            const int cols = min(QC / 4, q4 - c0);
 #pragma unroll 4
-        for (int c = 0; c < q4; c++) {
-            const f4 v = row[c];
-            ss += v.x * v.x;
-            ss += v.y * v.y;
-            ss += v.z * v.z;
-            ss += v.w * v.w;
+            for (int c = 0; c < cols; c++) {
+                const f4 v = row[c];
+                ss += v.x * v.x;
+                ss += v.y * v.y;
+                ss += v.z * v.z;
+                ss += v.w * v.w;
+            }
         }
+    }
+    if (sums) {
         float scale = 0.9957f * sqrtf(ss / (float)d);
         if (!(scale >= 1e-30f)) scale = 1e-30f;
-        s_scale[lane] = scale;
-        s_t3[lane] = quantize_step3(scale);
-        scales[r0 + lane] = scale;
+        const float t3 = quantize_step3(scale);
+        s_row[lane] = make_float2(scale, t3);
+        if (k0 + lane < n) scales[k0 + lane] = scale;
+        const bool inf = __ballot(t3 > 3.4028235e38f) != 0;
+        if (lane == 0) s_inf = inf;
     }
     __syncthreads();
     // Each float4 is one byte of codes; the quad's four bytes make a dword, and
@@ -187,34 +210,39 @@ __global__ __launch_bounds__(64) void k_quantize_rows(const float *__restrict__ 
     // loads' codes at once.
     uint32_t *dst = reinterpret_cast<uint32_t *>(codes + r0 * (d / 4));
     const int sub = lane & 3;
+    auto encode = [&](auto any_inf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int t = 0; t < NL; t += 4) {
-        uint32_t keep = 0;
+        for (int t = 0; t < NL; t += 4) {
+            uint32_t keep = 0;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int i = t + j;
-            if (64 * i < total) {  // uniform
-                const int e = min(64 * i + lane, total - 1);
-                const int r = e * inv >> 16;
-                const float s = s_scale[r], t3 = s_t3[r], t1 = -s, t2 = -s * 0x1p-24f;
-                uint32_t b = 0;
+            for (int j = 0; j < 4; j++) {
+                const int i = t + j;
+                if (DW || 64 * i < QR * q4) {
+                    const float2 row = s_row[QR * w + min(row_of(i), QR - 1)];
+                    const float t1 = -row.x, t2 = -row.x * 0x1p-24f, t3 = row.y;
+                    uint32_t b = 0;
 #pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const float v = x[i][c];
-                    uint32_t u = (uint32_t)(v >= t1) + (uint32_t)(v >= t2) + (uint32_t)(v >= t3);
-                    // An infinite scale (the sum overflowed): x / scale is 0 for a finite x, NaN otherwise.
-                    if (t3 > 3.4028235e38f) u = fabsf(v) <= 3.4028235e38f ? 2u : 0u;
-                    b |= u << (2 * c);
+                    for (int c = 3; c >= 0; c--) {
+                        const float v = x[i][c];
+                        uint32_t u = (uint32_t)(v >= t1) + (uint32_t)(v >= t2) + (uint32_t)(v >= t3);
+                        // An infinite scale (the sum overflowed): x / scale is 0 for a finite x, NaN otherwise.
+                        if (any_inf.value && t3 > 3.4028235e38f) u = fabsf(v) <= 3.4028235e38f ? 2u : 0u;
+                        b = 4 * b + u;
+                    }
+                    uint32_t word = b << (8 * sub);
+                    word |= st::xor_lane(word, 1, lane);
+                    word |= st::xor_lane(word, 2, lane);
+                    if (sub == j) keep = word;
                 }
-                uint32_t w = b << (8 * sub);
-                w |= st::xor_lane(w, 1, lane);
-                w |= st::xor_lane(w, 2, lane);
-                if (sub == j) keep = w;
             }
+            const int e0 = 64 * (t + sub) + (lane & ~3);  // first float4 of this lane's dword
+            if (e0 < total) dst[e0 >> 2] = keep;
         }
-        const int e0 = 64 * (t + sub) + (lane & ~3);  // first float4 of this lane's dword
-        if (e0 < total) dst[e0 >> 2] = keep;
-    }
+    };
+    if (s_inf)
+        encode(std::true_type());
+    else
+        encode(std::false_type());
 }
 
 // The reference's stored per-key norm (knn.rs:216): sum over the dims, in
@@ -1357,8 +1385,12 @@ extern "C" st_status st_knn_quantize_2bit(const float *keys, int64_t n, int64_t 
     if (n == 0) return ST_OK;
     if (!st::device_ok()) return ST_ERR_NO_DEVICE;
     // Wider rows, and keys that are not 16-byte aligned, take a thread per key.
-    if (d <= QD_MAX && (reinterpret_cast<uintptr_t>(keys) & 15) == 0 && cdiv(n, QR) <= INT32_MAX)
-        hipLaunchKernelGGL(k_quantize_rows, dim3((unsigned)cdiv(n, QR)), dim3(64), 0, st::stream_of(stream), keys, n,
+    auto rows = d == 64    ? k_quantize_rows<1>
+                : d == 128 ? k_quantize_rows<2>
+                : d == 256 ? k_quantize_rows<4>
+                           : k_quantize_rows<0>;
+    if (d <= QD_MAX && (reinterpret_cast<uintptr_t>(keys) & 15) == 0 && cdiv(n, QK) <= UINT32_MAX / (64 * QW))
+        hipLaunchKernelGGL(rows, dim3((unsigned)cdiv(n, QK)), dim3(64 * QW), 0, st::stream_of(stream), keys, n,
                            (int32_t)d, codes, scales);
     else
         hipLaunchKernelGGL(k_quantize, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, st::stream_of(stream), keys, n,

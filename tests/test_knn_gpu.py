@@ -15,7 +15,7 @@ D = 256
 @pytest.mark.parametrize("d", [16, 48, 64, 208, 256, 272])
 @pytest.mark.parametrize("n", [1, 15, 16, 17, 1003])
 def test_quantizer_widths_and_tails(dev, n, d):
-    """The wave-per-16-keys form (d <= 256, aligned keys) at its edges, bit for bit against the oracle and against the
+    """The workgroup-per-64-keys form (d <= 256, aligned keys) at its edges, bit for bit against the oracle and against the
     thread-per-key form (keys that start 4 bytes off)."""
     rng = np.random.default_rng(1000 * d + n)
     keys = (rng.standard_normal((n, d)) * 2.0 ** rng.integers(-40, 40, (n, 1))).astype(np.float32)
@@ -36,6 +36,21 @@ def test_quantizer_widths_and_tails(dev, n, d):
     b = knn.quantize_2bit(buf[1:].view(n, d))
     assert torch.equal(a[0], b[0])
     assert torch.equal(a[1].view(torch.int32), b[1].view(torch.int32))
+
+
+# Workgroups of 64 keys, four waves of 16: last ones of each size, widths with a form of their own and without, rows of
+# more than one 128-column stage.  A row whose sum overflows has an infinite scale (codes 2, 0 for NaN).
+@pytest.mark.parametrize("d", [64, 80, 128, 144, 256])
+@pytest.mark.parametrize("n", [33, 63, 64, 65, 129])
+def test_quantizer_workgroup_tails(dev, n, d):
+    rng = np.random.default_rng(2000 * d + n)
+    keys = (rng.standard_normal((n, d)) * 2.0 ** rng.integers(-40, 40, (n, 1))).astype(np.float32)
+    keys[n - 1] = 3e38
+    codes, scales = knn.quantize_2bit(torch.from_numpy(keys).to(dev))
+    wc, ws = oracle.quantize_2bit(keys, d)
+    assert np.isinf(ws[n - 1])
+    np.testing.assert_array_equal(codes.cpu().numpy(), wc)
+    np.testing.assert_array_equal(scales.cpu().numpy(), ws)
 
 
 def test_quantizer_is_bit_exact(dev):
