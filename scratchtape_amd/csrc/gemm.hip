@@ -291,11 +291,21 @@ __global__ __launch_bounds__(THREADS) void k_gemm(GemmArgs g) {
     SB sb[2];
     sb[0].zero_cs();
     sb[1].zero_cs();
-    f32x4 acc[FM][FN];
+    // f32 sums of the smaller tiles run in NA chains (every NA-th group of k),
+    // added at the end.  plan_tiles splits small products less than a slice per
+    // CU would, and longer sums err more: a step's products at 284 tokens x 320
+    // wide, against 64 bits, 2.3e-7 in the earlier splits, 3.2e-7 in one chain
+    // each, 1.7e-7 now, in the same time (260, 150 and 152 us for the 15).
+    constexpr int NA = F16 || FM * FN > 4 ? 1 : FM * FN > 1 ? 2 : 4;
+    f32x4 acc[FM][FN], more[NA > 1 ? NA - 1 : 1][FM][FN];
 #pragma unroll
     for (int i = 0; i < FM; i++)
 #pragma unroll
-        for (int j = 0; j < FN; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < FN; j++) {
+            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < NA - 1; c++) more[c][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
 
     // The partial k-stage comes first (k1 of k), so that every later one is
     // whole.
@@ -363,8 +373,12 @@ __global__ __launch_bounds__(THREADS) void k_gemm(GemmArgs g) {
 #pragma unroll
                     for (int i = 0; i < FM; i++)
 #pragma unroll
-                        for (int j = 0; j < FN; j++)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i][s], bf[j][s], acc[i][j], 0, 0, 0);
+                        for (int j = 0; j < FN; j++) {
+                            constexpr int PER_KC = NA == 4 ? 2 : 1;
+                            const int c = (kc * PER_KC + s % PER_KC) % NA;
+                            f32x4 &sum = c == 0 ? acc[i][j] : more[c > 0 ? c - 1 : 0][i][j];
+                            sum = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i][s], bf[j][s], sum, 0, 0, 0);
+                        }
             }
         }
     };
@@ -386,6 +400,13 @@ __global__ __launch_bounds__(THREADS) void k_gemm(GemmArgs g) {
         __syncthreads();
     }
     if (nst & 1) multiply(0);
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) {
+            if constexpr (NA == 2) acc[i][j] += more[0][i][j];
+            if constexpr (NA == 4) acc[i][j] = (acc[i][j] + more[0][i][j]) + (more[1][i][j] + more[NA - 2][i][j]);
+        }
     __syncthreads();
 
     // Column sums of this slice of B (tile row 0 only), reduced in slot order.

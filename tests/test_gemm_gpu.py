@@ -482,3 +482,17 @@ def test_grouped_step_set_with_tape_epilogues(dev):
     err, cs_err = bench.check_epilogue_set(ss)
     assert err <= 1e-5, err
     assert cs_err <= 1e-4, cs_err
+
+
+@pytest.mark.parametrize("m,k,n", [(284, 1280, 320), (150, 256, 64), (333, 1003, 999)])
+def test_any_shape_f32_sums_err_no_more_than_their_chains(dev, m, k, n):
+    """f32 products of the any-shape kernel against 64 bits.  A sum of L roundings of partial sums that grow as sqrt(i)
+    errs by about u sqrt(L / 2) of its size, u = 2^-24 / sqrt(3); the kernel adds 4 products at a time in at least two
+    chains, so L <= k / 8, doubled here for the products' own roundings and the final adds."""
+    g = torch.Generator(device="cpu").manual_seed(m + k + n)
+    a, b = torch.randn(m, k, generator=g).to(dev), torch.randn(k, n, generator=g).to(dev)
+    out = torch.zeros(m, n, device=dev)
+    st.matmul_f32(st.MatRef(a), st.MatRef(b), st.MatRef(out), 1, m, k, n)
+    want = a.double() @ b.double()
+    err = ((out.double() - want).norm() / want.norm()).item()
+    assert err <= 2.0 ** -24 / 3 ** 0.5 * (2 * (k / 8) / 2) ** 0.5
