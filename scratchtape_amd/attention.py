@@ -42,15 +42,25 @@ class AttnBuffers:
                            z(b * t * 3 * d))
 
 
+def _share(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether the two contiguous float32 tensors have memory in common."""
+    p, q = a.data_ptr(), b.data_ptr()
+    return p < q + 4 * b.numel() and q < p + 4 * a.numel()
+
+
 def _f32_step(qkv, dctx, buf: AttnBuffers, b: int, h: int, t: int, hd: int, use_f16: bool) -> bool:
     """Whether st_attention_fwd / _bwd take the step: its products all run in f32 (the six have one f16 rule: t % 64 ==
-    0 and hd % 32 == 0), the sizes fit, and the buffers hold the whole problems."""
+    0 and hd % 32 == 0), the sizes fit, the buffers hold the whole problems, and none shares memory in a way that only
+    the separate launches' order allows: ctx written over the scores, or dS over P or dctx (st_attention_bwd reads both
+    for dV after it has written dS; the separate launches make dV first)."""
     if (use_f16 and f16_route(t, hd, t)) or b < 1 or h < 1 or not _lib.lib().st_attention_fits(t, hd):
         return False
     n, tokens = b * h * t * t, b * t * h * hd
     sizes = [(qkv, 3 * tokens), (buf.s, n), (buf.p, n), (buf.ctx, tokens)] if dctx is None else \
         [(qkv, 3 * tokens), (dctx, tokens), (buf.p, n), (buf.dp, n), (buf.ds, n), (buf.dqkv, 3 * tokens)]
-    return all(x.numel() >= least for x, least in sizes)
+    if not all(x.numel() >= least for x, least in sizes):
+        return False
+    return not (_share(buf.s, buf.ctx) if dctx is None else _share(buf.ds, buf.p) or _share(buf.ds, dctx))
 
 
 def forward(qkv: torch.Tensor, buf: AttnBuffers, b: int, h: int, t: int, hd: int, use_f16: bool,

@@ -208,3 +208,23 @@ def test_packed_arguments_have_the_struct_layout(monkeypatch):
         mm._pack(mm._REF, *a.with_(off=1.5)._fields())
     with pytest.raises(TypeError):
         a.with_(offset=1)
+
+
+def test_f32_attention_step_leaves_shared_buffers_to_the_separate_launches():
+    """Buffers that may share memory under the separate launches' order (dS over P or dctx, ctx over the scores) are not
+    taken by st_attention_fwd / _bwd, whose order differs; buffers side by side in one allocation are."""
+    torch = pytest.importorskip("torch")
+    from scratchtape_amd import attention
+    b, h, t, hd = 1, 2, 16, 16
+    n = b * h * t * t  # == b * t * h * hd
+    qkv, dctx = torch.zeros(3 * n), torch.zeros(n)
+    step = lambda buf, d: attention._f32_step(qkv, d, buf, b, h, t, hd, False)
+    one = torch.zeros(5 * n)
+    part = lambda i: one[i * n:(i + 1) * n]
+    make = lambda **kw: attention.AttnBuffers(**{**dict(s=part(0), p=part(1), ctx=part(2), dp=part(3), ds=part(4),
+                                                        dqkv=torch.zeros(3 * n)), **kw})
+    assert step(make(), None) and step(make(), dctx)
+    assert step(make(s=part(1)), None) and step(make(dp=part(4)), dctx)  # in place: each element by one thread
+    assert not step(make(ctx=part(0)), None)
+    assert not step(make(ds=part(1)), dctx) and not step(make(ds=one[n + n // 2:2 * n + n // 2]), dctx)
+    assert not step(make(ds=dctx), dctx)

@@ -208,3 +208,26 @@ def test_f32_step_keeps_infinities_and_nans_where_the_separate_launches_have_the
             fine = np.isfinite(y)
             np.testing.assert_array_equal(np.isfinite(x), fine, err_msg=f"{name} {part} {row} {value}")
             assert np.max(np.abs(x[fine] - y[fine]), initial=0.0) <= 2e-4 * max(np.max(np.abs(y[fine]), initial=0.0), 1.0), name
+
+
+@pytest.mark.parametrize("which", ["ds is p", "ds is dctx", "ctx is s"])
+def test_f32_step_with_buffers_that_the_separate_launches_let_share_memory(dev, which):
+    """Buffers reused once the separate launches are done with them: dS in P's or dctx's memory, ctx in the scores'."""
+    b, h, t, hd = 2, 2, 64, 64  # (t == hd: dctx, ctx and the T x T buffers have one size)
+    g = torch.Generator(device="cpu").manual_seed(12)
+    qkv = torch.randn(b * t * 3 * h * hd, generator=g).to(dev)
+    dctx = torch.randn(b * t * h * hd, generator=g).to(dev)
+    want = attention.AttnBuffers.empty(b, h, t, hd, dev)
+    attention.step(qkv, dctx, want, b, h, t, hd, False)
+    buf = attention.AttnBuffers.empty(b, h, t, hd, dev)
+    if which == "ds is p":
+        buf.ds = buf.p
+    elif which == "ds is dctx":
+        dctx = buf.ds = dctx.clone()
+    else:
+        buf.ctx = buf.s
+    attention.step(qkv, dctx, buf, b, h, t, hd, False)
+    # Two orders of the same f32 sums (the bounds of the tests above, both sides off by as much).
+    for name, tol in (("ctx", 2e-5), ("dqkv", 2e-4)):
+        x, y = getattr(buf, name), getattr(want, name)
+        assert ((x - y).abs().max() / y.abs().max()).item() <= tol, name
