@@ -63,11 +63,44 @@ def _f32_step(qkv, dctx, buf: AttnBuffers, b: int, h: int, t: int, hd: int, use_
     return not (_share(buf.s, buf.ctx) if dctx is None else _share(buf.ds, buf.p) or _share(buf.ds, dctx))
 
 
+def _f32_step_pays(b: int, h: int, t: int, hd: int) -> bool:
+    """Whether st_attention_fwd / _bwd are faster than the separate launches, forward and backward timed in HIP graphs
+    for 1 to 384 problems x T = 8 to 512 x head widths of 16 to 128 (us, separate / one-launch, forward + backward):
+
+    - Head widths above 80 (compiled as 128), and above 64 off 4, run separately: 96 x 128 x 96 77 / 94, 96 x 448 x 96
+      410 / 1108, 96 x 256 x 128 198 / 204, 96 x 512 x 128 594 / 778; 96 x 100 x 128 is the exception (91 / 75).
+    - A workgroup holds 32 x T scores and a 64-row tile in LDS; with one workgroup per CU (over 80 KB) nothing hides its
+      chain of steps: 96 x 512 x 64 423 / 500, against 320 / 312 at T = 448.
+    - Widths off 4 are loaded element by element, and widths off 16 pad the 80-wide form: separate from T = 257 on (48 x
+      350 x 30 139 / 171, 64 x 288 x 72 178 / 194), as the 64-wide form with its T from 128 on.
+    - Narrow heads pay for any T up to 128 (4 x 128 x 32 32 / 28) and from 16 problems on (8 x 256 x 32 38 / 41, 16 x 256
+      x 32 47 / 42); widths up to 16 always (8 x 192 x 16 51 / 37), except where k_gemm_dma's 16 x 16 tiles take T x T x
+      T products (4 x 256 x 16 34 / 45).
+    - Otherwise a launch needs its workgroups: 128 of them (16 x 224 x 80 60 / 61, 24 x 224 x 80 67 / 62, 32 x 128 x 80 51 /
+      44, 8 x 256 x 80 49 / 63), or 192 where the products tile and run on the LDS-DMA kernel (16 x 256 x 64 47 / 55, 24 x
+      256 x 64 62 / 56, 96 x 128 x 64 67 / 51) or the width is padded.  Short sequences off 32 pay from one problem on
+      (1 x 50 x 64 33 / 27)."""
+    if hd > 80 or (hd > 64 and hd % 4):
+        return False
+    width = 32 if hd <= 32 and hd % 4 == 0 else 64 if hd <= 64 else 80
+    if 128 * ((t + 15) // 16 * 16 + 4) + 256 * (width + 4) > 80 << 10:  # bytes of LDS per workgroup
+        return False
+    padded = hd > 64 and hd % 16 != 0
+    if (hd % 4 or padded) and t > 256:
+        return False
+    if hd <= 32:
+        return t <= 128 or b * h >= 16 or (hd <= 16 and hd % 4 == 0 and t % 256 != 0)
+    if hd <= 64 and hd % 4 == 0 and t <= 112 and t % 32:
+        return True
+    tiled = t % 32 == 0 and hd % 32 == 0
+    return b * h * ((t + 31) // 32) >= (192 if tiled or padded else 128)
+
+
 def forward(qkv: torch.Tensor, buf: AttnBuffers, b: int, h: int, t: int, hd: int, use_f16: bool,
             stream=None) -> None:
     d = h * hd
     batch, scale = b * h, hd ** -0.5
-    if _f32_step(qkv, None, buf, b, h, t, hd, use_f16):
+    if _f32_step_pays(b, h, t, hd) and _f32_step(qkv, None, buf, b, h, t, hd, use_f16):
         _lib.call("st_attention_fwd", _ptr(qkv), _ptr(buf.s), _ptr(buf.p), _ptr(buf.ctx), b, h, t, hd, scale,
                   _stream(stream))
         return
@@ -84,7 +117,7 @@ def backward(qkv: torch.Tensor, dctx: torch.Tensor, buf: AttnBuffers, b: int, h:
     """dV = Pᵀ dO, dP = dO Vᵀ, dS = softmax backward, dQ = dS K, dK = dSᵀ Q, written into buf.dqkv."""
     d = h * hd
     batch, scale = b * h, hd ** -0.5
-    if _f32_step(qkv, dctx, buf, b, h, t, hd, use_f16):
+    if _f32_step_pays(b, h, t, hd) and _f32_step(qkv, dctx, buf, b, h, t, hd, use_f16):
         _lib.call("st_attention_bwd", _ptr(qkv), _ptr(dctx), _ptr(buf.p), _ptr(buf.dp), _ptr(buf.ds), _ptr(buf.dqkv), b,
                   h, t, hd, scale, _stream(stream))
         return

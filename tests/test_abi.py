@@ -228,3 +228,17 @@ def test_f32_attention_step_leaves_shared_buffers_to_the_separate_launches():
     assert not step(make(ctx=part(0)), None)
     assert not step(make(ds=part(1)), dctx) and not step(make(ds=one[n + n // 2:2 * n + n // 2]), dctx)
     assert not step(make(ds=dctx), dctx)
+
+
+# (b h, T, head width): one-launch forms measured faster (True) or slower (False) than the separate launches.
+@pytest.mark.parametrize("bh,t,hd,pays", [
+    (96, 200, 80, True), (128, 128, 64, True), (384, 448, 64, True), (24, 256, 64, True), (16, 256, 64, False),
+    (4, 256, 64, False), (96, 512, 64, False), (96, 500, 48, False), (96, 512, 32, True), (4, 128, 32, True),
+    (8, 256, 32, False), (8, 192, 16, True), (4, 256, 16, False), (96, 448, 80, True), (96, 480, 80, False),
+    (8, 256, 80, False), (64, 288, 72, False), (48, 350, 30, False), (96, 128, 96, False), (96, 448, 96, False),
+    (4, 64, 128, False), (96, 384, 128, False), (96, 160, 66, False), (1, 50, 64, True)])
+def test_f32_attention_takes_the_faster_launches(bh, t, hd, pays):
+    from scratchtape_amd import attention
+    assert attention._f32_step_pays(bh, 1, t, hd) is pays
+    if bh % 4 == 0:
+        assert attention._f32_step_pays(bh // 4, 4, t, hd) is pays

@@ -158,8 +158,7 @@ def f32_step(dev, b, h, t, hd, qkv, dctx, separate, monkeypatch):
     for x in (buf.s, buf.p, buf.ctx, buf.dp, buf.ds, buf.dqkv):
         x.fill_(7.0)
     with monkeypatch.context() as m:
-        if separate:
-            m.setattr(attention, "_f32_step", lambda *a: False)
+        m.setattr(attention, "_f32_step_pays", lambda *a: not separate)
         attention.step(qkv, dctx, buf, b, h, t, hd, False)
     return [x.cpu().double().numpy() for x in (buf.s, buf.p, buf.ctx, buf.dp, buf.ds, buf.dqkv)]
 
@@ -211,8 +210,9 @@ def test_f32_step_keeps_infinities_and_nans_where_the_separate_launches_have_the
 
 
 @pytest.mark.parametrize("which", ["ds is p", "ds is dctx", "ctx is s"])
-def test_f32_step_with_buffers_that_the_separate_launches_let_share_memory(dev, which):
+def test_f32_step_with_buffers_that_the_separate_launches_let_share_memory(dev, which, monkeypatch):
     """Buffers reused once the separate launches are done with them: dS in P's or dctx's memory, ctx in the scores'."""
+    monkeypatch.setattr(attention, "_f32_step_pays", lambda *a: True)
     b, h, t, hd = 2, 2, 64, 64  # (t == hd: dctx, ctx and the T x T buffers have one size)
     g = torch.Generator(device="cpu").manual_seed(12)
     qkv = torch.randn(b * t * 3 * h * hd, generator=g).to(dev)
