@@ -103,6 +103,15 @@ st_status st_matmul_with(const st_matref *a, const st_matref *b, const st_matref
                          int64_t batch, int64_t m, int64_t k, int64_t n, const st_epilogue *epi,
                          int32_t use_f16, st_stream stream);
 
+/* No reference counterpart; for tests and tuning.  What st_matmul_with
+ * launches for a call, found on the host without a device: plan[0] the kernel
+ * (0 any shape and alignment, 1 LDS-DMA tiles, 2 the grouped launch's 256 x 128
+ * tiles), for kernel 0 its tile's rows plan[1] and columns plan[2] and its
+ * slices of k plan[3], and plan[4] the bytes of split-k scratch. */
+st_status st_matmul_plan(const st_matref *a, const st_matref *b, const st_matref *out,
+                         int64_t batch, int64_t m, int64_t k, int64_t n, const st_epilogue *epi,
+                         int32_t use_f16, int64_t *plan);
+
 /* One GEMM of st_matmul_grouped: the arguments of st_matmul_with (an
  * all-zero epi is no epilogue). */
 typedef struct st_gemm {

@@ -150,6 +150,20 @@ extern "C" {
         use_f16: i32,
         stream: st_stream,
     ) -> st_status;
+    /// No reference counterpart: what `st_matmul_with` launches for a call (kernel, tile, slices, scratch), found
+    /// without a device.
+    pub fn st_matmul_plan(
+        a: *const st_matref,
+        b: *const st_matref,
+        out: *const st_matref,
+        batch: i64,
+        m: i64,
+        k: i64,
+        n: i64,
+        epi: *const st_epilogue,
+        use_f16: i32,
+        plan: *mut i64,
+    ) -> st_status;
     /// Independent GEMMs the reference issues back to back (`src/gpu_step/tape.rs:324-347`) as one
     /// submission; no GEMM may read or write memory another one writes.
     pub fn st_matmul_grouped(gemms: *const st_gemm, count: i64, stream: st_stream) -> st_status;

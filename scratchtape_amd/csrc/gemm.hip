@@ -647,20 +647,33 @@ TileCfg plan_tiles(bool f16, bool ta, bool tb, const st_epilogue &epi, const st_
     return best;
 }
 
+// What gemm_impl launches for a call that it accepts and that has work to do.
+enum { PLAN_ANY_SHAPE = 0, PLAN_DMA = 1, PLAN_GROUP = 2 };
+
+struct CallPlan {
+    int kernel;
+    TileCfg tc;  // any-shape kernel
+    size_t scratch;
+};
+
+CallPlan plan_call(const st_matref *a, const st_matref *b, const st_matref *out, int64_t batch, int64_t m, int64_t k,
+                   int64_t n, const st_epilogue &epi, bool use_f16) {
+    const bool f16 = f16_route(use_f16, epi, b, m, k, n);
+    const st::DmaGemm d = make_dma(a, b, out, batch, m, k, n, epi, f16);
+    if (st::group_of_one(d)) return {PLAN_GROUP, {}, st::gemm_group_scratch(&d, 1, f16, true)};
+    if (st::gemm_dma_takes(d)) return {PLAN_DMA, {}, st::gemm_dma_scratch(d)};
+    const TileCfg tc = plan_tiles(f16, a->trans, b->trans, epi, out, batch, m, k, n);
+    if (tc.splits <= 1) return {PLAN_ANY_SHAPE, tc, 0};
+    return {PLAN_ANY_SHAPE, tc, sizeof(float) * (size_t)(batch * tc.splits * (m * n + (epi.has_col_sum ? n : 0)))};
+}
+
 // Bytes of split-k scratch gemm_impl would request for these arguments (0
 // when it would request none or refuse them).
 size_t gemm_impl_scratch(const st_matref *a, const st_matref *b, const st_matref *out, int64_t batch, int64_t m,
                          int64_t k, int64_t n, const st_epilogue &epi, bool use_f16) {
     if (!a || !b || !out || !a->p || !b->p || !out->p || out->trans || batch <= 0 || m <= 0 || n <= 0 || k <= 0)
         return 0;
-    const bool f16 = f16_route(use_f16, epi, b, m, k, n);
-    const st::DmaGemm d = make_dma(a, b, out, batch, m, k, n, epi, f16);
-    if (st::group_of_one(d)) return st::gemm_group_scratch(&d, 1, f16, true);
-    size_t dma = 0;
-    if ((dma = st::gemm_dma_scratch(d)) || st::gemm_dma_takes(d)) return dma;
-    const int64_t splits = plan_tiles(f16, a->trans, b->trans, epi, out, batch, m, k, n).splits;
-    if (splits <= 1) return 0;
-    return sizeof(float) * (size_t)(batch * splits * m * n + (epi.has_col_sum ? batch * splits * n : 0));
+    return plan_call(a, b, out, batch, m, k, n, epi, use_f16).scratch;
 }
 
 st_status gemm_impl(const st_matref *a, const st_matref *b, const st_matref *out, int64_t batch, int64_t m,
@@ -783,6 +796,29 @@ extern "C" st_status st_matmul_with(const st_matref *a, const st_matref *b, cons
                                     int64_t batch, int64_t m, int64_t k, int64_t n, const st_epilogue *epi,
                                     int32_t use_f16, st_stream stream) {
     return gemm_impl(a, b, out, batch, m, k, n, epi, use_f16 != 0, st::stream_of(stream));
+}
+
+extern "C" st_status st_matmul_plan(const st_matref *a, const st_matref *b, const st_matref *out, int64_t batch,
+                                    int64_t m, int64_t k, int64_t n, const st_epilogue *epi_in, int32_t use_f16,
+                                    int64_t *plan) {
+    st::clear_error();
+    if (!plan) return st::fail(ST_ERR_INVALID, "plan is NULL");
+    const st_status s = check_call(a, b, out, batch, m, k, n);
+    if (s) return s;
+    st_epilogue epi;
+    std::memset(&epi, 0, sizeof epi);
+    if (epi_in) epi = *epi_in;
+    std::memset(plan, 0, 5 * sizeof *plan);
+    if (batch == 0 || m == 0 || n == 0) return ST_OK;
+    const CallPlan c = plan_call(a, b, out, batch, m, k, n, epi, use_f16 != 0);
+    plan[0] = c.kernel;
+    if (c.kernel == PLAN_ANY_SHAPE) {
+        plan[1] = c.tc.bm;
+        plan[2] = c.tc.bn;
+        plan[3] = c.tc.splits;
+    }
+    plan[4] = (int64_t)c.scratch;
+    return ST_OK;
 }
 
 extern "C" st_status st_matmul_grouped(const st_gemm *gemms, int64_t count, st_stream stream) {

@@ -7,6 +7,7 @@ ScratchtapeError with the message the reference would panic with.
 """
 from __future__ import annotations
 
+import ctypes
 import struct
 from dataclasses import dataclass
 from typing import Optional, Tuple
@@ -138,6 +139,19 @@ def matmul_with(a: MatRef, b: MatRef, out: MatRef, batch: int, m: int, k: int, n
                 epi: Optional[Epilogue], use_f16: bool, stream=None) -> None:
     """`matmul` with the f16 route chosen by the caller (matmul.rs:106)."""
     _call("st_matmul_with", a, b, out, batch, m, k, n, epi, int(bool(use_f16)), stream=stream)
+
+
+def matmul_plan(a: MatRef, b: MatRef, out: MatRef, batch: int, m: int, k: int, n: int, epi: Optional[Epilogue],
+                use_f16: bool) -> Tuple[int, int, int, int, int]:
+    """What matmul_with launches for these arguments (st_matmul_plan; no reference counterpart): the kernel (0 any
+    shape, 1 LDS-DMA tiles, 2 grouped 256 x 128 tiles), kernel 0's tile rows and columns and slices of k, and the bytes
+    of split-k scratch."""
+    plan = (ctypes.c_int64 * 5)()
+    _lib.check(_lib.packed("st_matmul_plan")(_pack(_REF, *a._fields()), _pack(_REF, *b._fields()),
+                                             _pack(_REF, *out._fields()), batch, m, k, n,
+                                             _pack(_EPI, *(epi._fields() if epi else _NO_EPI)), int(bool(use_f16)),
+                                             ctypes.addressof(plan)))
+    return tuple(plan)
 
 
 def matmul_grouped(calls, stream=None, noalloc: bool = False) -> None:

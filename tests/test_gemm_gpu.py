@@ -267,10 +267,13 @@ def tape_forms(dev, m, k, n, use_f16, seed):
 
 # The any-shape kernel around its tile edges (32, 64 and 128 rows and columns, k-stages of 32 and 64): last tiles
 # moved back to the edge, fewer rows or columns than a tile, a partial first k-stage; odd offsets and strides.  The
-# last f32 shapes are large enough for 128-row tiles, the last f16 ones for each tile.
+# last shapes of each route are large enough for its larger tiles (TILES; the others take 32 x 32 in some form).
 EDGE_F32 = [(1, 1, 1), (3, 5, 2), (31, 2, 33), (32, 31, 32), (33, 32, 31), (64, 33, 63), (65, 64, 64), (127, 65, 32),
-            (33, 1, 129), (200, 80, 200), (97, 300, 4), (1, 257, 130), (2500, 33, 2300), (1300, 3, 700)]
-EDGE_F16 = [(64, 32, 32), (64, 96, 160), (192, 64, 96), (320, 160, 1056), (4096, 32, 1056), (6400, 64, 1120)]
+            (33, 1, 129), (200, 80, 200), (97, 300, 4), (1, 257, 130), (2500, 33, 2300), (1300, 3, 700), (6401, 100, 259), (2305, 100, 3075)]
+EDGE_F16 = [(64, 32, 32), (64, 96, 160), (192, 64, 96), (320, 160, 1056), (4096, 32, 1056), (6400, 64, 1120),
+            (256, 96, 3104)]
+TILES = {(6401, 100, 259): (64, 64), (2305, 100, 3075): (128, 128), (4096, 32, 1056): (128, 64),
+         (6400, 64, 1120): (128, 64), (256, 96, 3104): (64, 64)}
 
 
 @pytest.mark.parametrize("route,shape", [(False, s) for s in EDGE_F32] + [(True, s) for s in EDGE_F16])
@@ -279,7 +282,12 @@ def test_any_shape_kernel_at_tile_edges(dev, route, shape):
     batch = 2 if m * n < 10000 else 1
     for i, (ta, tb) in enumerate([(False, False), (False, True), (True, False), (True, True)]):
         epi = (True, i % 2 == 0, True, True, True) if i < 3 else (False, False, False, False, True)
-        run_case(dev, 300 + 2 * i, (batch, m, k, n, ta, tb) + epi, route)
+        with oracle.threads(8):
+            p = prep_case(dev, 300 + 2 * i, (batch, m, k, n, ta, tb) + epi, route)
+        kernel, *tile = st.matmul_plan(*p["call"])[:3]
+        assert kernel == 0 and (tuple(tile) == TILES.get(shape, tuple(tile)) or p["f16"] != route), (shape, tile)
+        st.matmul_with(*p["call"])
+        check_case(p)
 
 
 @pytest.mark.parametrize("use_f16", [False, True])

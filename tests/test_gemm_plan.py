@@ -1,0 +1,42 @@
+"""Which kernel, tile and split a GEMM call takes (st_matmul_plan), on the CPU: the dispatch that the GPU tests' shapes
+rely on, seen from outside the kernels."""
+import ctypes
+
+import pytest
+
+from scratchtape_amd import _lib
+from test_gemm_gpu import EDGE_F16, EDGE_F32, TILES
+
+ANY_SHAPE, DMA, GROUP = 0, 1, 2
+FORMS = [(False, False), (False, True), (True, False), (True, True)]
+
+
+def plan(m, k, n, use_f16=False, ta=False, tb=False, batch=1, aligned=True, bias=False, accumulate=False, col_sum=False):
+    """(kernel, tile rows, tile columns, slices, scratch bytes) of a call on packed matrices."""
+    p = (1 << 20) + (0 if aligned else 4)
+    ref = lambda trans, size: _lib.StMatRef(p, 0, size, int(trans), 0, 0, 1, 0)
+    epi = _lib.StEpilogue()
+    epi.bias, epi.accumulate, epi.has_col_sum = p if bias else None, int(accumulate), int(col_sum)
+    out = (ctypes.c_int64 * 5)()
+    _lib.check(_lib.lib().st_matmul_plan(ref(ta, m * k), ref(tb, k * n), ref(False, m * n), batch, m, k, n, epi,
+                                         int(use_f16), out))
+    return tuple(out)
+
+
+@pytest.mark.parametrize("use_f16", [False, True])
+def test_the_edge_shapes_reach_every_tile(use_f16):
+    for ta, tb in FORMS:
+        tiles = {}
+        for shape in EDGE_F16 if use_f16 else EDGE_F32:
+            kernel, *tile = plan(*shape, use_f16, ta, tb, aligned=False, bias=True)[:3]
+            assert kernel == ANY_SHAPE and tuple(tile) == TILES.get(shape, tuple(tile)), (shape, ta, tb)
+            tiles[tuple(tile)] = shape
+        assert set(tiles) >= {(32, 32), (64, 64), (128, 64) if use_f16 else (128, 128)}, (ta, tb, tiles)
+
+
+def test_a_plan_needs_valid_arguments_and_no_device():
+    L, out = _lib.lib(), (ctypes.c_int64 * 5)(*[9] * 5)
+    ref = _lib.StMatRef(1 << 20, 0, 0, 0, 0, 0, 1, 0)
+    assert L.st_matmul_plan(ref, ref, ref, 1, 8, 8, 8, None, 0, None) == _lib.ST_ERR_INVALID
+    assert L.st_matmul_plan(ref, ref, None, 1, 8, 8, 8, None, 0, out) == _lib.ST_ERR_INVALID
+    assert L.st_matmul_plan(ref, ref, ref, 0, 8, 8, 8, None, 0, out) == 0 and list(out) == [0] * 5
