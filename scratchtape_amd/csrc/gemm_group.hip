@@ -1376,20 +1376,38 @@ size_t gemm_group_scratch(const DmaGemm *items, int count, bool f16, bool tall) 
 }
 
 // The grouped kernels' 256 x 128 tiles read the operands 1.5 times less than
-// gemm_dma's 128 x 128 and (f16) round each element once, but a CU gets few
-// units.  As single calls, gemm_dma against a group of one, us: f16 with 128
-// tiles 4096 x 256 x 1024 16.6 / 13.8, 16384 x 256 x 256 16.2 / 12.8; 512 tiles
-// 8192 x 512 x 2048 73.7 / 43.0; 2,048 tiles 16384 x 1024 x 4096 486 / 246; 64
-// tiles 4096 x 2048 x 512 33.8 / 43.2; 32 tiles 4096 x 256 x 256 8.5 / 12.7.  f32
-// with 256 tiles 8192 x 256 x 1024 53.0 / 44.7; 128 tiles 30.5 / 31.4.  Split
-// products by tiles x k-stages: 8 x 128 19.4 / 22.0 (f16) and 31.9 / 35.8 (f32),
-// 8 x 256 29.8 / 23.5 and 52.3 / 49.0, 128 x 512 710 / 330.
+// gemm_dma's 128 x 128 and (f16) round each element once, but a launch of few
+// units leaves CUs idle: up to 128 tall tiles gemm_dma's twice as many give
+// every CU at most one, from the next on they take a second round.  As single
+// calls in HIP graphs, gemm_dma / a group of one, us:
+//  - f16, 128 tiles: 4096 x 256 x 1024 12.9 / 13.3, masked 17.1 / 16.5, with bias
+//    and ReLU 16.7 / 15.4; 4096 x 1024 x 1024 masked 31.0 / 32.1, 16384 x 2048 x 256
+//    57 / 69 -- and a step that issues these layer by layer 161.3 / 168.9 (a group
+//    of one shares no CU with its neighbours).  132 tiles: 8448 x 256 x 512 21.7 /
+//    13.4; 256 and 512 tiles 1.2 to 1.9 times, 2,048 tiles 16384 x 1024 x 4096 486 /
+//    246.
+//  - f32, where a round of 256 tall tiles takes 139 us at k = 1024 and one of 256
+//    128 x 128 tiles 78, so that the rounds have to be nearly full: 256 tiles 156 /
+//    139 and 896 300 / 284, but 384 132 / 144 and 442 / 519, 640 198 / 206; products
+//    split into 576 units (1536 x 2048 x 1536) 123 / 129, into 864 (768 x 2048 x
+//    2304) 100 / 91.
+//  - Split products, by tiles x k-stages: f16 8 x 128 22.5 / 24.0, 8 x 256 33.6 / 28.9,
+//    64 x 32 32.5 / 31.6, 128 x 512 710 / 330.  f32 32 x 128 98 / 94, 128 x 64 175 / 161, but
+//    with shorter k 64 x 32 54.6 / 55.3, 128 x 32 90 / 99, 128 x 48 126 / 130.
 bool group_of_one(const DmaGemm &d) {
     if (!group_eligible(d) || !group_tall(d)) return false;
-    const int64_t tiles = d.batch * (d.m / Tall::TM) * (d.n / TN);
-    const bool split = can_split(d) && tiles * (d.k / BK) >= 2048;
-    if (tiles < (d.f16 ? 128 : 256) && !split) return false;
-    return gemm_group_scratch(&d, 1, d.f16 != 0, true) == 0 || gemm_dma_scratch(d) != 0;
+    const int64_t tiles = d.batch * (d.m / Tall::TM) * (d.n / TN), stages = d.k / BK;
+    const bool split = can_split(d) && tiles * stages >= (d.ta ? 2048 : 4096) && (d.f16 || stages >= 64);
+    if (tiles < (d.f16 ? 129 : 256) && !split) return false;
+    std::vector<int64_t> splits, slice_k;
+    if (d.f16) {
+        group_splits(&d, 1, Tall::TM, r16::Tall16::NS, r16::Tall16::FAIR_PART, group_cus(), splits, slice_k);
+    } else {
+        group_splits(&d, 1, Tall::TM, Tall::NS, Tall::FAIR_PART, group_cus(), splits, slice_k);
+        const int64_t units = tiles * splits[0];
+        if ((double)units < 0.84 * 256 * (double)cdiv(units, 256)) return false;
+    }
+    return splits[0] == 1 || gemm_dma_scratch(d) != 0;
 }
 
 st_status gemm_group(const DmaGemm *items, int count, bool f16, bool tall, hipStream_t stream) {

@@ -435,19 +435,27 @@ def test_grouped_random_groups_match_oracle(dev):
             check_case(p)
 
 
-# Single calls large enough for the grouped kernel's 256 x 128 tiles: 128 (f16) or 256 (f32) tiles with every
-# epilogue term, one fewer row of tiles (which are not), batches, and a product split over k with column sums.
-@pytest.mark.parametrize("case,use_f16", [
-    ((1, 2048, 128, 2048, False, False, True, True, True, True, True), True),
-    ((1, 1792, 128, 2048, False, True, True, False, False, False, False), True),
-    ((2, 1024, 160, 2048, True, True, False, False, False, True, False), True),
-    ((1, 4096, 128, 2048, False, True, True, True, True, True, True), False),
-    ((1, 3840, 128, 2048, True, False, False, False, False, False, True), False),
-    ((1, 512, 8192, 512, True, False, False, False, False, False, True), True),
-    ((1, 512, 8192, 512, True, False, False, False, False, False, True), False)])
-def test_single_calls_on_the_grouped_kernel(dev, case, use_f16):
+# Single calls around the sizes from which the grouped kernel's 256 x 128 tiles take them (kernel 2): more than 128 tiles
+# (f16) or 256 (f32, but not 257 to 384) with every epilogue term, batches, and a product split over k with column
+# sums; calls just below stay on the LDS-DMA kernel (1).  (Column sums of a transposed b put an f16 call on the f32
+# route.)
+@pytest.mark.parametrize("case,use_f16,kernel", [
+    ((1, 2048, 128, 2048, False, False, True, True, True, True, True), True, 1),
+    ((1, 2048, 128, 2176, False, False, True, True, True, True, True), True, 2),
+    ((1, 1792, 128, 2048, False, True, True, False, False, False, False), True, 1),
+    ((2, 1024, 160, 2048, True, True, False, False, False, True, False), True, 1),
+    ((3, 1024, 160, 1408, True, False, False, False, False, True, False), True, 2),
+    ((1, 4096, 128, 2048, False, True, True, True, True, True, True), False, 2),
+    ((1, 3840, 128, 2048, True, False, False, False, False, False, True), False, 1),
+    ((1, 4096, 128, 2176, False, True, True, False, True, False, True), False, 1),
+    ((1, 512, 8192, 512, True, False, False, False, False, False, True), True, 2),
+    ((1, 512, 8192, 512, True, False, False, False, False, False, True), False, 2)])
+def test_single_calls_on_the_grouped_kernel(dev, case, use_f16, kernel):
     with oracle.threads(8):
-        run_case(dev, 900, case, use_f16, aligned16=True, packed=True)
+        p = prep_case(dev, 900, case, use_f16, aligned16=True, packed=True)
+    assert st.matmul_plan(*p["call"])[0] == kernel
+    st.matmul_with(*p["call"])
+    check_case(p)
 
 
 @pytest.mark.parametrize("use_f16", [False, True])

@@ -34,6 +34,22 @@ def test_the_edge_shapes_reach_every_tile(use_f16):
         assert set(tiles) >= {(32, 32), (64, 64), (128, 64) if use_f16 else (128, 128)}, (ta, tb, tiles)
 
 
+# Single calls on either side of the grouped kernel's rule, at the sizes whose two times decided it (see group_of_one).
+@pytest.mark.parametrize("m,k,n,use_f16,form,kernel", [
+    (4096, 256, 1024, True, "nn", DMA), (4096, 256, 1024, True, "plain", DMA), (4096, 1024, 1024, True, "nt", DMA),
+    (16384, 2048, 256, True, "nn", DMA), (8448, 256, 512, True, "plain", GROUP), (8448, 256, 512, True, "nn", GROUP),
+    (16384, 1024, 4096, True, "nt", GROUP), (8192, 256, 1024, False, "nn", GROUP), (8192, 2048, 384, False, "nn", DMA),
+    (16384, 256, 768, False, "nt", DMA), (24576, 512, 512, False, "nn", DMA), (40960, 512, 512, False, "nn", DMA),
+    (57344, 512, 512, False, "nn", GROUP), (8192, 512, 2048, False, "nt", GROUP), (256, 4096, 1024, True, "tn", DMA),
+    (256, 8192, 1024, True, "tn", GROUP), (1024, 1024, 4096, False, "tn", DMA), (1024, 2048, 4096, False, "tn", GROUP),
+    (1024, 4096, 1024, False, "tn", GROUP), (1536, 2048, 1536, False, "tn", DMA), (1536, 4096, 1536, False, "tn", DMA),
+    (768, 2048, 2304, False, "tn", GROUP), (2048, 2048, 512, True, "plain", DMA), (2048, 2048, 512, True, "tn", GROUP),
+    (2048, 2048, 1024, True, "plain", GROUP)])
+def test_single_calls_take_the_faster_kernel(m, k, n, use_f16, form, kernel):
+    kw = dict(tn=dict(ta=True, accumulate=True, col_sum=True), nt=dict(tb=True, bias=True), nn=dict(bias=True), plain={})
+    assert plan(m, k, n, use_f16, **kw[form])[0] == kernel
+
+
 def test_a_plan_needs_valid_arguments_and_no_device():
     L, out = _lib.lib(), (ctypes.c_int64 * 5)(*[9] * 5)
     ref = _lib.StMatRef(1 << 20, 0, 0, 0, 0, 0, 1, 0)
