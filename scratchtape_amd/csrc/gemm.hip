@@ -625,23 +625,44 @@ TileCfg plan_tiles(bool f16, bool ta, bool tb, const st_epilogue &epi, const st_
         const int64_t part = (int64_t)sizeof(float) * batch * (m * n + (epi.has_col_sum ? n : 0));
         most = std::max<int64_t>(1, std::min<int64_t>(std::max(cdiv(cus, tiles64), (8 << 20) / part), k / (4 * BK)));
     }
-    TileCfg best = {32, 32, 1, std::max<int64_t>(1, cdiv(k, BK)) * BK};
+    const int64_t S = std::max<int64_t>(1, cdiv(k, BK));  // k-stages
+    TileCfg best = {32, 32, 1, S * BK};
     double best_t = -1;
     for (const Cand &c : cands) {
         if (c.bm > 32 && (m < c.bm || n < c.bn)) continue;  // (see WHOLE)
         const int64_t tiles = batch * cdiv(m, c.bm) * cdiv(n, c.bn);
-        for (int64_t sp = 1; sp <= most; sp++) {
-            const int64_t slice = std::max<int64_t>(1, cdiv(cdiv(k, sp), BK)) * BK;
-            const int64_t splits = std::max<int64_t>(1, cdiv(k, slice));
-            if (splits != sp) continue;
-            const double stages = (double)(slice / BK), w = (double)cdiv(tiles * splits, cus);
-            const double per_wg = stages + (f16 ? c.lead16 : c.lead);
-            double t = per_wg * std::max(f16 ? c.alone16 : c.alone, w * (f16 ? c.shared16 : c.shared));
-            if (splits > 1) t += 3.0 + 8.0 * (double)(splits * batch * m * n) / 4e6;
-            if (best_t < 0 || t < best_t) {
-                best_t = t;
-                best = {c.bm, c.bn, splits, slice};
+        const double alone = f16 ? c.alone16 : c.alone, shared = f16 ? c.shared16 : c.shared;
+        const double lead = f16 ? c.lead16 : c.lead;
+        auto time = [&](int64_t sp, int64_t stages) {
+            double t = ((double)stages + lead) * std::max(alone, (double)cdiv(tiles * sp, cus) * shared);
+            if (sp > 1) t += 3.0 + 8.0 * (double)(sp * batch * m * n) / 4e6;
+            return t;
+        };
+        int64_t c_sp = 1, c_stages = S;
+        double c_t = time(1, S);
+        // The best slice count without trying them all (k / 128 of them for a dot product): by rounds w of
+        // workgroups over the CUs.  No count in round w takes less than `shared` times all its stages and leads
+        // spread over the CUs, which grows with w; within a round more slices are shorter, and fewer save only
+        // partials, so the walk down from the most of them soon ends.
+        for (int64_t w = cdiv(2 * tiles, cus); most > 1; w++) {
+            if (shared * ((double)(S * tiles) / (double)cus + lead * (double)w) + 3.0 > c_t) break;
+            const int64_t lo = std::max<int64_t>(2, cus * (w - 1) / tiles + 1), hi = std::min(most, cus * w / tiles);
+            if (lo > most) break;
+            for (int64_t sp = hi; sp >= lo; sp--) {
+                const int64_t stages = cdiv(S, sp);
+                sp = cdiv(S, stages);  // the fewest slices of that length
+                if (sp < lo || ((double)stages + lead) * std::max(alone, (double)w * shared) + 3.0 > c_t) break;
+                const double t = time(sp, stages);
+                if (t < c_t || (t == c_t && sp < c_sp)) {
+                    c_t = t;
+                    c_sp = sp;
+                    c_stages = stages;
+                }
             }
+        }
+        if (best_t < 0 || c_t < best_t) {
+            best_t = c_t;
+            best = {c.bm, c.bn, c_sp, c_stages * BK};
         }
     }
     return best;

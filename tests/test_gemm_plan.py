@@ -1,6 +1,7 @@
 """Which kernel, tile and split a GEMM call takes (st_matmul_plan), on the CPU: the dispatch that the GPU tests' shapes
 rely on, seen from outside the kernels."""
 import ctypes
+import time
 
 import pytest
 
@@ -56,3 +57,18 @@ def test_a_plan_needs_valid_arguments_and_no_device():
     assert L.st_matmul_plan(ref, ref, ref, 1, 8, 8, 8, None, 0, None) == _lib.ST_ERR_INVALID
     assert L.st_matmul_plan(ref, ref, None, 1, 8, 8, 8, None, 0, out) == _lib.ST_ERR_INVALID
     assert L.st_matmul_plan(ref, ref, ref, 0, 8, 8, 8, None, 0, out) == 0 and list(out) == [0] * 5
+
+
+@pytest.mark.parametrize("m,k,n,slices", [(1, 1 << 20, 1, 512), (16, 1 << 20, 16, 512), (1, 1 << 24, 1, 512),
+                                          (4, 100000, 4, 447), (64, 65536, 64, 128), (1, 1 << 28, 1, 512)])
+def test_a_long_small_product_is_planned_in_microseconds(m, k, n, slices):
+    """A small output's slice count is found without walking every possible one (k / 128 of them).  Host time of the
+    whole query, ctypes included: about 4 us, which the bound leaves room for a busy machine; walking takes 60 us to
+    13 ms on the shapes of 2^20 and more."""
+    best = float("inf")
+    for _ in range(20):
+        t = time.perf_counter()
+        got = plan(m, k, n, aligned=False)
+        best = min(best, time.perf_counter() - t)
+    assert got[:4] == (ANY_SHAPE, 32, 32, slices)
+    assert best < 40e-6, best
