@@ -87,7 +87,8 @@ typedef struct st_epilogue {
  * (out->trans must be 0: "out is stored row-major", matmul.rs:107).  Runs
  * f16-in/f32-accumulate when st_f16_enabled() and the shape tiles
  * (k % 32 == 0, m % 64 == 0, n % 32 == 0, and not col_sum with b
- * transposed: matmul.rs:108-112, 524-534), else f32.  epi may be NULL. */
+ * transposed: matmul.rs:108-112, 524-534), else f32.  epi may be NULL.
+ * Shapes that do not tile take up to 8,388,480 rows (m) and 65,535 matrices. */
 st_status st_matmul(const st_matref *a, const st_matref *b, const st_matref *out, int64_t batch,
                     int64_t m, int64_t k, int64_t n, const st_epilogue *epi, st_stream stream);
 
@@ -107,7 +108,8 @@ st_status st_matmul_with(const st_matref *a, const st_matref *b, const st_matref
  * launches for a call, found on the host without a device: plan[0] the kernel
  * (0 any shape and alignment, 1 LDS-DMA tiles, 2 the grouped launch's 256 x 128
  * tiles), for kernel 0 its tile's rows plan[1] and columns plan[2] and its
- * slices of k plan[3], and plan[4] the bytes of split-k scratch. */
+ * slices of k plan[3], and plan[4] the bytes of split-k scratch.  A call that
+ * st_matmul_with would refuse is refused with the same error. */
 st_status st_matmul_plan(const st_matref *a, const st_matref *b, const st_matref *out,
                          int64_t batch, int64_t m, int64_t k, int64_t n, const st_epilogue *epi,
                          int32_t use_f16, int64_t *plan);

@@ -263,13 +263,14 @@ __global__ __launch_bounds__(THREADS) void k_gemm(GemmArgs g) {
     // Workgroups are dealt to the 8 XCDs round-robin by linear id; remap so
     // each XCD gets a contiguous run of tiles (columns fastest), which share A
     // rows (and k-slices) in that XCD's L2.
-    int64_t lin = blockIdx.x + (int64_t)gridDim.x * blockIdx.z;
-    const int64_t total = (int64_t)gridDim.x * gridDim.z;
+    const int64_t gxy = (int64_t)gridDim.x * gridDim.y, total = gxy * gridDim.z;
+    int64_t lin = blockIdx.x + (int64_t)gridDim.x * (blockIdx.y + (int64_t)gridDim.y * blockIdx.z);
     if (total % 8 == 0) lin = (lin % 8) * (total / 8) + lin / 8;
     const int nbx = (g.n + BN - 1) / BN;
-    const int64_t z = lin / gridDim.x;
-    const int tile = (int)(lin % gridDim.x);
+    const int64_t z = lin / gxy;
+    const int tile = (int)(lin % gxy);
     const int bx = tile % nbx, by = tile / nbx;
+    if (by * BM >= g.m) return;  // a grid of several rows may be larger than the tiles
     const int64_t zb = z / g.splits;
     const int slice = (int)(z % g.splits);
     // The tile's own rows and columns begin at row_own, col_own; the last tile
@@ -668,6 +669,22 @@ TileCfg plan_tiles(bool f16, bool ta, bool tb, const st_epilogue &epi, const st_
     return best;
 }
 
+// The limits of the any-shape kernel: its grid's, 31-bit tile numbers, and
+// the rows that it has always taken.
+constexpr int64_t ANY_SHAPE_ROWS = 65535 * 128;
+
+st_status check_any_shape(const TileCfg &tc, int64_t batch, int64_t m, int64_t n) {
+    if (batch * tc.splits > 65535)
+        return st::fail(ST_ERR_INVALID, "batch %lld too large for one launch", (long long)batch);
+    if (m > ANY_SHAPE_ROWS)
+        return st::fail(ST_ERR_INVALID, "m = %lld: the any-shape kernel takes at most %lld rows", (long long)m,
+                        (long long)ANY_SHAPE_ROWS);
+    if (cdiv(n, tc.bn) * cdiv(m, tc.bm) > INT32_MAX)
+        return st::fail(ST_ERR_INVALID, "m = %lld x n = %lld: too many tiles for one launch", (long long)m,
+                        (long long)n);
+    return ST_OK;
+}
+
 // What gemm_impl launches for a call that it accepts and that has work to do.
 enum { PLAN_ANY_SHAPE = 0, PLAN_DMA = 1, PLAN_GROUP = 2 };
 
@@ -726,8 +743,7 @@ st_status gemm_impl(const st_matref *a, const st_matref *b, const st_matref *out
 
     const TileCfg tc = plan_tiles(f16, a->trans, b->trans, epi, out, batch, m, k, n);
     const int64_t splits = tc.splits, slice_k = tc.slice_k;
-    if (batch * splits > 65535) return st::fail(ST_ERR_INVALID, "batch %lld too large for one launch", (long long)batch);
-    if (cdiv(m, 128) > 65535) return st::fail(ST_ERR_INVALID, "m = %lld too large for one launch", (long long)m);
+    if ((s = check_any_shape(tc, batch, m, n))) return s;
 
     GemmArgs g;
     std::memset(&g, 0, sizeof g);
@@ -775,9 +791,9 @@ st_status gemm_impl(const st_matref *a, const st_matref *b, const st_matref *out
     const bool whole = m >= tc.bm && n >= tc.bn;
     const KernelFn fn = f16 ? pick_kernel<64, true>(tc, a->trans, b->trans, whole)
                             : pick_kernel<32, false>(tc, a->trans, b->trans, whole);
-    const int64_t tiles = cdiv(n, tc.bn) * cdiv(m, tc.bm);
-    if (tiles > INT32_MAX / THREADS) return st::fail(ST_ERR_INVALID, "m = %lld too large for one launch", (long long)m);
-    dim3 grid((unsigned)tiles, 1, (unsigned)(batch * splits));
+    // Rows of 2^23 workgroups (a grid has fewer than 2^32 threads along x).
+    const int64_t tiles = cdiv(n, tc.bn) * cdiv(m, tc.bm), gx = std::min<int64_t>(tiles, 1 << 23);
+    dim3 grid((unsigned)gx, (unsigned)cdiv(tiles, gx), (unsigned)(batch * splits));
     hipLaunchKernelGGL(fn, grid, dim3(THREADS), 0, stream, g);
     ST_LAUNCH_CHECK();
 
@@ -834,6 +850,8 @@ extern "C" st_status st_matmul_plan(const st_matref *a, const st_matref *b, cons
     const CallPlan c = plan_call(a, b, out, batch, m, k, n, epi, use_f16 != 0);
     plan[0] = c.kernel;
     if (c.kernel == PLAN_ANY_SHAPE) {
+        const st_status r = check_any_shape(c.tc, batch, m, n);
+        if (r) return r;
         plan[1] = c.tc.bm;
         plan[2] = c.tc.bn;
         plan[3] = c.tc.splits;

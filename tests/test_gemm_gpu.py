@@ -512,3 +512,14 @@ def test_any_shape_f32_sums_err_no_more_than_their_chains(dev, m, k, n):
     want = a.double() @ b.double()
     err = ((out.double() - want).norm() / want.norm()).item()
     assert err <= 2.0 ** -24 / 3 ** 0.5 * (2 * (k / 8) / 2) ** 0.5
+
+
+def test_any_shape_grid_of_several_rows(dev):
+    """More 32 x 32 tiles than one row of the grid holds (2^23): 1 x 1 x 2^28 + 4,097 with the last columns ragged."""
+    n = (1 << 28) + 4097
+    a = torch.tensor([[3.0]], device=dev)
+    b = torch.arange(n, device=dev, dtype=torch.int32).remainder_(9973).float()
+    out = torch.full((n + 1,), -1.0, device=dev)
+    assert st.matmul_plan(st.MatRef(a), st.MatRef(b), st.MatRef(out), 1, 1, 1, n, None, False)[:3] == (0, 32, 32)
+    st.matmul_f32(st.MatRef(a), st.MatRef(b), st.MatRef(out), 1, 1, 1, n)
+    assert torch.equal(out[:n], 3.0 * b) and out[n].item() == -1.0

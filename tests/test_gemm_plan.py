@@ -72,3 +72,18 @@ def test_a_long_small_product_is_planned_in_microseconds(m, k, n, slices):
         best = min(best, time.perf_counter() - t)
     assert got[:4] == (ANY_SHAPE, 32, 32, slices)
     assert best < 40e-6, best
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 4, 300_000_000), (31, 1, (1 << 30) - 1), (100_000, 32, 100_000), (64, 1, 1 << 27),
+                                   (8_388_480, 3, 31)])
+def test_large_outputs_of_small_tiles_are_accepted(m, k, n):
+    """Up to 33 million 32 x 32 tiles, where the device holds the output."""
+    kernel, bm, bn = plan(m, k, n, aligned=False, bias=True)[:3]
+    assert (kernel, bm, bn) == (ANY_SHAPE, 32, 32) or bm > 32
+
+
+def test_what_the_any_shape_kernel_refuses():
+    for m, n, batch, msg in [(8_388_481, 3, 1, "8388480 rows"), (33, 5, 65536, "batch 65536"),
+                             (8_388_480, (1 << 30) - 1, 1, "m = 8388480 x n = 1073741823")]:
+        with pytest.raises(_lib.ScratchtapeError, match=msg):
+            plan(m, 5, n, batch=batch, aligned=False, bias=True)
