@@ -764,26 +764,36 @@ extern "C" st_status st_knn_probe(const int8_t *digits, const int32_t *cexp, con
             break;
         }
     }
-    // Queries in chunks (multiples of 64) whose candidate slots fit CAND_BUDGET.
-    const int64_t S = cdiv(ntiles, 2 * ht);
-    const int64_t per_q = S * CAPQ * (int64_t)(sizeof(uint64_t) + sizeof(int32_t)) + S * (int64_t)sizeof(int32_t);
-    int64_t chunk = CAND_BUDGET / per_q;
-    chunk = chunk < QG ? QG : chunk / QG * QG;
-    if (chunk > nq) chunk = cdiv(nq, QG) * QG;
-    if (S * cdiv(chunk, QG) > INT32_MAX) return st::fail(ST_ERR_INVALID, "probe: too many centroids");
     // With more than one workgroup per CU, about one per CU that walks the query
     // groups (MANY), whose digits lie behind the candidates.  Without room for
-    // them (an arena that may not grow during a capture), one group each.
-    bool many = ht == HT_MAX && S * cdiv(chunk, QG) > 256;
-    const size_t part_bytes = (size_t)((chunk * per_q + 15) / 16 * 16);
-    const size_t digit_bytes = (size_t)chunk * (TILE_BYTES / TILE + sizeof(int32_t));
-    char *base = static_cast<char *>(st::scratch(st::SCRATCH_KNN, part_bytes + (many ? digit_bytes : 0), s));
-    if (!base && many) {
-        many = false;
+    // what is wanted (an arena that may not grow during a capture; smaller
+    // slices need more room for the same queries), one group each and larger
+    // slices, whose results are the same.
+    bool many = ht == HT_MAX;
+    int64_t S, chunk, per_q;
+    size_t part_bytes;
+    char *base;
+    for (;;) {
+        // Queries in chunks (multiples of 64) whose candidate slots fit CAND_BUDGET.
+        S = cdiv(ntiles, 2 * ht);
+        per_q = S * CAPQ * (int64_t)(sizeof(uint64_t) + sizeof(int32_t)) + S * (int64_t)sizeof(int32_t);
+        chunk = CAND_BUDGET / per_q;
+        chunk = chunk < QG ? QG : chunk / QG * QG;
+        if (chunk > nq) chunk = cdiv(nq, QG) * QG;
+        if (S * cdiv(chunk, QG) > INT32_MAX) return st::fail(ST_ERR_INVALID, "probe: too many centroids");
+        many = many && S * cdiv(chunk, QG) > 256;
+        part_bytes = (size_t)((chunk * per_q + 15) / 16 * 16);
+        const size_t digit_bytes = (size_t)chunk * (TILE_BYTES / TILE + sizeof(int32_t));
         st::clear_error();
-        base = static_cast<char *>(st::scratch(st::SCRATCH_KNN, part_bytes, s));
+        base = static_cast<char *>(st::scratch(st::SCRATCH_KNN, part_bytes + (many ? digit_bytes : 0), s));
+        if (base) break;
+        if (many)
+            many = false;
+        else if (ht < HT_MAX)
+            ht = ht < 3 ? ht + 1 : HT_MAX;
+        else
+            return st::scratch_status();
     }
-    if (!base) return st::scratch_status();
     // [candidate keys][candidate ids][counts][query digits][query exponents]
     uint64_t *ck = reinterpret_cast<uint64_t *>(base);
     int32_t *ci = reinterpret_cast<int32_t *>(ck + chunk * S * CAPQ);

@@ -98,6 +98,31 @@ def test_captured_probe_without_room_for_the_query_digits(dev):
     st.lib().st_scratch_release()
 
 
+def test_captured_probe_of_fewer_queries_than_before(dev):
+    # 320 queries over 2,048 cells take 32 slices (320 x 32 x 772 bytes of candidates, and a quarter more of arena), 256
+    # queries 64 smaller ones (256 x 64 x 772), which a capture has no room for: they take larger slices instead.
+    st.lib().st_scratch_release()
+    g = torch.Generator(device=dev).manual_seed(10)
+    c = knn.Centroids(torch.randn((2048, D), generator=g, device=dev))
+    queries = torch.randn((320, D), generator=g, device=dev)
+    want = c.probe(queries, 16)
+    few = queries[:256].contiguous()
+    out = torch.empty((256, 16), dtype=torch.int32, device=dev)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        c.probe(few, 16, out=out)
+    for _ in range(3):
+        out.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[:256])
+        assert torch.equal(c.probe(few, 16), want[:256])  # eager: grows the arena the first time
+    del graph
+    torch.cuda.synchronize()
+    st.lib().st_scratch_release()
+
+
 def test_probe_edge_cases(dev):
     rng = np.random.default_rng(32)
     nlist = 200
