@@ -305,13 +305,14 @@ __global__ __launch_bounds__(256) void k_ln_fwd4(const float *__restrict__ x, in
 }
 
 // The backward's row pass.  grid (chunks of `rows_pc` rows per model, models),
-// rows_pc a multiple of LNV_ROWS; wave w takes rows w, w + 4, .. of its chunk:
-// dx as k_ln_bwd_dx, and each lane adds dy xhat and dy of its columns over the
-// wave's rows (in row order).
+// rows_pc a multiple of LNV_ROWS (ONE: LNV_ROWS itself, whose trips are unrolled:
+// 20,000 rows x 256 in 4 models 16.3 us without, 14.9 with); wave w takes rows w,
+// w + 4, .. of its chunk: dx as k_ln_bwd_dx, and each lane adds dy xhat and dy of
+// its columns over the wave's rows (in row order).
 // The four waves' sums are added in a fixed order into the chunk's partial,
 // part[(m nch + c) 2d + j], which k_ln_bwd_sum4 adds up.  dy and x are read
 // once for both gradients.
-template <int NV>
+template <int NV, bool ONE>
 __global__ __launch_bounds__(256) void k_ln_bwd4(const float *__restrict__ dy, const float *__restrict__ x,
                                                  const float *__restrict__ mean, const float *__restrict__ rstd,
                                                  int64_t d, int64_t rows_pm, const float *__restrict__ params,
@@ -335,8 +336,7 @@ __global__ __launch_bounds__(256) void k_ln_bwd4(const float *__restrict__ dy, c
     // RB rows' loads in flight together; a row past the chunk's end loads the
     // chunk's last row (always in bounds) and contributes nothing.
     constexpr int RB = NV >= 4 ? 2 : 4;
-    const int trips = (int)(rend - rbeg + 4 * RB - 1) / (4 * RB);
-    for (int t0 = 0; t0 < trips * RB; t0 += RB) {
+    auto trip = [&](int t0) __attribute__((always_inline)) {
         float4 dyv[RB][NV], xv[RB][NV];
         float mu[RB], rs[RB];
         bool live[RB];
@@ -404,6 +404,13 @@ __global__ __launch_bounds__(256) void k_ln_bwd4(const float *__restrict__ dy, c
                 pb[i].w += dv.w;
             }
         }
+    };
+    if constexpr (ONE) {
+#pragma unroll
+        for (int t0 = 0; t0 < LNV_ROWS / 4; t0 += RB) trip(t0);
+    } else {
+        const int trips = (int)(rend - rbeg + 4 * RB - 1) / (4 * RB);
+        for (int t0 = 0; t0 < trips * RB; t0 += RB) trip(t0);
     }
 #pragma unroll
     for (int i = 0; i < NV; i++) {
@@ -515,15 +522,26 @@ extern "C" st_status st_layer_norm_backward(const float *dy, const float *x, con
     // partials (2 d floats each) stay small beside the rows: at 65,536 x 768
     // k_ln_bwd_sum4 took 22.7 us over 4,096 chunks of 16 and takes 6.6 over 1,024
     // of 64 (forward and backward together 199 -> 187 us).
-    const int64_t rows_pc =
+    // Wide rows (d > 512), whose workgroups are few per CU for their LDS, take 16
+    // fewer where the chunks would leave a fifth of the CUs idle at the end:
+    // 17,000 x 640 31.1 -> 29.0 us, 50,000 x 1024 140 -> 134.
+    int64_t rows_pc =
         LNV_ROWS * std::max<int64_t>(1, (rows_pm + LNV_ROWS * LNV_CHUNKS - 1) / (LNV_ROWS * LNV_CHUNKS));
-    const int64_t vch = (rows_pm + rows_pc - 1) / rows_pc;
+    int64_t vch = (rows_pm + rows_pc - 1) / rows_pc;
+    if (d > 512 && rows_pc > LNV_ROWS && 5 * models * vch < 4 * 256 * ((models * vch + 255) / 256)) {
+        rows_pc -= LNV_ROWS;
+        vch = (rows_pm + rows_pc - 1) / rows_pc;
+    }
     if (ln_vec_ok(d, off, model_stride, {dy, x, params, dx}) && vch <= INT32_MAX && models <= 65535) {
         float *part = static_cast<float *>(
             st::scratch(st::SCRATCH_ROWS, (size_t)(models * vch * 2 * d) * sizeof(float), s));
         if (!part) return st::scratch_status();
         const int nv = (int)((d + 255) / 256);
-        auto k = nv == 1 ? k_ln_bwd4<1> : nv == 2 ? k_ln_bwd4<2> : nv == 3 ? k_ln_bwd4<3> : k_ln_bwd4<4>;
+        auto k = nv == 1 ? k_ln_bwd4<1, false> : nv == 2 ? k_ln_bwd4<2, false> : nv == 3 ? k_ln_bwd4<3, false>
+                                                                              : k_ln_bwd4<4, false>;
+        if (rows_pc == LNV_ROWS)
+            k = nv == 1 ? k_ln_bwd4<1, true> : nv == 2 ? k_ln_bwd4<2, true> : nv == 3 ? k_ln_bwd4<3, true>
+                                                                            : k_ln_bwd4<4, true>;
         hipLaunchKernelGGL(k, dim3((unsigned)vch, (unsigned)models), dim3(256), 0, s, dy, x, mean, rstd, d, rows_pm,
                            params, off, model_stride, dx, accumulate, part, (int32_t)vch, (int32_t)rows_pc);
         ST_LAUNCH_CHECK();

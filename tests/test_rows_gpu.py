@@ -81,8 +81,10 @@ def test_layer_norm_vector_forms(dev, nrows, d, off):
 
 
 # Above 16 x 1,024 rows per model a chunk takes 32 rows or more: the first such size, a last chunk of one row, three
-# register columns per lane, and two models of which each does.
-@pytest.mark.parametrize("nrows,d,models", [(16385, 8, 1), (33 * 1024 + 1, 36, 1), (17000, 516, 1), (2 * 16400, 12, 2)])
+# register columns per lane, and two models of which each does.  Wide rows take 16 fewer where the last round of chunks
+# would be mostly empty (17,000 x 516: 16 instead of 32; 38,001 x 1020: 32 instead of 48).
+@pytest.mark.parametrize("nrows,d,models", [(16385, 8, 1), (33 * 1024 + 1, 36, 1), (17000, 516, 1), (20500, 516, 1),
+                                            (38001, 1020, 1), (2 * 16400, 12, 2)])
 def test_layer_norm_vector_forms_with_longer_chunks(dev, nrows, d, models):
     run_case(dev, nrows, d, 4, models, seed=nrows)
 
