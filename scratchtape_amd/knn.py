@@ -118,10 +118,13 @@ def _check_out(out, nq: int, k: int, device) -> Tuple[torch.Tensor, torch.Tensor
 
 def _split_work(nq: int, device, stream) -> Tuple[Optional[torch.Tensor], int, int]:
     """Memory for a small batch's candidate lists (st_knn_split_bytes): the tensor (held by the caller until its launch
-    is enqueued), its address and its size.  It is an allocation of the current stream, which keeps it until the work
-    enqueued there is done, so a call on another stream gets none."""
+    is enqueued), its address and its size.  It is an allocation of the current stream of `device`, which keeps it until
+    the work enqueued there is done, so a call on another stream (or from another current device, whose stream the
+    launch goes to) gets none."""
     nbytes = int(_lib.lib().st_knn_split_bytes(nq))
-    if nbytes <= 0 or (stream is not None and _stream(stream) != _stream(None)):
+    if nbytes <= 0 or device.index != torch.cuda.current_device():
+        return None, 0, 0
+    if stream is not None and _stream(stream) != _stream(None):
         return None, 0, 0
     work = torch.empty(nbytes, dtype=torch.uint8, device=device)
     return work, work.data_ptr(), nbytes

@@ -242,3 +242,21 @@ def test_f32_attention_takes_the_faster_launches(bh, t, hd, pays):
     assert attention._f32_step_pays(bh, 1, t, hd) is pays
     if bh % 4 == 0:
         assert attention._f32_step_pays(bh // 4, 4, t, hd) is pays
+
+
+def test_split_work_belongs_to_the_launch_stream(monkeypatch):
+    """Memory for a split search is an allocation of the stream that the launch goes to, or is not given: not for a call
+    on another stream, nor for queries on another device than the current one (whose stream the launch uses)."""
+    torch = pytest.importorskip("torch")
+    import importlib
+    import types
+    knn = importlib.import_module("scratchtape_amd.knn")
+    monkeypatch.setattr(knn, "_stream", lambda s: 5 if s is None else s)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch, "empty", lambda n, **kw: types.SimpleNamespace(data_ptr=lambda: 64, n=n, **kw))
+    nbytes = scratchtape_amd.lib().st_knn_split_bytes(4)
+    here, there = torch.device("cuda", 0), torch.device("cuda", 1)
+    assert knn._split_work(4, here, None)[1:] == (64, nbytes) and knn._split_work(4, here, 5)[1:] == (64, nbytes)
+    assert knn._split_work(4, here, 6) == (None, 0, 0)
+    assert knn._split_work(4, there, None) == (None, 0, 0)
+    assert knn._split_work(300, here, None) == (None, 0, 0)
