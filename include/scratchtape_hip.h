@@ -88,7 +88,10 @@ typedef struct st_epilogue {
  * f16-in/f32-accumulate when st_f16_enabled() and the shape tiles
  * (k % 32 == 0, m % 64 == 0, n % 32 == 0, and not col_sum with b
  * transposed: matmul.rs:108-112, 524-534), else f32.  epi may be NULL.
- * Shapes that do not tile take up to 8,388,480 rows (m) and 65,535 matrices. */
+ * Shapes that do not tile take up to 8,388,480 rows (m) and 65,535 matrices.
+ * Large f16 products (more than 128 output tiles of 256 x 128, or long sums
+ * split over k; st_matmul_plan says kernel 2) run on the grouped launch's
+ * kernel, whose bounded waits st_sync checks. */
 st_status st_matmul(const st_matref *a, const st_matref *b, const st_matref *out, int64_t batch,
                     int64_t m, int64_t k, int64_t n, const st_epilogue *epi, st_stream stream);
 
@@ -398,14 +401,16 @@ st_status st_scratch_release(void);
  * device for slot waits of the grouped f16 GEMM kernel that gave up (each
  * wait is bounded so that the kernel always ends; a give-up means its
  * producer and consumer waves lost step, and the outputs of the grouped f16
- * GEMMs run since the last check are not valid): ST_ERR_HIP with a message
- * if there were any, and the count is cleared.  Reference failures surface
- * as panics (tensor.rs:253, gpu_step/matmul.rs:107). */
+ * GEMMs and the large single ones (see st_matmul) run since the last check are
+ * not valid): ST_ERR_HIP with a message if there were any, and the count is
+ * cleared.  A caller that synchronises the stream by other means has to call
+ * st_sync as well to hear of them.  Reference failures surface as panics
+ * (tensor.rs:253, gpu_step/matmul.rs:107). */
 st_status st_sync(st_stream stream);
 
 /* No reference counterpart; for tests of the check above.  Sets how many
- * times a slot wait of the grouped f16 GEMM kernel polls its counter before
- * it gives up, for launches enqueued afterwards (process-wide; a negative
+ * times a slot wait of the grouped f16 GEMM kernel (which large single f16
+ * products use too) polls its counter before it gives up, for launches enqueued afterwards (process-wide; a negative
  * value restores the default, 2^20). */
 st_status st_set_wait_limit(int64_t polls);
 

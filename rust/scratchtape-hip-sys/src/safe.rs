@@ -731,7 +731,8 @@ pub fn knn_search_masked_2bit<H: DeviceBuffer + ?Sized>(
     });
 }
 
-/// Waits for the calling thread's stream.
+/// Waits for the calling thread's stream, then panics if a bounded wait of the grouped f16 kernel (grouped
+/// calls and large single f16 products) gave up since the last check.
 pub fn sync() {
     check(unsafe { sys::st_sync(stream()) });
 }

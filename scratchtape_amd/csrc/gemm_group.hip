@@ -1362,8 +1362,8 @@ st_status check_group_waits() {
     const uint32_t zero = 0;
     ST_HIP_CHECK(hipMemcpy(p, &zero, sizeof zero, hipMemcpyHostToDevice));
     return fail(ST_ERR_HIP,
-                "grouped GEMM: %u slot wait(s) gave up after %u polls; the outputs of the grouped f16 GEMMs run "
-                "since the last st_sync are not valid",
+                "grouped f16 kernel: %u slot wait(s) gave up after %u polls; the outputs of the grouped and the large "
+                "single f16 GEMMs run since the last st_sync are not valid",
                 n, g_wait_polls.load(std::memory_order_relaxed));
 }
 

@@ -180,8 +180,9 @@ def f16_route(m: int, k: int, n: int, col_sum: bool = False, b_trans: bool = Fal
 
 
 def sync(stream=None) -> None:
-    """st_sync: waits for `stream`, then raises ScratchtapeError if a grouped f16 GEMM's bounded slot wait gave up
-    since the last check (its outputs are not valid)."""
+    """st_sync: waits for `stream`, then raises ScratchtapeError if a bounded slot wait of the grouped f16 kernel gave
+    up since the last check: the outputs of matmul_grouped's f16 GEMMs, and of single f16 calls that matmul_plan puts on
+    that kernel (2), are then not valid."""
     _lib.call("st_sync", _stream(stream))
 
 

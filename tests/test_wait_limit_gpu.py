@@ -41,3 +41,27 @@ def test_a_wait_that_gives_up_is_reported(dev):
     want = X.half().double() @ W.half().double()
     err = ((Y.double() - want).abs().max() / want.abs().max()).item()
     assert err <= 1e-5, err
+
+
+def test_a_large_single_call_reports_its_waits_and_a_smaller_one_has_none(dev):
+    """Single f16 products of more than 128 tiles of 256 x 128 run on the same kernel; 128 do not."""
+    gen = torch.Generator(device="cpu").manual_seed(6)
+    X, W = torch.randn(4352, 128, generator=gen).to(dev), torch.randn(128, 1024, generator=gen).to(dev)
+    Y = torch.zeros(4352, 1024, device=dev)
+    call = lambda m: (MatRef(X), MatRef(W), MatRef(Y), 1, m, 128, 1024, None, True)
+    assert st.matmul_plan(*call(4352))[0] == 2 and st.matmul_plan(*call(4096))[0] == 1
+    st.sync()
+    try:
+        st.set_wait_limit(0)
+        st.matmul_with(*call(4096))
+        st.sync()
+        st.matmul_with(*call(4352))
+        with pytest.raises(st.ScratchtapeError, match="single f16 GEMMs"):
+            st.sync()
+    finally:
+        st.set_wait_limit(-1)
+    st.sync()
+    want = X.half().double() @ W.half().double()
+    st.matmul_with(*call(4352))
+    st.sync()
+    assert ((Y.double() - want).abs().max() / want.abs().max()).item() <= 1e-5
