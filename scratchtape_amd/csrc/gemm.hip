@@ -511,13 +511,17 @@ struct TileCfg {
     int64_t splits, slice_k;
 };
 
-template <int BK, bool F16>
-KernelFn pick_kernel(const TileCfg &tc, bool ta, bool tb, bool whole) {
-    if (!whole) return pick_trans<32, 32, BK, F16, false>(ta, tb);
-    if (tc.bm == 128 && tc.bn == 128) return pick_trans<128, 128, BK, F16, true>(ta, tb);
-    if (tc.bm == 128) return pick_trans<128, 64, BK, F16, true>(ta, tb);
-    if (tc.bm == 64) return pick_trans<64, 64, BK, F16, true>(ta, tb);
-    return pick_trans<32, 32, BK, F16, true>(ta, tb);
+// The tiles that plan_tiles picks.  (f16: m % 64 == 0 and n % 32 == 0, so every
+// tile is whole.)
+KernelFn pick_kernel(const TileCfg &tc, bool f16, bool ta, bool tb, bool whole) {
+    if (f16) {
+        if (tc.bm == 128) return pick_trans<128, 64, 64, true, true>(ta, tb);
+        if (tc.bm == 64) return pick_trans<64, 64, 64, true, true>(ta, tb);
+        return pick_trans<32, 32, 64, true, true>(ta, tb);
+    }
+    if (tc.bm == 128) return pick_trans<128, 128, 32, false, true>(ta, tb);
+    if (tc.bm == 64) return pick_trans<64, 64, 32, false, true>(ta, tb);
+    return whole ? pick_trans<32, 32, 32, false, true>(ta, tb) : pick_trans<32, 32, 32, false, false>(ta, tb);
 }
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -595,9 +599,10 @@ st::DmaGemm make_dma(const st_matref *a, const st_matref *b, const st_matref *ou
 // overlap and take W `shared` per stage; `lead` stages stand for each
 // workgroup's first loads and its stores.  The constants are fitted to f32
 // products from 64 x 80 x 64 (20 workgroups of 32 x 32: 5.0 us, 64 x 64: 8.2) to
-// 3001 x 1003 x 2000 (32 x 32: 150 us, 64 x 64: 120, 128 x 64: 129, 128 x 128:
-// 152) and agree with them to about 15 %; the f16 ones, where a stage is
-// bound by its loads and conversions, to f16 shapes.
+// 3001 x 1003 x 2000 (32 x 32: 150 us, 64 x 64: 120, 128 x 128: 152) and agree with
+// them to about 15 %; the f16 ones, where a stage is bound by its loads and
+// conversions, to f16 shapes.  (f32 tiles of 128 x 64 at 1.28 us a stage and f16
+// ones of 128 x 128 at 1.3 are never better than twice as many of half the size.)
 // Split-k as the reference allows it (matmul.rs:117-123): no epilogue but +=,
 // packed out; each slice at least 4 k-stages, the partials summed by a launch of
 // its own.
@@ -605,15 +610,12 @@ TileCfg plan_tiles(bool f16, bool ta, bool tb, const st_epilogue &epi, const st_
                    int64_t n) {
     struct Cand {
         int bm, bn;
-        double alone, shared, lead;        // us per 32-deep f32 stage
-        double alone16, shared16, lead16;  // us per 64-deep f16 stage
+        double alone, shared, lead;  // us per stage (32 deep in f32, 64 in f16)
     };
     // 32 x 32 tiles of operands whose rows are contiguous load with a quarter of the threads.
     const double narrow = ta && !tb ? 1.45 : ta || !tb ? 1.1 : 1.0;
-    const Cand cands[] = {{128, 128, 2.46, 2.05, 3.0, 1.4, 1.3, 8.0},
-                          {128, 64, 1.38, 1.28, 3.0, 0.76, 0.53, 8.0},
-                          {64, 64, 0.80, 0.59, 3.0, 0.56, 0.33, 8.0},
-                          {32, 32, 0.36, 0.19 * narrow, 1.5, 0.29, 0.145, 8.0}};
+    const Cand cands32[] = {{128, 128, 2.46, 2.05, 3.0}, {64, 64, 0.80, 0.59, 3.0}, {32, 32, 0.36, 0.19 * narrow, 1.5}};
+    const Cand cands16[] = {{128, 64, 0.76, 0.53, 8.0}, {64, 64, 0.56, 0.33, 8.0}, {32, 32, 0.29, 0.145, 8.0}};
     const int BK = f16 ? 64 : 32;
     const bool epi_free = !epi.bias && !epi.relu && !epi.mask && !epi.residual;
     const bool packed_out = (out->ld == 0 || out->ld == n) && out->group <= 1;
@@ -629,11 +631,10 @@ TileCfg plan_tiles(bool f16, bool ta, bool tb, const st_epilogue &epi, const st_
     const int64_t S = std::max<int64_t>(1, cdiv(k, BK));  // k-stages
     TileCfg best = {32, 32, 1, S * BK};
     double best_t = -1;
-    for (const Cand &c : cands) {
+    for (const Cand &c : f16 ? cands16 : cands32) {
         if (c.bm > 32 && (m < c.bm || n < c.bn)) continue;  // (see WHOLE)
         const int64_t tiles = batch * cdiv(m, c.bm) * cdiv(n, c.bn);
-        const double alone = f16 ? c.alone16 : c.alone, shared = f16 ? c.shared16 : c.shared;
-        const double lead = f16 ? c.lead16 : c.lead;
+        const double alone = c.alone, shared = c.shared, lead = c.lead;
         auto time = [&](int64_t sp, int64_t stages) {
             double t = ((double)stages + lead) * std::max(alone, (double)cdiv(tiles * sp, cus) * shared);
             if (sp > 1) t += 3.0 + 8.0 * (double)(sp * batch * m * n) / 4e6;
@@ -789,8 +790,7 @@ st_status gemm_impl(const st_matref *a, const st_matref *b, const st_matref *out
     }
 
     const bool whole = m >= tc.bm && n >= tc.bn;
-    const KernelFn fn = f16 ? pick_kernel<64, true>(tc, a->trans, b->trans, whole)
-                            : pick_kernel<32, false>(tc, a->trans, b->trans, whole);
+    const KernelFn fn = pick_kernel(tc, f16, a->trans, b->trans, whole);
     // Rows of 2^23 workgroups (a grid has fewer than 2^32 threads along x).
     const int64_t tiles = cdiv(n, tc.bn) * cdiv(m, tc.bm), gx = std::min<int64_t>(tiles, 1 << 23);
     dim3 grid((unsigned)gx, (unsigned)cdiv(tiles, gx), (unsigned)(batch * splits));
