@@ -9,8 +9,9 @@
  *    written in place.  The library owns only a grow-only scratch arena per
  *    device and use (split-k partials, probe-selection distances, LayerNorm
  *    column partials), like the reference's `split_scratch`
- *    (gpu_step/matmul.rs:207-217); the kNN search keeps its candidate lists
- *    in LDS and allocates nothing.  An arena grows only outside graph
+ *    (gpu_step/matmul.rs:207-217); a query-major kNN search keeps its
+ *    candidate lists in LDS (the _split forms in memory of the caller's) and
+ *    allocates nothing.  An arena grows only outside graph
  *    capture: a call that would grow it while its stream is being captured
  *    fails with ST_ERR_INVALID (run the call once before capturing).  A
  *    superseded arena buffer is kept, not freed, until st_scratch_release(),

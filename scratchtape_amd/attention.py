@@ -5,8 +5,10 @@ between them (gpu_step/tape.rs:196-212, 349-372, 475-491; rows.rs:101-123):
 Q, K, V are head views of a fused [B*T, 3D] buffer, the scores S and
 probabilities P are stacked [B*H*T, T], the context is written into the merged
 [B*T, D] layout.  Every product goes through the GEMM of this package and the
-softmax through its row kernels; `use_f16` picks the f16-in/f32-acc route for
-the six products (the reference keeps them f32: matmul.rs:90-95).
+softmax through its row kernels, or, where all six products run in f32 and that
+is faster (_f32_step_pays), through three launches that keep a block of score
+rows on chip and write the same buffers; `use_f16` picks the f16-in/f32-acc
+route for the six products (the reference keeps them f32: matmul.rs:90-95).
 
 `fused_forward` / `fused_backward` compute the same attention in two launches
 that never write S or P (the reference's next step, docs/tiers_design.md:891-893):

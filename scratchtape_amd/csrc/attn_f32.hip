@@ -244,8 +244,12 @@ __global__ __launch_bounds__(THREADS) void k_attn_rows(AttnArgs g) {
                     }
                 }
             }
-            // e / sum, correctly rounded, from one reciprocal per row: the quotient's
-            // remainder is exact in an FMA (1 <= sum <= t and 0 <= e <= 1, or NaN).
+            // e / sum from one reciprocal per row and one correction per quotient, by
+            // Markstein's method (IBM J. Res. Dev. 34(1), 1990): the quotient's remainder
+            // is exact in an FMA, which makes the result the correctly rounded one (1 <=
+            // sum <= t and 0 <= e <= 1, or NaN) unless quotient or remainder underflow:
+            // an e below about 1e-30 may give a neighbour of it (1.4e-45 away among the
+            // subnormal numbers).
             sum = group_sum(sum, lane);
             const float inv = 1.0f / sum;
             for (int j0 = c16; j0 < tcols; j0 += 16 * G) {
@@ -449,7 +453,12 @@ __global__ __launch_bounds__(THREADS) void k_attn_cols(AttnArgs g) {
     }
 }
 
-// Launches f<width class>(): the narrowest of the compiled head widths that holds hd.
+// Launches f<width class>(): the narrowest of the compiled head widths that
+// holds hd.  A width is padded to its class, at the class's cost and more (96
+// problems of T = 200, forward rows and both backward launches, us: 80 wide in
+// its own class 106, 96 wide in that of 128 243, 128 wide 185), so there is one
+// for each of the widths in use, 32, 64 and 80; 128 takes the rest, where the
+// separate launches are mostly faster (a caller of the C interface chooses).
 template <class F>
 st_status by_width(int64_t hd, F f) {
     if (hd % 4)

@@ -113,7 +113,7 @@ __global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ keys
 // sums all 64 rows, lane r row r in index order: a wave of 16 keys on its own
 // issues as many instructions for its sums with a quarter of the lanes, and
 // that form was bound by its 3,000 instructions per 16 keys.  2^20 keys, us, a
-// thread per key, a wave per 16 keys and now: x 256 4,635, 260, 192 (6.0 TB/s);
+// thread per key, a wave per 16 keys and now: x 256 4,635, 245, 185 (6.2 TB/s);
 // x 128 147 -> 97; x 64 101 -> 46.  The codes need no division per component: x / scale + 1.5 and the
 // two roundings are monotone in x, so each code step is a threshold on x
 // (quantize_step3), found once per row.  Widths of 64, 128 and 256 know at
@@ -1469,7 +1469,8 @@ static double cell_major_us(int64_t nq, int64_t nprobe, int64_t ncells, int64_t 
 // their lists: one per CU in all.  20 queries' worth of runs of 40 chunks each
 // take 36 us, merge included, where one workgroup per query takes 118 to 200;
 // two per CU (512 in all) measured 51 against 36 us at 16 queries of 632
-// chunks, 61 against 56 at 64, and 74 against 79 at 100.
+// chunks, 61 against 56 at 64, and 74 against 79 at 100.  129 to 255 queries
+// stay at one each (two each would be up to 510; not measured).
 static int64_t query_splits(int64_t nq) {
     const int64_t n = nq > 0 ? 256 / nq : 1;
     return n < 2 ? 1 : std::min<int64_t>(n, SPLIT_MAX);

@@ -25,22 +25,23 @@
 // + 15, so an operand is one ds_read_b128 per k-step.
 //
 // k_probe_prep turns the centroids into digit tiles, exponents and norms once
-// per index.  Two launches per chunk of queries:
-//   k_probe_part  grid = centroid slices (up to 12 tiles) x groups of 64
-//                 queries.  The workgroup turns its 64 queries into digit
-//                 tiles in LDS (as k_probe_prep would), stages its slice in
-//                 LDS, and each wave
-//                 scores its 16 queries against it, keeping the 12 x 4
-//                 order-preserving dd keys of its lane in registers.  A
-//                 per-query threshold -- the nprobe-th smallest of the 16
-//                 per-lane minima, so at least nprobe keys lie at or below it
-//                 and with them the slice's top nprobe -- leaves a few
-//                 candidates per (query, slice), which go to a fixed slot of
-//                 the scratch arena.  A slot that would overflow gets the
-//                 slice's exact top nprobe instead (successive minima over the
-//                 registers).
-//   k_probe_merge one wave per query: the exact top nprobe by (dd, id) over
-//                 its slots' candidates.
+// per index.  Two launches per chunk of queries (three with MANY, whose
+// queries' digits k_probe_prep makes first):
+//   k_probe_part  grid = centroid slices (2 HT = 2, 4, 6 or 12 tiles) x groups
+//                 of 64 queries, or (MANY) slices x workgroups that walk
+//                 several groups.  The workgroup stages its slice in LDS and
+//                 turns its 64 queries into digit tiles there (as k_probe_prep
+//                 would; MANY reads them made).  Each wave scores 16 queries
+//                 against half of the slice, keeping the HT x 4 order-preserving
+//                 dd keys of its lane in registers.  A per-query threshold --
+//                 the nprobe-th smallest of the 32 minima of its lanes in both
+//                 halves, so at least nprobe keys lie at or below it and with
+//                 them the slice's top nprobe -- leaves a few candidates per
+//                 (query, slice), which go to a fixed slot of the scratch arena.
+//                 A slot that would overflow gets each half's exact top nprobe
+//                 instead (successive minima over the registers).
+//   k_probe_merge one workgroup of four waves per query: the exact top nprobe
+//                 by (dd, id) over its slots' candidates.
 // A k_probe_part workgroup is 8 waves: two per query tile, each scoring half
 // of the slice's tiles (two waves per SIMD hide each other's latencies).
 // dd never leaves the chip; per query only the candidates (about nprobe per
@@ -193,10 +194,11 @@ constexpr int32_t INONE = 0x7fffffff;
 // lane per slot reads an entry of consecutive slots with one coalesced load;
 // pcnt[q S + s] counts them.
 //
-// grid: S * gy workgroups of 256 threads; workgroup b takes (slice, query
-// group) = (idx / gy, idx % gy) with idx dealt so that the gy workgroups of a
-// slice are consecutive on one XCD (workgroup ids go round robin over the 8
-// XCDs), which then reads the slice's digits from HBM once.
+// grid: S * gw workgroups of PART_T threads (gw = gy, the query groups, unless
+// MANY); workgroup b takes slice idx / gw and the query groups from idx % gw on
+// with idx dealt so that the gw workgroups of a slice are consecutive on one
+// XCD (workgroup ids go round robin over the 8 XCDs), which then reads the
+// slice's digits from HBM once.
 //
 // A slice is 2 HT tiles: 12 when there are enough (slice, query group) pairs
 // to fill the chip, fewer for small indexes and batches, where each workgroup
@@ -210,9 +212,10 @@ constexpr int32_t INONE = 0x7fffffff;
 // while it forms its keys.  Without it every (slice, group) pair stages the
 // slice and turns the queries into digits again, 64 times over for a large
 // index.  Bound by the VALU (about 2,000 instructions per wave and group: the
-// keys, their order, the candidates).  Both launches, us, one group each and
-// now: 4,096 queries over 12,288 cells 298 -> 180, over 6,000 (16 probes) 178 ->
-// 109, over 20,000 487 -> 370; 512 over 12,288 44 -> 39; 2,048 over 4,000 61 -> 49.
+// keys, their order, the candidates).  All launches, us, one group each and
+// now, 8 probes: 4,096 queries over 12,288 cells 298 -> 180, over 20,000 487 -> 370;
+// 512 over 12,288 44 -> 39; 2,048 over 4,000 61 -> 49; 16 probes: 4,096 over 6,000
+// 178 -> 109, over 12,288 328 -> 190.
 template <int HT, bool MANY>
 __global__ __launch_bounds__(PART_T) void k_probe_part(const float *__restrict__ queries,
                                                     const int8_t *__restrict__ qdig,
@@ -555,7 +558,7 @@ __device__ __forceinline__ int slot_size(int32_t c) { return (c & 0xffff) + ((c 
 // (One wave per query with a lane per slot took the general path for
 // nearly every query at nprobe = 16, and whenever there were fewer slots than
 // probes: 4 queries x 16 probes over 4,096 cells took 64 us for both launches,
-// 15 now; 4,096 queries over 12,288 cells 873, 298 now.)
+// 15 with this merge; 4,096 queries x 16 probes over 12,288 cells 873, then 328.)
 constexpr int MERGE_W = 4;
 constexpr int ME_MAX = CAPQ / MERGE_W;  // entries per thread, at most
 __global__ __launch_bounds__(64 * MERGE_W) void k_probe_merge(const uint64_t *__restrict__ ck,
