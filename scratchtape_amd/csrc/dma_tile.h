@@ -145,11 +145,21 @@ __device__ __forceinline__ void wait_stage(int ahead) {
 // Workgroup barrier without the memory fence of __syncthreads() (which would
 // wait for every load of this wave, the DMA of the younger stages included);
 // the empty asm statements keep the compiler from moving memory accesses
-// across it.
+// across it.  It waits for nothing: the wave's LDS reads before it are over
+// where their values have been used (a multiplication, an addition), its LDS
+// writes are not.
 __device__ __forceinline__ void bar() {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+}
+
+// bar() once this wave's LDS writes are done, for what other waves read behind
+// it (a write that was only issued may land after their reads).
+__device__ __forceinline__ void bar_written() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    bar();
 }
 
 // Element offset (from the operand's matrix base, at k = 0) of the 16 bytes

@@ -227,7 +227,7 @@ __global__ __launch_bounds__(THREADS) void k_gemm_dma(KArgs g) {
                 for (int r = 0; r < 4; r++)
                     lds[(wm * WM + i * 16 + 4 * (lane >> 4) + r) * TP + wn * WN + j * 16 + (lane & 15)] = acc[i][j][r];
     }
-    bar();
+    bar_written();
     if (g.splits > 1) {
         float *P = g.out + (zb * g.splits + slice) * (int64_t)g.m * g.n;
         for (int e = tid; e < BM * BN / 4; e += THREADS) {
