@@ -1103,6 +1103,14 @@ bool group_eligible(const DmaGemm &d) {
     if (d.f16) {
         const auto panel_ok = [&](int64_t ld) { return (d.k + 256) * ld * 4 + 4096 < ((int64_t)1 << 31); };
         if (!panel_ok(d.lda) || !panel_ok(d.ldb)) return false;
+    } else {
+        // The f32 kernel's lane offsets are 32-bit bytes from the matrix (at the
+        // unit's k): every row of an operand with contiguous k, else a stage's
+        // k-lines.
+        const auto span_ok = [&](bool kc, int64_t rows, int64_t ld) {
+            return 4 * (kc ? rows * ld + BK : BK * ld + rows) < ((int64_t)1 << 32);
+        };
+        if (!span_ok(!d.ta, d.m, d.lda) || !span_ok(d.tb, d.n, d.ldb)) return false;
     }
     return fits32(d.batch * (d.m / Square::TM) * (d.n / TN) * (d.k / BK));
 }

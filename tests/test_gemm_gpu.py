@@ -269,7 +269,8 @@ def tape_forms(dev, m, k, n, use_f16, seed):
 # moved back to the edge, fewer rows or columns than a tile, a partial first k-stage; odd offsets and strides.  The
 # last shapes of each route are large enough for its larger tiles (TILES; the others take 32 x 32 in some form).
 EDGE_F32 = [(1, 1, 1), (3, 5, 2), (31, 2, 33), (32, 31, 32), (33, 32, 31), (64, 33, 63), (65, 64, 64), (127, 65, 32),
-            (33, 1, 129), (200, 80, 200), (97, 300, 4), (1, 257, 130), (2500, 33, 2300), (1300, 3, 700), (6401, 100, 259), (2305, 100, 3075)]
+            (33, 1, 129), (200, 80, 200), (97, 300, 4), (1, 257, 130), (2500, 33, 2300), (1300, 3, 700),
+            (6401, 100, 259), (2305, 100, 3075)]
 EDGE_F16 = [(64, 32, 32), (64, 96, 160), (192, 64, 96), (320, 160, 1056), (4096, 32, 1056), (6400, 64, 1120),
             (256, 96, 3104)]
 TILES = {(6401, 100, 259): (64, 64), (2305, 100, 3075): (128, 128), (4096, 32, 1056): (128, 64),
@@ -435,10 +436,10 @@ def test_grouped_random_groups_match_oracle(dev):
             check_case(p)
 
 
-# Single calls around the sizes from which the grouped kernel's 256 x 128 tiles take them (kernel 2): more than 128 tiles
-# (f16) or 256 (f32, but not 257 to 384) with every epilogue term, batches, and a product split over k with column
-# sums; calls just below stay on the LDS-DMA kernel (1).  (Column sums of a transposed b put an f16 call on the f32
-# route.)
+# Single calls around the sizes from which the grouped kernel's 256 x 128 tiles take them (kernel 2): more than 128
+# tiles (f16) or 256 (f32, but not 257 to 384) with every epilogue term, batches, and a product split over k with
+# column sums; calls just below stay on the LDS-DMA kernel (1).  (Column sums of a transposed b put an f16 call on
+# the f32 route.)
 @pytest.mark.parametrize("case,use_f16,kernel", [
     ((1, 2048, 128, 2048, False, False, True, True, True, True, True), True, 1),
     ((1, 2048, 128, 2176, False, False, True, True, True, True, True), True, 2),
@@ -523,3 +524,20 @@ def test_any_shape_grid_of_several_rows(dev):
     assert st.matmul_plan(st.MatRef(a), st.MatRef(b), st.MatRef(out), 1, 1, 1, n, None, False)[:3] == (0, 32, 32)
     st.matmul_f32(st.MatRef(a), st.MatRef(b), st.MatRef(out), 1, 1, 1, n)
     assert torch.equal(out[:n], 3.0 * b) and out[n].item() == -1.0
+
+
+@pytest.mark.parametrize("grouped", [False, True])
+def test_f32_operand_past_4_gib(dev, grouped):
+    """A of 2^20 x 1056 (4.4 GB): every row of the product, its last ones past the first 4 GiB of A."""
+    m, k, n = 1 << 20, 1056, 128
+    a = torch.full((m, k), 0.25, device=dev)
+    a += torch.arange(m, device=dev, dtype=torch.float32).remainder_(1021).view(m, 1)  # a row's values tell it apart
+    b = torch.ones(k, n, device=dev)
+    out = torch.zeros(m, n, device=dev)
+    call = (st.MatRef(a), st.MatRef(b), st.MatRef(out), 1, m, k, n, None, False)
+    if grouped:
+        st.matmul_grouped([call])
+    else:
+        st.matmul_with(*call)
+    want = a[:, :1] * k  # sums of 1,056 equal values, each partial sum a multiple of 1/4 below 2^21: exact
+    assert bool((out == want).all())

@@ -12,7 +12,8 @@ ANY_SHAPE, DMA, GROUP = 0, 1, 2
 FORMS = [(False, False), (False, True), (True, False), (True, True)]
 
 
-def plan(m, k, n, use_f16=False, ta=False, tb=False, batch=1, aligned=True, bias=False, accumulate=False, col_sum=False):
+def plan(m, k, n, use_f16=False, ta=False, tb=False, batch=1, aligned=True, bias=False, accumulate=False,
+         col_sum=False):
     """(kernel, tile rows, tile columns, slices, scratch bytes) of a call on packed matrices."""
     p = (1 << 20) + (0 if aligned else 4)
     ref = lambda trans, size: _lib.StMatRef(p, 0, size, int(trans), 0, 0, 1, 0)
@@ -47,8 +48,17 @@ def test_the_edge_shapes_reach_every_tile(use_f16):
     (768, 2048, 2304, False, "tn", GROUP), (2048, 2048, 512, True, "plain", DMA), (2048, 2048, 512, True, "tn", GROUP),
     (2048, 2048, 1024, True, "plain", GROUP)])
 def test_single_calls_take_the_faster_kernel(m, k, n, use_f16, form, kernel):
-    kw = dict(tn=dict(ta=True, accumulate=True, col_sum=True), nt=dict(tb=True, bias=True), nn=dict(bias=True), plain={})
+    kw = dict(tn=dict(ta=True, accumulate=True, col_sum=True), nt=dict(tb=True, bias=True), nn=dict(bias=True),
+              plain={})
     assert plan(m, k, n, use_f16, **kw[form])[0] == kernel
+
+
+@pytest.mark.parametrize("m,k,n,ta,tb,kernel", [(1 << 20, 1024, 128, False, False, DMA),
+                                                (1 << 20, 992, 128, False, True, GROUP),
+                                                (1 << 20, 1024, 128, True, False, GROUP),
+                                                (256, 1024, 1 << 20, False, True, DMA)])
+def test_f32_operands_past_4_gib_stay_off_the_grouped_kernels_32_bit_offsets(m, k, n, ta, tb, kernel):
+    assert plan(m, k, n, False, ta, tb, bias=True)[0] == kernel
 
 
 def test_a_plan_needs_valid_arguments_and_no_device():
@@ -74,7 +84,8 @@ def test_a_long_small_product_is_planned_in_microseconds(m, k, n, slices):
     assert best < 40e-6, best
 
 
-@pytest.mark.parametrize("m,k,n", [(1, 4, 300_000_000), (31, 1, (1 << 30) - 1), (100_000, 32, 100_000), (64, 1, 1 << 27),
+@pytest.mark.parametrize("m,k,n", [(1, 4, 300_000_000), (31, 1, (1 << 30) - 1), (100_000, 32, 100_000),
+                                   (64, 1, 1 << 27),
                                    (8_388_480, 3, 31)])
 def test_large_outputs_of_small_tiles_are_accepted(m, k, n):
     """Up to 33 million 32 x 32 tiles, where the device holds the output."""
